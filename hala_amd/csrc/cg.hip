@@ -169,10 +169,10 @@ __global__ __launch_bounds__(256) void cg_spmv_pz_kernel(int n, const int *__res
 
 // x += a p; r += (-a) Ap; <r,r> (and <r, r./d> for Jacobi).  The last block
 // takes the stop decision and, for identity/Jacobi, the new beta.
-// lslot (ILU on the column layout, may be null): r also goes straight into the
-// L sweep's slot-order input (the sweep's gather pass, fused here), and x is
-// left alone (null): the L sweep's helper workgroups update it meanwhile, and
-// cg_xfinal does the pass whose sweep the stop gated off.
+// lslot (fused ILU, may be null): r also goes straight into the first sweep's
+// input (the sweep's gather pass, fused here), and x is left alone (null): it
+// is updated later in the pass, by the column sweep's helper workgroups or by
+// cg_pupdate_kernel, and cg_xfinal does the pass that the stop gated off.
 template <int PREC>
 __global__ __launch_bounds__(256) void cg_update_kernel(int n, const double *__restrict__ p,
                                                         const double *__restrict__ ap, const double *__restrict__ d,
@@ -307,22 +307,26 @@ __global__ __launch_bounds__(256) void cg_zscatter_rz_kernel(int n, const int *_
     }
 }
 
-// p = beta p; p += 1 z   (z = r for identity, r ./ d for Jacobi)
+// p = beta p; p += 1 z   (z = r for identity, r ./ d for Jacobi).  x (nullable):
+// x += alpha p with the old p first (the pass's update of x, which reads p anyway).
 template <int PREC>
 __global__ void cg_pupdate_kernel(int n, const double *__restrict__ z, const double *__restrict__ r,
-                                  const double *__restrict__ d, double *__restrict__ p, const cg_state *st) {
+                                  const double *__restrict__ d, double *__restrict__ p, const cg_state *st,
+                                  double *__restrict__ x = nullptr) {
     if (st->done) return;
-    const double b = st->beta;
+    const double b = st->beta, a = st->alpha;
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; i < n; i += stride) {
         double zi = (PREC == PREC_ID) ? r[i] : (PREC == PREC_JAC ? r[i] / d[i] : z[i]);
-        p[i] = b * p[i] + 1.0 * zi;
+        const double pi = p[i];
+        if (x) x[i] = x[i] + a * pi;
+        p[i] = b * pi + 1.0 * zi;
     }
 }
 
-// x += alpha p for the last pass of a fused ILU-PCG solve (whose L sweep, and
-// with it the helpers' update of x, the stop flag gated off)
+// x += alpha p for the last pass of a fused ILU-PCG solve (whose update of x
+// the stop flag gated off)
 __global__ void cg_xfinal(int n, double *__restrict__ x, const double *__restrict__ p, const cg_state *st) {
     const double a = st->alpha;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
@@ -402,7 +406,8 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
     cg_residual_kernel<false><<<gs, 256, 0, c->stream>>>(n, pntr, indx, vals, x, b, r);
     HALA_CHECK_LAUNCH();
     const int *gate = &st->done;
-    const bool fused = P.prec == PREC_ILU && !P.transposed && c->opt.cg_fuse && ilu_fused64(P.M);
+    ilu_ends ends{};
+    const bool fused = P.prec == PREC_ILU && c->opt.cg_fuse && ilu_fused64(P.M, P.transposed, ends);
     auto precond = [&](const double *in, double *out, const int *g) {
         if (P.transposed) ilu_apply_t64(P.M, in, out, g);
         else ilu_apply64(P.M, in, out, g);
@@ -466,22 +471,21 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
             break;
         default:
             if (fused) {  // the sweeps' gather and scatter passes fused into the update and r.z
-                tri_plan &L = P.M->L, &U = P.M->U;
                 const int xu = c->opt.cg_xcd ? 1 : 0;
                 cg_update_kernel<PREC_ILU><<<xu ? xcd_grid(ge) : ge, 256, 0, c->stream>>>(
-                    n, p, ap, nullptr, nullptr, r, part, part2, wait_error_flag(c), st, L.slot_of_row.as<int>(),
-                    L.col.xs64.as<double>(), xu);
+                    n, p, ap, nullptr, nullptr, r, part, part2, wait_error_flag(c), st, ends.in_slot, ends.in, xu);
                 const col_axpy ax{x, p, &st->alpha, n};  // x += alpha p on the L sweep's helper workgroups
-                ilu_apply64_mid(P.M, gate, &ax);
-                cg_zscatter_rz_kernel<<<ge, 256, 0, c->stream>>>(n, U.slot_of_row.as<int>(), U.out64.as<double>(), r, z,
-                                                                 part, wait_error_flag(c), st);
+                ilu_apply64_mid(P.M, P.transposed, gate, ends.axpy ? &ax : nullptr);
+                cg_zscatter_rz_kernel<<<ge, 256, 0, c->stream>>>(n, ends.out_slot, ends.out, r, z, part,
+                                                                 wait_error_flag(c), st);
             } else {
                 cg_update_kernel<PREC_ILU><<<ge, 256, 0, c->stream>>>(n, p, ap, nullptr, x, r, part, part2,
                                                                       wait_error_flag(c), st);
                 precond(r, z, gate);
                 cg_rz_kernel<<<ge, 256, 0, c->stream>>>(n, r, z, part, wait_error_flag(c), st);
             }
-            cg_pupdate_kernel<PREC_ILU><<<gp, 256, 0, c->stream>>>(n, z, nullptr, nullptr, p, st);
+            cg_pupdate_kernel<PREC_ILU><<<gp, 256, 0, c->stream>>>(n, z, nullptr, nullptr, p, st,
+                                                                   fused && !ends.axpy ? x : nullptr);
         }
         HALA_CHECK_LAUNCH();
     };

@@ -212,6 +212,7 @@ static int *option_slot(hala_ctx c, const char *name) {
     if (k == "tri_col") return &c->opt.tri_col;
     if (k == "tri_col_cols") return &c->opt.tri_col_cols;
     if (k == "tri_col_split") return &c->opt.tri_col_split;
+    if (k == "tri_grid") return &c->opt.tri_grid;
     if (k == "cg_fuse") return &c->opt.cg_fuse;
     if (k == "cg_xcd") return &c->opt.cg_xcd;
     if (k == "cg_batch_max") return &c->opt.cg_batch_max;

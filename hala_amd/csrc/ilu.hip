@@ -230,13 +230,45 @@ __global__ void set_int(int *p, int v) { *p = v; }
 // the pencil schedule applies (a stencil pattern, and the option allows it)
 static bool use_stencil(hala_ilu M) { return M->sp && M->ctx->opt.tri_stencil; }
 
-bool ilu_fused64(hala_ilu M) {
-    return M->factored && !use_stencil(M) && col_usable(M->ctx, M->L, true) && col_usable(M->ctx, M->U, true) &&
-           M->L.col.hand64;
+// both triangles on the grid sweeps, in one packed order
+static bool use_grid(hala_ilu M, bool is64) {
+    return !use_stencil(M) && grid_pair_usable(M->ctx, M->L, M->U, is64);
 }
 
-void ilu_apply64_mid(hala_ilu M, const int *gate, const col_axpy *ax) {
+static bool use_columns(hala_ilu M) {
+    return !use_stencil(M) && col_usable(M->ctx, M->L, true) && col_usable(M->ctx, M->U, true) && M->L.col.hand64;
+}
+
+bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
     hala_ctx c = M->ctx;
+    if (!M->factored) return false;
+    if (transposed) ilu_prepare_adjoint(M);
+    tri_plan &first = transposed ? M->Ut : M->L, &second = transposed ? M->Lt : M->U;
+    if (transposed ? grid_pair_usable(c, first, second, true) : use_grid(M, true)) {
+        grid_reserve(c, first, true, 1);
+        grid_reserve(c, second, true, 1);
+        e = ilu_ends{first.grid.slot.as<int>(), first.grid.in64.as<double>(), first.grid.slot.as<int>(),
+                     second.grid.out64.as<double>(), false};
+        return true;
+    }
+    if (!transposed && use_columns(M)) {
+        e = ilu_ends{first.slot_of_row.as<int>(), first.col.xs64.as<double>(), second.slot_of_row.as<int>(),
+                     second.out64.as<double>(), true};
+        return true;
+    }
+    return false;
+}
+
+void ilu_apply64_mid(hala_ilu M, bool transposed, const int *gate, const col_axpy *ax) {
+    hala_ctx c = M->ctx;
+    if (transposed) {
+        grid_pair_mid64(c, M->Ut, M->Lt, 1, gate);
+        return;
+    }
+    if (use_grid(M, true)) {
+        grid_pair_mid64(c, M->L, M->U, 1, gate);
+        return;
+    }
     // L's helpers re-arm U's polled output, U's helpers L's for the next apply
     col_sweep64(c, M->L, TRI_SUB, 1.0, gate, &M->U, &M->U, ax);
     col_sweep64(c, M->U, TRI_SUB, 1.0, gate, nullptr, &M->L);
@@ -249,7 +281,11 @@ void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate) {
         stencil_apply<double, double, double>(M, x, r, gate);
         return;
     }
-    if (ilu_fused64(M)) {  // L's output handed to U in slot order
+    if (use_grid(M, true)) {
+        grid_exec_pair<double, double>(c, M->L, M->U, x, 0, r, 0, 1, gate);
+        return;
+    }
+    if (use_columns(M)) {  // L's output handed to U in slot order
         tri_col_exec<double, double>(c, M->L, TRI_SUB, 1.0, x, nullptr, gate, &M->U);
         col_sweep64(c, M->U, TRI_SUB, 1.0, gate, nullptr, &M->L);
         col_scatter64(c, M->U, r, gate);
@@ -268,6 +304,10 @@ void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate) {
     }
     if (use_stencil(M)) {
         stencil_apply<float, double, double>(M, x, r, gate);
+        return;
+    }
+    if (use_grid(M, false)) {
+        grid_exec_pair<float, double>(c, M->L, M->U, x, 0, r, 0, 1, gate);
         return;
     }
     tri_exec<float, double, double>(c, M->L, TRI_SUB, 1.0f, x, M->tmp64.as<double>(), gate);
@@ -297,6 +337,10 @@ void ilu_apply_t64(hala_ilu M, const double *x, double *r, const int *gate) {
     hala_ctx c = M->ctx;
     HALA_REQUIRE(M->factored, HALA_ERR_ARG, "ILU apply before factorisation");
     ilu_prepare_adjoint(M);
+    if (grid_pair_usable(c, M->Ut, M->Lt, true)) {
+        grid_exec_pair<double, double>(c, M->Ut, M->Lt, x, 0, r, 0, 1, gate);
+        return;
+    }
     tri_exec<double, double, double>(c, M->Ut, TRI_SUB, 1.0, x, M->tmp64.as<double>(), gate);
     tri_exec<double, double, double>(c, M->Lt, TRI_SUB, 1.0, M->tmp64.as<double>(), r, gate);
 }
@@ -539,6 +583,11 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         (void)hipEventDestroy(ev[0]);
         (void)hipEventDestroy(ev[1]);
         col_set_handoff(c, M->L, M->U);
+        // the grid sweeps' vectors come from the context's cache, as the rest of the factor
+        for (tri_plan *p : {&M->L, &M->U}) {
+            if (p->grid.ok) grid_reserve(c, *p, true, 1);
+            if (p->grid.ok && want_f32) grid_reserve(c, *p, false, 1);
+        }
         if (M->sp) stencil_load(M, want_f32);
         check_wait_error(c);  // synchronises; a dependency wait that gave up throws here
         const int b = fetch_i32(c, bad);
@@ -570,6 +619,8 @@ int hala_ilu_apply_f32(hala_ilu M, const float *x, float *r) {
         set_device(c);
         if (use_stencil(M)) {
             stencil_apply<float, float, float>(M, x, r, nullptr);
+        } else if (use_grid(M, false)) {
+            grid_exec_pair<float, float>(c, M->L, M->U, x, 0, r, 0, 1, nullptr);
         } else {
             M->tmp32.reserve((size_t)M->n * sizeof(float));
             tri_exec<float, float, float>(c, M->L, TRI_SUB, 1.0f, x, M->tmp32.as<float>());

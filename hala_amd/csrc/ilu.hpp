@@ -57,14 +57,21 @@ void tri_trsm_cols(hala_tri T, char transb, int nrhs, size_t esize, void *B, int
 // r = (LU)^-1 x in the requested precision (see hala_ilu_apply_*)
 // gate (nullable, device flag): skip the apply when *gate != 0 (solver stop flag)
 void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
-// Both triangles on the column layout: the apply's ends can be fused by the
-// caller.  ilu_apply64_mid runs L from its gathered input (L's col.xs64 filled
-// by the caller; the polled outputs were re-armed by the previous apply's
-// sweeps), which hands its results to U's input itself, then U; the result
-// stays in U.out64 in slot order.  ax (nullable): a vector update the L
-// sweep's helper workgroups do meanwhile (see col_sweep64).
-bool ilu_fused64(hala_ilu M);
-void ilu_apply64_mid(hala_ilu M, const int *gate, const hala_amd::col_axpy *ax = nullptr);
+// An FP64 apply whose ends the caller fuses into its own passes: it fills the
+// first sweep's input (row r at in[in_slot[r]]), ilu_apply64_mid runs both
+// sweeps, and the result of row r lies at out[out_slot[r]].  The sweeps re-arm
+// each other's polled outputs.  Column sweeps (axpy true) can also do a vector
+// update on their helper workgroups meanwhile (ax, see col_sweep64; ignored by
+// the grid sweeps).  False: the factor has no such form.
+struct ilu_ends {
+    const int *in_slot;
+    double *in;
+    const int *out_slot;
+    const double *out;
+    bool axpy;
+};
+bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e);
+void ilu_apply64_mid(hala_ilu M, bool transposed, const int *gate, const hala_amd::col_axpy *ax = nullptr);
 void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_apply_t64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_prepare_adjoint(hala_ilu M);

@@ -183,6 +183,10 @@ void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *o
     constexpr bool is64 = sizeof(T) == 8;
     HALA_REQUIRE(is64 ? p.has64 : p.has32, HALA_ERR_ARG, "triangular solve: values not loaded for this precision");
     static_assert(std::is_same<TIN, TOUT>::value, "input and output share a type");
+    if (grid_usable(c, p, is64)) {
+        grid_exec<T, TIN>(c, p, mode, alpha, in, 0, out_nat, 0, 1, gate);
+        return;
+    }
     if (col_usable(c, p, is64)) {  // (its gather pass re-arms the polled output)
         tri_col_exec<T, TOUT>(c, p, mode, alpha, in, out_nat, gate);
         return;

@@ -1,0 +1,73 @@
+// trgrid.hpp -- triangular sweeps of complete 5-point (2-D) and 7-point (3-D)
+// grid patterns as register wavefronts.
+//
+// A plan whose rows are the points (i, j, k) of an nx x ny x nz grid in natural
+// order (row = i + nx j + nx ny k) and whose row depends on exactly its in-grid
+// neighbours at i-1, j-1 and k-1 (backward plans: the mirrored grid) is swept
+// line by line.  A wavefront owns a tile of 8 x 8 lines (64 x 1 in 2-D), one
+// lane per line, and a lane computes one row of its line per step, row (i, j, k)
+// at step i + a + 2 b (a, b: its line's place in the tile).  The i-1 value is
+// then the lane's own previous result, the j-1 value its left neighbour's
+// previous result (a DPP move), the k-1 value comes through LDS and was formed
+// two steps earlier, so that nothing but a few FP operations lies between one
+// step and the next, and no barrier is needed.
+//
+// Vectors live in the packed order of the tiles' steps: element
+// ((tile * S) + step) * 64 + lane.  A backward plan runs the same kernel on the
+// mirrored grid, whose packed order is the forward one reversed, so an ILU's
+// two sweeps share one order and need no permutation between them.
+#pragma once
+#include "common.hpp"
+
+namespace hala_amd {
+
+struct tri_plan;
+
+struct grid_geom {
+    int nx = 0, ny = 0, nz = 0;   // nz == 1: 2-D
+    int ntj = 0, ntk = 0, S = 0;  // tiles along j and k, steps per tile
+    int64_t N = 0;                // packed elements of a vector
+    bool same(const grid_geom &o) const { return nx == o.nx && ny == o.ny && nz == o.nz; }
+};
+
+// The grid side of a plan (member of tri_plan).
+struct tri_gridplan {
+    bool ok = false;
+    bool zyx = true;  // a row's terms in the order k-1, j-1, i-1 (else i-1, j-1, k-1)
+    grid_geom g;
+    dbuf order;         // tile per ticket, in dependency order
+    dbuf slot;          // packed element (forward order) of every natural row
+    dbuf rec64, rec32;  // per (tile, step) the step's coefficients and diagonal (see grid_pack)
+    bool has64 = false, has32 = false;
+    // packed input, output and frames (boundary results the tiles poll; sentinels
+    // before a sweep) of `rhs64` / `rhs32` vectors, made on first use
+    dbuf in64, in32, out64, out32, fr64, fr32;
+    int rhs64 = 0, rhs32 = 0;
+};
+
+// Recognises p's pattern from its dependency lists and lays the grid plan out
+// (p.grid.ok tells).  Reads a few integers back (synchronises).
+void build_grid_plan(hala_ctx c, tri_plan &p);
+// The factor's values into the step records of one precision.
+void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
+// The plan runs on the grid sweep in this precision (pattern, values, options).
+bool grid_usable(hala_ctx c, const tri_plan &p, bool is64);
+// ... and so does second, in first's packed order (an ILU's two triangles).
+bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64);
+// Packed vectors for nrhs right-hand sides.
+void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs);
+
+// out_k = op^-1 in_k for nrhs vectors in natural order (in + k ldin, out + k ldout), TRI_SUB / TRI_SUM as tri_exec.
+template <class T, class TIO>
+void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_t ldin, TIO *out, int64_t ldout,
+               int nrhs, const int *gate);
+// The two sweeps of an apply (TRI_SUB, first forward, second backward or the
+// reverse), natural order in and out.  Plans run as a pair are only run as one.
+template <class T, class TIO>
+void grid_exec_pair(hala_ctx c, tri_plan &first, tri_plan &second, const TIO *in, int64_t ldin, TIO *out,
+                    int64_t ldout, int nrhs, const int *gate);
+// The pair without its ends: first's packed input (in64, filled by the caller)
+// to second's packed output (out64), both by first's slot map.
+void grid_pair_mid64(hala_ctx c, tri_plan &first, tri_plan &second, int nrhs, const int *gate);
+
+}  // namespace hala_amd

@@ -384,6 +384,7 @@ void build_schedule(hala_ctx c, tri_plan &p, bool want32, bool have_levels) {
     // the column layout lays the slots out in its own order; else (or when it
     // gave up before) the level order does
     if (c->opt.tri_col) build_col_plan(c, p, c->opt.tri_col_cols);
+    build_grid_plan(c, p);
     if (!p.laid_out) lay_out_slots(c, p, p.perm.as<int>());
     p.out64.reserve((size_t)nslots * sizeof(double));
     if (want32) p.out32.reserve((size_t)nslots * sizeof(float));
@@ -448,11 +449,13 @@ static void load_values(hala_ctx c, tri_plan &p, const double *factor, dbuf &ent
 void load_values64(hala_ctx c, tri_plan &p, const double *factor) {
     load_values<double>(c, p, factor, p.ent_val64, p.dg_val64);
     col_load_values(c, p, factor, false);
+    grid_load_values(c, p, factor, false);
     p.has64 = true;
 }
 void load_values32(hala_ctx c, tri_plan &p, const double *factor) {
     load_values<float>(c, p, factor, p.ent_val32, p.dg_val32);
     col_load_values(c, p, factor, true);
+    grid_load_values(c, p, factor, true);
     if (!p.out32.p) {
         p.out32.reserve((size_t)p.nchunk * WAVE * sizeof(float));
         tri_rearm(c, p);

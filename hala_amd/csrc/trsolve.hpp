@@ -18,6 +18,7 @@
 #pragma once
 #include <vector>
 
+#include "trgrid.hpp"
 #include "util.hpp"
 
 namespace hala_amd {
@@ -76,6 +77,7 @@ struct tri_plan {
     // polled outputs in slot order (re-armed to sentinels at the start of every sweep)
     dbuf out64, out32;
     tri_colplan col;
+    tri_gridplan grid;  // complete 5-/7-point grid patterns (trgrid.hip)
 };
 
 // dependency selection for build_deps()

@@ -61,7 +61,8 @@ int hala_ctx_device(hala_ctx ctx, int *device);
  * "cg_batch_max", "spmv_blocks_per_cu" (the fused SpMV + dot of CG: 0, the
  * default, launches a workgroup per 256-row block, k > 0 at most k per CU over
  * a grid-stride loop).  Paths: "tri_col" (1: column-blocked
- * sweeps where the plan fits, 0: level pool), "tri_stencil" (1: pencil sweeps
+ * sweeps where the plan fits, 0: level pool), "tri_grid" (1: register-wavefront sweeps on
+ * complete 5-/7-point grids while the column options are automatic, 0: column sweeps), "tri_stencil" (1: pencil sweeps
  * for stencil patterns, read when the ILU object is created), "cg_fuse" (1:
  * the sweeps' permutations fused into the PCG vector kernels), "cg_xcd" (1:
  * with cg_fuse, the r update and its scatter into the L sweep's input in
