@@ -9,7 +9,8 @@
 //         x_k += a_k p_k; r_k += (-a_k) Ap_k;
 //         stop if it == max_iter or max_k ||r_k|| < tol (batch_max_norm2);
 //         z = M r; nzr_k = <r_k, z_k>; b_k = nzr_k / zr_k; p_k = b_k p_k; p += 1*z; zr = nzr
-// All columns iterate until the stop.  The dots are this build's canonical
+// The sweeps of all columns run in one launch (64^3, 8 columns: 17.8 ms per solve
+// of 124 passes; one apply after the other 78 ms).  All columns iterate until the stop.  The dots are this build's canonical
 // order per column; the product reads each matrix tile once for up to
 // CGB_GROUP columns.
 #include <algorithm>
@@ -18,6 +19,7 @@
 
 #include "blas1.hpp"
 #include "solvers.hpp"
+#include "spmm.hpp"
 
 namespace hala_amd {
 
@@ -91,68 +93,61 @@ __global__ __launch_bounds__(256) void cgb_start(int n, const double *__restrict
     }
 }
 
-// Ap_k = A p_k for columns c0 .. c0+nc-1 (nc <= CGB_GROUP), each matrix tile
-// read once; fused <p_k, Ap_k>, and block 0 forms a_k = zr_k / <p_k, Ap_k>.
+// Ap_k = A p_k for columns c0 .. c0+nc-1 (nc <= G), each matrix entry read
+// once; fused <p_k, Ap_k>, and block k forms a_k = zr_k / <p_k, Ap_k> (a
+// collector per column: one block collecting eight in turn costs eight
+// reduction latencies).
+template <int G, class TI>
 __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int *__restrict__ pntr,
-                                                const int *__restrict__ indx, const double *__restrict__ vals,
+                                                const TI *__restrict__ indx, const double *__restrict__ vals,
                                                 const double *__restrict__ Pv, double *__restrict__ AP, double *part,
                                                 const double *zr, double *al, cgb_state *st, int *err) {
     if (st->done) return;
-    constexpr int TILE = spmv_tile<double>::value;
-    __shared__ double prod[TILE];
+    __shared__ double sv[spmm_tile<double>::value];
+    __shared__ unsigned so[spmm_tile<double>::value];
     const int64_t nb = ((int64_t)n + CB - 1) / CB;
-    const int r0 = blockIdx.x * SPMV_ROWS, row = r0 + threadIdx.x, rlast = min(r0 + SPMV_ROWS, n);
-    const int bstart = pntr[r0], bend = pntr[rlast];
-    int rs = 0, re = 0;
-    if (row < n) {
-        rs = pntr[row];
-        re = pntr[row + 1];
-    }
-    double acc[CGB_GROUP];
+    const int row = blockIdx.x * SPMV_ROWS + threadIdx.x;
+    const char *xb[G];
 #pragma unroll
-    for (int k = 0; k < CGB_GROUP; k++) acc[k] = 0.0;
-    for (int base = bstart; base < bend; base += TILE) {
-        const int cnt = min(TILE, bend - base);
-        const int lo = max(rs, base), hi = min(re, base + cnt);
+    for (int k = 0; k < G; k++) xb[k] = reinterpret_cast<const char *>(Pv + (int64_t)(c0 + min(k, nc - 1)) * n);
+    double acc[G];
 #pragma unroll
-        for (int k = 0; k < CGB_GROUP; k++) {
-            if (k >= nc) break;
-            const double *p = Pv + (int64_t)(c0 + k) * n;
-            for (int e = threadIdx.x; e < cnt; e += SPMV_ROWS) prod[e] = vals[base + e] * p[indx[base + e]];
-            __syncthreads();
-            double a = acc[k];
-            for (int j = lo; j < hi; j++) a = a + prod[j - base];
-            acc[k] = a;
-            __syncthreads();
-        }
-    }
-    __shared__ double sh[CB];
+    for (int k = 0; k < G; k++) acc[k] = 0.0;
+    csr_block_rowsums<double, G, TI, false, unsigned>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false,
+                                                      false, sv, so, acc);
+    static_assert(G * CB <= spmm_tile<double>::value, "tree scratch");
 #pragma unroll
-    for (int k = 0; k < CGB_GROUP; k++) {
-        if (k >= nc) break;
-        const int64_t o = (int64_t)(c0 + k) * n;
+    for (int k = 0; k < G; k++) {
         double v = 0.0;
-        if (row < n) {
+        if (row < n && k < nc) {
+            const int64_t o = (int64_t)(c0 + k) * n + row;
             const double y = 1.0 * acc[k] + 0.0;
-            AP[o + row] = y;
-            v = Pv[o + row] * y;
+            AP[o] = y;
+            v = Pv[o] * y;
         }
-        v = tree256_1<double>(v, sh);
-        if (threadIdx.x == 0) st_agent(part + (int64_t)(c0 + k) * nb + blockIdx.x, v);
+        acc[k] = v;
     }
-    if (is_collector()) {
-        for (int k = 0; k < nc; k++) {
-            double t = final_pass<double>(part + (int64_t)(c0 + k) * nb, nb, sh, err);
-            if (threadIdx.x == 0) al[c0 + k] = zr[c0 + k] / t;
+    tree256<double, G>(acc, sv);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < G; k++)
+            if (k < nc) st_agent(part + (int64_t)(c0 + k) * nb + blockIdx.x, acc[k]);
+    }
+    for (int k = blockIdx.x; k < nc; k += gridDim.x) {
+        double t = final_pass<double>(part + (int64_t)(c0 + k) * nb, nb, sv, err);
+        if (threadIdx.x == 0) {
+            al[c0 + k] = zr[c0 + k] / t;
+            if (c0 + k == 0) st->it = st->it + 1;
         }
-        if (threadIdx.x == 0 && c0 == 0) st->it = st->it + 1;
     }
 }
 
-// x_k += a_k p_k; r_k += (-a_k) Ap_k; rr_k = <r_k, r_k>
+// x_k += a_k p_k; r_k += (-a_k) Ap_k; rr_k = <r_k, r_k>.  lslot (fused ILU, may
+// be null): r_k also into the first sweep's packed input lxs + k N.
 __global__ __launch_bounds__(256) void cgb_update(int n, const double *__restrict__ Pv, const double *__restrict__ AP,
                                                   double *__restrict__ X, double *__restrict__ R, double *part,
-                                                  const double *al, double *rr, const cgb_state *st, int *err) {
+                                                  const double *al, double *rr, const cgb_state *st, int *err,
+                                                  const int *__restrict__ lslot, double *__restrict__ lxs, int64_t N) {
     if (st->done) return;
     __shared__ double sh[CB * EKB];
     const int64_t nb = ((int64_t)n + CB - 1) / CB, o = (int64_t)blockIdx.y * n;
@@ -166,6 +161,7 @@ __global__ __launch_bounds__(256) void cgb_update(int n, const double *__restric
             X[o + i] = X[o + i] + (1.0 * a) * Pv[o + i];
             double ri = R[o + i] + (-1.0 * a) * AP[o + i];
             R[o + i] = ri;
+            if (lslot) lxs[(int64_t)blockIdx.y * N + lslot[i]] = ri;
             q = ri * ri;
         }
         v[k] = q;
@@ -191,11 +187,13 @@ __global__ void cgb_stop(int nrhs, const double *rr, cgb_state *st) {
     if (it == st->max_iter || rn < st->tol) st->done = 1;
 }
 
-// nzr_k = <r_k, z_k>; b_k = nzr_k / zr_k; zr_k = nzr_k
+// nzr_k = <r_k, z_k>; b_k = nzr_k / zr_k; zr_k = nzr_k.  uslot (fused ILU, may
+// be null): z_k first from the second sweep's packed output uout + k N.
 template <bool IDENT>
-__global__ __launch_bounds__(256) void cgb_rz(int n, const double *__restrict__ R, const double *__restrict__ Z,
+__global__ __launch_bounds__(256) void cgb_rz(int n, const double *__restrict__ R, double *__restrict__ Z,
                                               double *part, double *zr, double *al, const cgb_state *st,
-                                              int *err) {
+                                              int *err, const int *__restrict__ uslot = nullptr,
+                                              const double *__restrict__ uout = nullptr, int64_t N = 0) {
     if (st->done) return;
     __shared__ double sh[CB * EKB];
     const int64_t nb = ((int64_t)n + CB - 1) / CB, o = (int64_t)blockIdx.y * n;
@@ -204,6 +202,7 @@ __global__ __launch_bounds__(256) void cgb_rz(int n, const double *__restrict__ 
     for (int k = 0; k < EKB; k++) {
         int64_t i = ((int64_t)blockIdx.x * EKB + k) * CB + threadIdx.x;
         double ri = i < n ? R[o + i] : 0.0;
+        if (!IDENT && uslot && i < n) Z[o + i] = uout[(int64_t)blockIdx.y * N + uslot[i]];
         v[k] = (i < n) ? ri * (IDENT ? ri : Z[o + i]) : 0.0;
     }
     double *pk = part + blockIdx.y * nb;
@@ -265,9 +264,11 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
     cgb_residual<<<dim3(gs, nrhs), 256, 0, c->stream>>>(n, A->pntr, A->indx, vals, X, B, R);
     HALA_CHECK_LAUNCH();
     const int *gate = &st->done;
-    auto precond = [&](const int *g) {
-        for (int k = 0; k < nrhs; k++) ilu_apply64(M, R + (size_t)k * n, Z + (size_t)k * n, g);
-    };
+    auto precond = [&](const int *g) { ilu_apply64_cols(M, R, Z, nrhs, g); };
+    // the sweeps' gather and scatter ride in the update and the r.z pass where the factor has that form
+    ilu_ends ends{};
+    int64_t N_ = 0;
+    const bool fused = !ident && c->opt.cg_fuse && ilu_fused64_cols(M, nrhs, ends, N_);
     if (ident) {
         cgb_start<true><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, nullptr, Pv, part, zr, wait_error_flag(c));
     } else {
@@ -276,17 +277,36 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
     }
     HALA_CHECK_LAUNCH();
     auto one_pass = [&]() {
-        for (int c0 = 0; c0 < nrhs; c0 += CGB_GROUP)
-            cgb_spmm<<<gs, 256, 0, c->stream>>>(n, c0, std::min(CGB_GROUP, nrhs - c0), A->pntr, A->indx, vals, Pv, AP,
-                                                part, zr, al, st, wait_error_flag(c));
-        cgb_update<<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, Pv, AP, X, R, part, al, rr, st, wait_error_flag(c));
+        for (int c0 = 0; c0 < nrhs; c0 += CGB_GROUP) {
+            const int nc = std::min(CGB_GROUP, nrhs - c0);
+            const short *bo = A->boff.as<short>();
+#define HALA_CGB(GG)                                                                                          \
+    if (bo)                                                                                                   \
+        cgb_spmm<GG, short><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, bo, vals, Pv, AP, part, zr, al, st,  \
+                                                       wait_error_flag(c));                                   \
+    else                                                                                                      \
+        cgb_spmm<GG, int><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->indx, vals, Pv, AP, part, zr, al,   \
+                                                     st, wait_error_flag(c))
+            if (nc > 4) {
+                HALA_CGB(8);
+            } else if (nc > 2) {
+                HALA_CGB(4);
+            } else {
+                HALA_CGB(2);
+            }
+#undef HALA_CGB
+        }
+        cgb_update<<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, Pv, AP, X, R, part, al, rr, st, wait_error_flag(c),
+                                                          fused ? ends.in_slot : nullptr, ends.in, N_);
         cgb_stop<<<1, 1, 0, c->stream>>>(nrhs, rr, st);
         if (ident) {
             cgb_rz<true><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, nullptr, part, zr, al, st, wait_error_flag(c));
             cgb_pupdate<true><<<dim3(gp, nrhs), 256, 0, c->stream>>>(n, R, nullptr, Pv, al, st);
         } else {
-            precond(gate);
-            cgb_rz<false><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, Z, part, zr, al, st, wait_error_flag(c));
+            if (fused) ilu_apply64_cols_mid(M, nrhs, gate);
+            else precond(gate);
+            cgb_rz<false><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, Z, part, zr, al, st, wait_error_flag(c),
+                                                                 fused ? ends.out_slot : nullptr, ends.out, N_);
             cgb_pupdate<false><<<dim3(gp, nrhs), 256, 0, c->stream>>>(n, nullptr, Z, Pv, al, st);
         }
         HALA_CHECK_LAUNCH();

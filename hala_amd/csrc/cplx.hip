@@ -16,35 +16,12 @@
 #include <climits>
 
 #include "ilu.hpp"
+#include "scalar.hpp"
+#include "spmm.hpp"
 #include "spmv.hpp"
 
 namespace hala_amd {
 
-template <class R>
-struct cx {
-    R re, im;
-};
-template <class R>
-__device__ __forceinline__ cx<R> cadd(cx<R> a, cx<R> b) {
-    return {a.re + b.re, a.im + b.im};
-}
-template <class R>
-__device__ __forceinline__ cx<R> csub(cx<R> a, cx<R> b) {
-    return {a.re - b.re, a.im - b.im};
-}
-template <class R>
-__device__ __forceinline__ cx<R> cmul(cx<R> a, cx<R> b) {
-    return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-template <class R>
-__device__ __forceinline__ cx<R> cdiv(cx<R> a, cx<R> b) {
-    const R d = b.re * b.re + b.im * b.im;
-    return {(a.re * b.re + a.im * b.im) / d, (a.im * b.re - a.re * b.im) / d};
-}
-template <class R>
-__device__ __forceinline__ cx<R> cconj(cx<R> a) {
-    return {a.re, -a.im};
-}
 template <class R>
 __device__ __forceinline__ cx<R> ld(const R *p, int64_t i) {
     return {p[2 * i], p[2 * i + 1]};
@@ -142,37 +119,6 @@ __global__ void zscal_kernel(int64_t n, cx<R> a, R *__restrict__ x) {
     for (; i < n; i += stride) st(x, i, cmul(a, ld(x, i)));
 }
 
-// y_i = alpha * (sum_j A_ij x_j, j in CSR order) + beta * y_i  (beta == 0: y not read)
-template <class R>
-__global__ void zspmv_n_kernel(int nrows, const int *__restrict__ pntr, const int *__restrict__ indx,
-                               const R *__restrict__ vals, const R *__restrict__ x, cx<R> alpha, cx<R> beta,
-                               R *__restrict__ y) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nrows) return;
-    cx<R> acc = {R(0), R(0)};
-    for (int j = pntr[i]; j < pntr[i + 1]; j++) acc = cadd(acc, cmul(ld(vals, j), ld(x, indx[j])));
-    cx<R> out = cmul(alpha, acc);
-    if (beta.re != R(0) || beta.im != R(0)) out = cadd(out, cmul(beta, ld(y, i)));
-    st(y, i, out);
-}
-
-// y_k = beta y_k (0 when beta == 0), then y_k += (alpha x_i) * op(A_ik) for the entries
-// of column k in increasing source row i (the reference's scatter order); op = conj for 'C'
-template <class R>
-__global__ void zspmv_t_kernel(int ncols, const int *__restrict__ tpntr, const int *__restrict__ trow,
-                               const int *__restrict__ tmap, const R *__restrict__ vals, const R *__restrict__ x,
-                               cx<R> alpha, cx<R> beta, int conj, R *__restrict__ y) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= ncols) return;
-    cx<R> acc = (beta.re != R(0) || beta.im != R(0)) ? cmul(beta, ld(y, k)) : cx<R>{R(0), R(0)};
-    for (int e = tpntr[k]; e < tpntr[k + 1]; e++) {
-        cx<R> v = ld(vals, tmap[e]);
-        if (conj) v = cconj(v);
-        acc = cadd(acc, cmul(cmul(alpha, ld(x, trow[e])), v));
-    }
-    st(y, k, acc);
-}
-
 // IKJ ILU(0) of the rows of one level (the operation order of the real factor in ilu.hip, complex arithmetic)
 template <class R>
 __global__ void zilu_level_kernel(const int *__restrict__ rows, int count, const int *__restrict__ pntr,
@@ -234,30 +180,26 @@ __global__ void zupper_level(const int *__restrict__ rows, int count, const int 
 template <class R, bool CONJ>
 __global__ void ztri_level(const int *__restrict__ rows, int count, const int *__restrict__ dptr,
                            const int *__restrict__ ddep, const int *__restrict__ dsrc, const int *__restrict__ dgs,
-                           const R *__restrict__ vals, cx<R> alpha, const R *__restrict__ b, R *__restrict__ x) {
+                           const R *__restrict__ vals, cx<R> alpha, const R *b, R *x, int64_t ldb, int64_t inc) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count) return;
+    b += 2 * (blockIdx.y * ldb);  // column blockIdx.y; x may be b (a row reads its own entry and solved ones)
+    x += 2 * (blockIdx.y * ldb);
     const int r = rows[t];
     cx<R> s = {R(0), R(0)};
     for (int k = dptr[r]; k < dptr[r + 1]; k++) {
         cx<R> v = ld(vals, dsrc[k]);
         if (CONJ) v = cconj(v);
-        s = cadd(s, cmul(v, ld(x, ddep[k])));
+        s = cadd(s, cmul(v, ld(x, ddep[k] * inc)));
     }
-    cx<R> y = csub(cmul(alpha, ld(b, r)), s);
+    cx<R> y = csub(cmul(alpha, ld(b, r * inc)), s);
     const int dp = dgs[r];
     if (dp >= 0) {
         cx<R> d = ld(vals, dp);
         if (CONJ) d = cconj(d);
         y = cdiv(y, d);
     }
-    st(x, r, y);
-}
-
-template <class R>
-__global__ void zconj_kernel(int n, R *__restrict__ x) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[2 * (int64_t)i + 1] = -x[2 * (int64_t)i + 1];
+    st(x, r * inc, y);
 }
 
 template <class R>
@@ -347,7 +289,8 @@ void zilu_apply(hala_ilu M, const R *x, R *r) {
 }
 
 template <class R>
-void ztrsv(hala_tri T, char trans, cx<R> alpha, const R *vals, const R *b, R *x) {
+void ztrsv(hala_tri T, char trans, cx<R> alpha, const R *vals, const R *b, R *x, int64_t ldb = 0, int64_t inc = 1,
+           int nrhs = 1) {
     HALA_REQUIRE(T && vals && b && x, HALA_ERR_ARG, "complex trsv: null argument");
     const bool tr = !(trans == 'N' || trans == 'n');
     const bool cj = trans == 'C' || trans == 'c';
@@ -357,16 +300,23 @@ void ztrsv(hala_tri T, char trans, cx<R> alpha, const R *vals, const R *b, R *x)
     tri_plan &p = tr ? T->T : T->N;
     const std::vector<int> &lp = p.h_level_ptr;
     const int *perm = p.perm.as<int>();
-    for (int l = 0; l < p.nlev; l++) {
-        const int cnt = lp[l + 1] - lp[l];
-        if (cnt <= 0) continue;
-        const int g = (cnt + 255) / 256;
-        if (cj)
-            ztri_level<R, true><<<g, 256, 0, c->stream>>>(perm + lp[l], cnt, p.dptr.as<int>(), p.ddep.as<int>(),
-                                                          p.dsrc.as<int>(), p.diag_src.as<int>(), vals, alpha, b, x);
-        else
-            ztri_level<R, false><<<g, 256, 0, c->stream>>>(perm + lp[l], cnt, p.dptr.as<int>(), p.ddep.as<int>(),
-                                                           p.dsrc.as<int>(), p.diag_src.as<int>(), vals, alpha, b, x);
+    for (int k0 = 0; k0 < nrhs; k0 += 65535) {  // (grid limit)
+        const int m = std::min(nrhs - k0, 65535);
+        const R *bk = b + 2 * (k0 * ldb);
+        R *xk = x + 2 * (k0 * ldb);
+        for (int l = 0; l < p.nlev; l++) {
+            const int cnt = lp[l + 1] - lp[l];
+            if (cnt <= 0) continue;
+            const dim3 g((cnt + 255) / 256, m);
+            if (cj)
+                ztri_level<R, true><<<g, 256, 0, c->stream>>>(perm + lp[l], cnt, p.dptr.as<int>(), p.ddep.as<int>(),
+                                                              p.dsrc.as<int>(), p.diag_src.as<int>(), vals, alpha, bk,
+                                                              xk, ldb, inc);
+            else
+                ztri_level<R, false><<<g, 256, 0, c->stream>>>(perm + lp[l], cnt, p.dptr.as<int>(), p.ddep.as<int>(),
+                                                               p.dsrc.as<int>(), p.diag_src.as<int>(), vals, alpha, bk,
+                                                               xk, ldb, inc);
+        }
     }
     HALA_CHECK_LAUNCH();
 }
@@ -378,18 +328,8 @@ void zspmv(hala_csr A, char trans, cx<R> alpha, const R *vals, const R *x, cx<R>
                  HALA_ERR_ARG, "complex spmv: trans must be N, T or C");
     hala_ctx c = A->ctx;
     set_device(c);
-    if (trans == 'N' || trans == 'n') {
-        if (A->nrows == 0) return;
-        zspmv_n_kernel<R><<<(A->nrows + 255) / 256, 256, 0, c->stream>>>(A->nrows, A->pntr, A->indx, vals, x, alpha,
-                                                                         beta, y);
-    } else {
-        ensure_transpose(A);
-        if (A->ncols == 0) return;
-        zspmv_t_kernel<R><<<(A->ncols + 255) / 256, 256, 0, c->stream>>>(
-            A->ncols, A->tp.tpntr.as<int>(), A->tp.trow.as<int>(), A->tp.tmap.as<int>(), vals, x, alpha, beta,
-            (trans == 'C' || trans == 'c') ? 1 : 0, y);
-    }
-    HALA_CHECK_LAUNCH();
+    const cx<R> *v = reinterpret_cast<const cx<R> *>(vals), *xx = reinterpret_cast<const cx<R> *>(x);
+    spmm_columns<cx<R>>(A, trans, alpha, v, xx, 0, 1, false, beta, reinterpret_cast<cx<R> *>(y), 0, 1);
 }
 
 }  // namespace
@@ -444,16 +384,8 @@ using namespace hala_amd;
         return guard([&] {                                                                                       \
             HALA_REQUIRE(A, HALA_ERR_ARG, "complex spmm: null matrix");                                           \
             set_device(A->ctx);                                                                                  \
-            hala_ctx cx_ = A->ctx;                                                                               \
-            spmm_cols(                                                                                           \
-                A, transa, transb, b_rows, b_cols, 2 * sizeof(R), B, ldb, C, ldc,                                \
-                [&](const void *x, void *y) {                                                                    \
-                    zspmv<R>(A, transa, cx<R>{are, aim}, vals, (const R *)x, cx<R>{bre, bim}, (R *)y);           \
-                },                                                                                               \
-                [&](void *t, int n) {                                                                            \
-                    if (n > 0) zconj_kernel<R><<<(n + 255) / 256, 256, 0, cx_->stream>>>(n, (R *)t);             \
-                    HALA_CHECK_LAUNCH();                                                                         \
-                });                                                                                              \
+            spmm<cx<R>>(A, transa, transb, b_rows, b_cols, cx<R>{are, aim}, (const cx<R> *)vals, (const cx<R> *)B, ldb, \
+                        cx<R>{bre, bim}, (cx<R> *)C, ldc);                                                       \
         });                                                                                                      \
     }                                                                                                            \
     int hala_trsv_##SUF(hala_tri T, char trans, R are, R aim, const R *vals, const R *b, R *x) {                 \
@@ -464,9 +396,8 @@ using namespace hala_amd;
         return guard([&] {                                                                                       \
             HALA_REQUIRE(T && vals, HALA_ERR_ARG, "complex trsm: null argument");                                 \
             set_device(T->ctx);                                                                                  \
-            tri_trsm_cols(T, transb, nrhs, 2 * sizeof(R), B, ldb, [&](const void *in, void *out) {                \
-                ztrsv<R>(T, transa, cx<R>{are, aim}, vals, (const R *)in, (R *)out);                              \
-            });                                                                                                  \
+            const trsm_layout l = tri_trsm_layout(T, transb, nrhs, B, ldb);                                       \
+            if (nrhs > 0) ztrsv<R>(T, transa, cx<R>{are, aim}, vals, B, B, l.ldb, l.inc, nrhs);                   \
         });                                                                                                      \
     }
 

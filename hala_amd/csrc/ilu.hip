@@ -295,6 +295,38 @@ void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate) {
     tri_exec<double, double, double>(c, M->U, TRI_SUB, 1.0, M->tmp64.as<double>(), r, gate);
 }
 
+// Vectors swept together at most: enough to fill the chip, and a bound on the packed copies
+static constexpr int64_t COLS_ELEMS = 1ll << 28;
+static int cols_at_once(int64_t N, int nrhs) { return (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, COLS_ELEMS / N, 4096})); }
+
+void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const int *gate) {
+    hala_ctx c = M->ctx;
+    HALA_REQUIRE(M->factored, HALA_ERR_ARG, "ILU apply before factorisation");
+    const int64_t n = M->n;
+    const bool grid = use_grid(M, true);
+    const int step = grid ? cols_at_once(M->L.grid.g.N, nrhs) : 1;
+    for (int k = 0; k < nrhs; k += step) {
+        const int m = std::min(step, nrhs - k);
+        if (grid) grid_exec_pair<double, double>(c, M->L, M->U, x + k * n, n, r + k * n, n, m, gate);
+        else ilu_apply64(M, x + k * n, r + k * n, gate);
+    }
+}
+
+bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
+    if (!use_grid(M, true)) return false;
+    N = M->L.grid.g.N;
+    if (cols_at_once(N, nrhs) < nrhs) return false;
+    grid_reserve(M->ctx, M->L, true, nrhs);
+    grid_reserve(M->ctx, M->U, true, nrhs);
+    e = ilu_ends{M->L.grid.slot.as<int>(), M->L.grid.in64.as<double>(), M->L.grid.slot.as<int>(),
+                 M->U.grid.out64.as<double>(), false};
+    return true;
+}
+
+void ilu_apply64_cols_mid(hala_ilu M, int nrhs, const int *gate) {
+    grid_pair_mid64(M->ctx, M->L, M->U, nrhs, gate);
+}
+
 void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate) {
     hala_ctx c = M->ctx;
     HALA_REQUIRE(M->factored && M->has32, HALA_ERR_ARG, "FP32 ILU apply needs hala_ilu_factor_f64(..., want_f32=1)");

@@ -1,6 +1,5 @@
 // ilu.hpp -- ILU(0) handle (the gpu_ilu of gpu/hala_gpu_ilu.hpp:45-195).
 #pragma once
-#include <functional>
 #include <memory>
 #include "spmv.hpp"
 #include "trsolve.hpp"
@@ -49,11 +48,12 @@ struct hala_tri_s {
 };
 
 namespace hala_amd {
-// Multi-right-hand-side triangular solve (hala_trsm_*): B <- op(T)^-1 (alpha B)
-// column by column through `col`, which solves one column from a contiguous
-// input into a contiguous output.  esize: bytes per element.
-void tri_trsm_cols(hala_tri T, char transb, int nrhs, size_t esize, void *B, int ldb,
-                   const std::function<void(const void *, void *)> &col);
+// The columns of op(B) in hala_trsm_*: element r of column k at B[k ldb + r inc]
+// (checks the arguments; ldb < 0: the minimum).
+struct trsm_layout {
+    int64_t ldb, inc;
+};
+trsm_layout tri_trsm_layout(hala_tri T, char transb, int nrhs, const void *B, int ldb);
 // r = (LU)^-1 x in the requested precision (see hala_ilu_apply_*)
 // gate (nullable, device flag): skip the apply when *gate != 0 (solver stop flag)
 void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
@@ -72,6 +72,11 @@ struct ilu_ends {
 };
 bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e);
 void ilu_apply64_mid(hala_ilu M, bool transposed, const int *gate, const hala_amd::col_axpy *ax = nullptr);
+// nrhs vectors at once: column k at x + k n, r + k n.  The fused form as above
+// over packed vectors of stride N (grid sweeps only).
+void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const int *gate);
+bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N);
+void ilu_apply64_cols_mid(hala_ilu M, int nrhs, const int *gate);
 void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_apply_t64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_prepare_adjoint(hala_ilu M);

@@ -467,6 +467,9 @@ bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req) {
             HALA_CHECK_LAUNCH();
             const bool upward = fetch_i32(c, gap.as<int>()) != 0;
             if (upward && (c->opt.tri_col_split == 0 || ncol > c->num_cus)) B = 1;
+            p.col.upward = upward && B > 1;
+        } else {
+            p.col.upward = false;
         }
         const int A = ncol / B;
         // the widest level spreads over ncol cells, so one holds at least maxw / ncol
@@ -675,6 +678,8 @@ struct col_args {
     T *out;
     T *hand;              // HAND: the next sweep's input, at the slot each record carries (col_set_handoff)
     int ncol;             // columns; workgroups past them are helpers
+    int nrhs;             // vectors swept at once (no helpers if more than one), xstride slots apart
+    int64_t xstride;
     T *arm;               // helpers: re-arm arm[0 .. narm) with sentinels (another sweep's polled output)
     int narm;
     col_axpy ax;          // helpers: ax.x += *ax.alpha * ax.p over ax.n rows (ax.x null: none)
@@ -791,7 +796,7 @@ __global__ __launch_bounds__(BT) void tri_col_kernel(col_args<T, TOUT> a) {
         win[zidx] = T(0);
     }
     __syncthreads();
-    const int col = col_s;
+    const int col = col_s / a.nrhs, rhs = col_s % a.nrhs;
     if (col >= a.ncol) {  // helper
         const int nh = (int)gridDim.x - a.ncol;
         for (int s = (col - a.ncol) * (int)blockDim.x + t; s < a.narm; s += nh * (int)blockDim.x)
@@ -810,6 +815,8 @@ __global__ __launch_bounds__(BT) void tri_col_kernel(col_args<T, TOUT> a) {
         }
         return;
     }
+    const T *const axs = a.xs + rhs * a.xstride;
+    T *const aout = a.out + rhs * a.xstride;
     const int first = a.colrange[2 * col], last = a.colrange[2 * col + 1];
 
     const int nl = last - first + 1;
@@ -829,7 +836,7 @@ __global__ __launch_bounds__(BT) void tri_col_kernel(col_args<T, TOUT> a) {
         auto raw = [&](int lam, int e) { return a.ext_slot[cis[lam * CI + 3] + l + WAVE * e]; };
         // polled address: workgroup-uniform base + 32-bit byte offset (no 64-bit
         // register pair per slot, so a freshly loaded slot is used where it lands)
-        const char *obase = reinterpret_cast<const char *>(a.out);
+        const char *obase = reinterpret_cast<const char *>(aout);
         auto at = [&](int slot) { return reinterpret_cast<const T *>(obase + (unsigned)slot * (unsigned)sizeof(T)); };
         T ev[PE][EL];
         int esr[P][EL];
@@ -903,7 +910,7 @@ __global__ __launch_bounds__(BT) void tri_col_kernel(col_args<T, TOUT> a) {
             const unsigned s = (unsigned)(slot0 + t);
             r.slot = t < size ? (int)s : -1;
             // slot arrays are padded past their end: idle lanes read in bounds
-            r.xin = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(a.xs) + s * (unsigned)sizeof(T));
+            r.xin = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(axs) + s * (unsigned)sizeof(T));
             const int4 *src = reinterpret_cast<const int4 *>(reinterpret_cast<const char *>(a.rec) + s * (unsigned)(16 * NQ));
 #pragma unroll
             for (int i = 0; i < NQ; i++) r.q[i] = src[i];
@@ -960,7 +967,7 @@ __global__ __launch_bounds__(BT) void tri_col_kernel(col_args<T, TOUT> a) {
                 if (!UNIT) acc = acc / rec_val<T>(r.q, 2 * MAXD);
                 win[(lvl % K) * CP + t] = acc;
                 if (valid)
-                    st_agent(reinterpret_cast<T *>(reinterpret_cast<char *>(a.out) + (unsigned)r.slot * (unsigned)sizeof(T)),
+                    st_agent(reinterpret_cast<T *>(reinterpret_cast<char *>(aout) + (unsigned)r.slot * (unsigned)sizeof(T)),
                              acc);
                 if (HAND && valid)
                     *reinterpret_cast<T *>(reinterpret_cast<char *>(a.hand) +
@@ -986,7 +993,7 @@ void launch_col_el(hala_ctx c, const tri_colplan &q, col_args<T, TOUT> &a, size_
     constexpr int PE = poll_ahead(MAXD);
     static_assert(PE <= PE_MAX, "LDS sized for PE_MAX polls in flight");
     constexpr int BT = (MAXD == 4 ? CPMAX : CPMAX_LONG) + WAVE;
-    const int nwg = q.ncol + (a.narm > 0 || a.ax.x ? ARM_HELPERS : 0);
+    const int nwg = q.ncol * a.nrhs + (a.narm > 0 || a.ax.x ? ARM_HELPERS : 0);
     tri_col_kernel<T, TOUT, MODE, UNIT, HAND, MAXD, P, PE, EL, BT><<<dim3(nwg), dim3(q.CP + WAVE), lds, c->stream>>>(a);
 }
 
@@ -1022,7 +1029,7 @@ namespace {
 // re-armed by helper workgroups.
 template <class T, class TOUT>
 void col_sweep(hala_ctx c, tri_plan &p, int mode, T alpha, const int *gate, tri_plan *next, T *arm, int narm,
-               const col_axpy *ax = nullptr) {
+               const col_axpy *ax = nullptr, int nrhs = 0) {
     constexpr bool is64 = sizeof(T) == 8;
     tri_colplan &q = p.col;
     col_args<T, TOUT> a;
@@ -1036,8 +1043,14 @@ void col_sweep(hala_ctx c, tri_plan &p, int mode, T alpha, const int *gate, tri_
     a.xs = is64 ? reinterpret_cast<T *>(q.xs64.p) : reinterpret_cast<T *>(q.xs32.p);
     a.alpha = alpha;
     a.out = is64 ? reinterpret_cast<T *>(p.out64.p) : reinterpret_cast<T *>(p.out32.p);
+    if (nrhs > 0) {  // vectors in buffers of their own
+        a.xs = q.mxs.as<T>();
+        a.out = q.mout.as<T>();
+    }
     a.hand = nullptr;
     a.ncol = q.ncol;
+    a.nrhs = std::max(nrhs, 1);
+    a.xstride = (int64_t)p.nchunk * WAVE + BTMAX;
     a.arm = arm;
     a.narm = arm ? narm : 0;
     a.ax = ax ? *ax : col_axpy{nullptr, nullptr, nullptr, 0};
@@ -1086,6 +1099,46 @@ void tri_col_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TOUT *in, TO
         HALA_CHECK_LAUNCH();
     }
 }
+
+namespace {
+
+// strided vectors (element r of vector blockIdx.y at b[y ldb + r inc]) into slot order, and back
+template <class T>
+__global__ void col_gather_cols(int nslots, int64_t stride, const int *__restrict__ chunk_row, const T *__restrict__ b,
+                                int64_t ldb, int64_t inc, T *__restrict__ xs, T *__restrict__ out) {
+    const int s = xcd_block((nslots + 255) / 256) * 256 + threadIdx.x;
+    if (s >= nslots) return;
+    const int64_t o = blockIdx.y * stride + s;
+    out[o] = sentinel<T>();
+    const int r = chunk_row[s];
+    if (r >= 0) xs[o] = b[blockIdx.y * ldb + r * inc];
+}
+template <class T>
+__global__ void col_scatter_cols(int n, int64_t stride, const int *__restrict__ slot_of_row, const T *__restrict__ out,
+                                 T *__restrict__ b, int64_t ldb, int64_t inc) {
+    const int r = xcd_block((n + 255) / 256) * 256 + threadIdx.x;
+    if (r < n) b[blockIdx.y * ldb + r * inc] = out[blockIdx.y * stride + slot_of_row[r]];
+}
+
+}  // namespace
+
+template <class T>
+void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
+    tri_colplan &q = p.col;
+    const int nslots = p.nchunk * WAVE;
+    const int64_t stride = nslots + BTMAX;
+    q.mxs.reserve((size_t)(stride * nrhs) * sizeof(T));
+    q.mout.reserve((size_t)(stride * nrhs) * sizeof(T));
+    col_gather_cols<T><<<dim3(xcd_grid((nslots + 255) / 256), nrhs), 256, 0, c->stream>>>(
+        nslots, stride, p.chunk_row.as<int>(), b, ldb, inc, q.mxs.as<T>(), q.mout.as<T>());
+    HALA_CHECK_LAUNCH();
+    col_sweep<T, T>(c, p, mode, alpha, nullptr, nullptr, nullptr, 0, nullptr, nrhs);
+    col_scatter_cols<T><<<dim3(xcd_grid((p.n + 255) / 256), nrhs), 256, 0, c->stream>>>(
+        p.n, stride, p.slot_of_row.as<int>(), q.mout.as<T>(), b, ldb, inc);
+    HALA_CHECK_LAUNCH();
+}
+template void tri_col_cols<double>(hala_ctx, tri_plan &, int, double, double *, int64_t, int64_t, int);
+template void tri_col_cols<float>(hala_ctx, tri_plan &, int, float, float *, int64_t, int64_t, int);
 
 void col_sweep64(hala_ctx c, tri_plan &p, int mode, double alpha, const int *gate, tri_plan *next, tri_plan *arm,
                  const col_axpy *ax) {

@@ -4,6 +4,7 @@
 #include <climits>
 #include <type_traits>
 
+#include "spmv.hpp"
 #include "trsolve.hpp"
 
 namespace hala_amd {
@@ -222,6 +223,39 @@ void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *o
     kernel<<<blocks, 256, 0, c->stream>>>(a);
     HALA_CHECK_LAUNCH();
 }
+
+// 64^3 lower triangle, 8 vectors: 155 us, of which the values' packing is 45;
+// one solve per vector took 926 us.
+template <class T>
+void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
+    constexpr bool is64 = sizeof(T) == 8;
+    constexpr int64_t ELEMS = 1ll << 28;  // elements of one packed copy at most
+    const bool grid = grid_usable(c, p, is64), col = !grid && col_usable(c, p, is64) && !p.col.upward;
+    const int64_t per = grid ? p.grid.g.N : (int64_t)p.nchunk * WAVE + SLOT_PAD;
+    const int at_once = (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, ELEMS / per, 4096}));
+    if (grid || (col && at_once > 1)) {
+        for (int k = 0; k < nrhs; k += at_once) {
+            const int m = std::min(at_once, nrhs - k);
+            T *bk = b + k * ldb;
+            if (grid) grid_exec<T, T>(c, p, mode, alpha, bk, ldb, bk, ldb, m, nullptr, inc);
+            else tri_col_cols<T>(c, p, mode, alpha, bk, ldb, inc, m);
+        }
+        return;
+    }
+    tmp_scope ts(c);
+    dbuf &t1 = ts.get();
+    dbuf &t2 = ts.get();
+    t1.reserve((size_t)p.n * sizeof(T));
+    if (inc != 1) t2.reserve((size_t)p.n * sizeof(T));
+    for (int k = 0; k < nrhs; k++) {
+        T *bk = b + k * ldb;
+        strided_copy(c, p.n, sizeof(T), bk, inc, t1.p, 1);
+        tri_exec<T, T, T>(c, p, mode, alpha, t1.as<T>(), inc == 1 ? bk : t2.as<T>());
+        if (inc != 1) strided_copy(c, p.n, sizeof(T), t2.p, 1, bk, inc);
+    }
+}
+template void tri_exec_cols<double>(hala_ctx, tri_plan &, int, double, double *, int64_t, int64_t, int);
+template void tri_exec_cols<float>(hala_ctx, tri_plan &, int, float, float *, int64_t, int64_t, int);
 
 template void tri_exec<double, double, double>(hala_ctx, tri_plan &, int, double, const double *, double *, const int *);
 template void tri_exec<float, double, double>(hala_ctx, tri_plan &, int, float, const double *, double *, const int *);

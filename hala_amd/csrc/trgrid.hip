@@ -172,12 +172,12 @@ __global__ void grid_arm(T *__restrict__ x, int64_t n) {
 // (nullable): nf values per vector refilled with sentinels (the sweep's frames).
 template <class T, class TIN>
 __global__ __launch_bounds__(256) void grid_gather(int n, int64_t N, const int *__restrict__ slot,
-                                                   const TIN *__restrict__ in, int64_t ldin, T *__restrict__ xp,
-                                                   T *__restrict__ arm, int64_t nf, const int *gate) {
+                                                   const TIN *__restrict__ in, int64_t ldin, int64_t inc,
+                                                   T *__restrict__ xp, T *__restrict__ arm, int64_t nf, const int *gate) {
     if (gate && *gate) return;
     const int r = xcd_block((n + 255) / 256) * 256 + threadIdx.x;
     const int64_t o = (int64_t)blockIdx.y * N;
-    if (r < n) xp[o + slot[r]] = (T)in[(int64_t)blockIdx.y * ldin + r];
+    if (r < n) xp[o + slot[r]] = (T)in[(int64_t)blockIdx.y * ldin + r * inc];
     if (arm)
         for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < nf; e += (int64_t)gridDim.x * 256)
             arm[(int64_t)blockIdx.y * nf + e] = sentinel<T>();
@@ -187,10 +187,10 @@ __global__ __launch_bounds__(256) void grid_gather(int n, int64_t N, const int *
 template <class T, class TOUT>
 __global__ __launch_bounds__(256) void grid_scatter(int n, int64_t N, const int *__restrict__ slot,
                                                     const T *__restrict__ xp, TOUT *__restrict__ out, int64_t ldout,
-                                                    const int *gate) {
+                                                    int64_t inc, const int *gate) {
     if (gate && *gate) return;
     const int r = xcd_block((n + 255) / 256) * 256 + threadIdx.x;
-    if (r < n) out[(int64_t)blockIdx.y * ldout + r] = (TOUT)xp[(int64_t)blockIdx.y * N + slot[r]];
+    if (r < n) out[(int64_t)blockIdx.y * ldout + r * inc] = (TOUT)xp[(int64_t)blockIdx.y * N + slot[r]];
 }
 
 // ---- the sweep --------------------------------------------------------------
@@ -807,16 +807,16 @@ void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs) {
 
 template <class T, class TIO>
 void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_t ldin, TIO *out, int64_t ldout,
-               int nrhs, const int *gate) {
+               int nrhs, const int *gate, int64_t inc) {
     tri_gridplan &q = p.grid;
     grid_reserve(c, p, sizeof(T) == 8, nrhs);
     T *xp = buf<T>(q.in64, q.in32), *op = buf<T>(q.out64, q.out32), *fr = buf<T>(q.fr64, q.fr32);
     const int64_t nf = frame_values(q.g);
     const dim3 g((unsigned)xcd_grid((p.n + 255) / 256), (unsigned)nrhs);
-    grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(p.n, q.g.N, q.slot.as<int>(), in, ldin, xp, fr, nf, gate);
+    grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(p.n, q.g.N, q.slot.as<int>(), in, ldin, inc, xp, fr, nf, gate);
     HALA_CHECK_LAUNCH();
     sweep<T>(c, p, mode, alpha, xp, op, fr, fr + nf * nrhs, nrhs, gate);
-    grid_scatter<T, TIO><<<g, 256, 0, c->stream>>>(p.n, q.g.N, q.slot.as<int>(), op, out, ldout, gate);
+    grid_scatter<T, TIO><<<g, 256, 0, c->stream>>>(p.n, q.g.N, q.slot.as<int>(), op, out, ldout, inc, gate);
     HALA_CHECK_LAUNCH();
 }
 
@@ -842,18 +842,19 @@ void grid_exec_pair(hala_ctx c, tri_plan &first, tri_plan &second, const TIO *in
     grid_reserve(c, second, sizeof(T) == 8, nrhs);
     const tri_gridplan &q = first.grid;
     const dim3 g((unsigned)xcd_grid((first.n + 255) / 256), (unsigned)nrhs);
-    grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(), in, ldin, buf<T>(q.in64, q.in32),
-                                                  nullptr, 0, gate);
+    grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(), in, ldin, 1,
+                                                  buf<T>(q.in64, q.in32), nullptr, 0, gate);
     HALA_CHECK_LAUNCH();
     pair_mid<T>(c, first, second, nrhs, gate);
     grid_scatter<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(),
-                                                   buf<T>(second.grid.out64, second.grid.out32), out, ldout, gate);
+                                                   buf<T>(second.grid.out64, second.grid.out32), out, ldout, 1,
+                                                   gate);
     HALA_CHECK_LAUNCH();
 }
 
 #define HALA_GRID(T, TIO)                                                                                           \
     template void grid_exec<T, TIO>(hala_ctx, tri_plan &, int, T, const TIO *, int64_t, TIO *, int64_t, int,        \
-                                    const int *);                                                                  \
+                                    const int *, int64_t);                                                                  \
     template void grid_exec_pair<T, TIO>(hala_ctx, tri_plan &, tri_plan &, const TIO *, int64_t, TIO *, int64_t,    \
                                          int, const int *);
 HALA_GRID(double, double)

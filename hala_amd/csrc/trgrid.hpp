@@ -57,10 +57,11 @@ bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second,
 // Packed vectors for nrhs right-hand sides.
 void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs);
 
-// out_k = op^-1 in_k for nrhs vectors in natural order (in + k ldin, out + k ldout), TRI_SUB / TRI_SUM as tri_exec.
+// out_k = op^-1 in_k for nrhs vectors in natural order (element r of vector k at in[k ldin + r inc] and
+// out[k ldout + r inc]; out may be in), TRI_SUB / TRI_SUM as tri_exec.
 template <class T, class TIO>
 void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_t ldin, TIO *out, int64_t ldout,
-               int nrhs, const int *gate);
+               int nrhs, const int *gate, int64_t inc = 1);
 // The two sweeps of an apply (TRI_SUB, first forward, second backward or the
 // reverse), natural order in and out.  Plans run as a pair are only run as one.
 template <class T, class TIO>

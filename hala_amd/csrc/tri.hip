@@ -53,8 +53,7 @@ void strided_copy(hala_ctx c, int n, size_t esize, const void *src, int64_t ss, 
 
 static bool is_n(char t) { return t == 'N' || t == 'n'; }
 
-void tri_trsm_cols(hala_tri T, char transb, int nrhs, size_t esize, void *B, int ldb,
-                   const std::function<void(const void *, void *)> &col) {
+trsm_layout tri_trsm_layout(hala_tri T, char transb, int nrhs, const void *B, int ldb) {
     HALA_REQUIRE(T && (B || nrhs == 0) && nrhs >= 0, HALA_ERR_ARG, "hala_trsm: bad argument");
     HALA_REQUIRE(is_n(transb) || transb == 'T' || transb == 't' || transb == 'C' || transb == 'c', HALA_ERR_ARG,
                  "hala_trsm: transb must be N, T or C");
@@ -62,24 +61,27 @@ void tri_trsm_cols(hala_tri T, char transb, int nrhs, size_t esize, void *B, int
     const bool bn = is_n(transb);
     if (ldb < 0) ldb = bn ? n : nrhs;
     HALA_REQUIRE(ldb >= (bn ? n : nrhs) && ldb >= 1, HALA_ERR_ARG, "hala_trsm: ldb below the minimum");
+    // column k of op(B): column k of the stored B, or its row k
+    return bn ? trsm_layout{ldb, 1} : trsm_layout{1, ldb};
+}
+
+static bool trans_checked(char trans, const char *who) {
+    const bool tr = !is_n(trans);
+    HALA_REQUIRE(!tr || trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', HALA_ERR_ARG,
+                 std::string(who) + ": trans must be N, T or C");
+    return tr;
+}
+
+// FP32 values into the plan (its loader takes FP64 values; the widening and its narrowing back are exact)
+static void load_narrow(hala_tri T, tri_plan &p, const float *vals) {
     hala_ctx c = T->ctx;
     tmp_scope ts(c);
-    dbuf &t1 = ts.get();
-    dbuf &t2 = ts.get();
-    t1.reserve((size_t)n * esize);
-    t2.reserve((size_t)n * esize);
-    char *b = static_cast<char *>(B);
-    for (int i = 0; i < nrhs; i++) {
-        if (bn) {  // column i is contiguous: a copy of it is the right-hand side, the solution lands in place
-            char *bc = b + (size_t)i * (size_t)ldb * esize;
-            HALA_HIP(hipMemcpyAsync(t1.p, bc, (size_t)n * esize, hipMemcpyDeviceToDevice, c->stream));
-            col(t1.p, bc);
-        } else {  // column i is row i of the stored B: gather, solve, scatter
-            strided_copy(c, n, esize, b + (size_t)i * esize, ldb, t1.p, 1);
-            col(t1.p, t2.p);
-            strided_copy(c, n, esize, t2.p, 1, b + (size_t)i * esize, ldb);
-        }
-    }
+    dbuf &w = ts.get();
+    w.reserve((size_t)T->nnz * sizeof(double));
+    f32_to_f64<<<(int)((T->nnz + 255) / 256), 256, 0, c->stream>>>(T->nnz, vals, w.as<double>());
+    HALA_CHECK_LAUNCH();
+    load_values32(c, p, w.as<double>());
+    HALA_HIP(hipStreamSynchronize(c->stream));
 }
 
 }  // namespace hala_amd
@@ -156,10 +158,7 @@ int hala_trsv_f64(hala_tri T, char trans, double alpha, const double *vals, cons
         HALA_REQUIRE(T && vals && b && x, HALA_ERR_ARG, "hala_trsv_f64: null argument");
         hala_ctx c = T->ctx;
         set_device(c);
-        bool tr = !(trans == 'N' || trans == 'n');
-        HALA_REQUIRE(!tr || trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', HALA_ERR_ARG,
-                     "hala_trsv_f64: trans must be N, T or C");
-        tri_plan &p = tr ? T->T : T->N;
+        tri_plan &p = trans_checked(trans, "hala_trsv_f64") ? T->T : T->N;
         load_values64(c, p, vals);
         tri_exec<double, double, double>(c, p, TRI_SUM, alpha, b, x);
         if (c->opt.sync_checks) check_wait_error(c);
@@ -173,34 +172,29 @@ int hala_trsv_f32(hala_tri T, char trans, float alpha, const float *vals, const 
         HALA_REQUIRE(T && vals && b && x, HALA_ERR_ARG, "hala_trsv_f32: null argument");
         hala_ctx c = T->ctx;
         set_device(c);
-        bool tr = !(trans == 'N' || trans == 'n');
-        HALA_REQUIRE(!tr || trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', HALA_ERR_ARG,
-                     "hala_trsv_f32: trans must be N, T or C");
-        tri_plan &p = tr ? T->T : T->N;
-        {  // the plan's loader takes FP64 values; the widening and its narrowing back are exact
-            tmp_scope ts(c);
-            dbuf &w = ts.get();
-            w.reserve((size_t)T->nnz * sizeof(double));
-            f32_to_f64<<<(int)((T->nnz + 255) / 256), 256, 0, c->stream>>>(T->nnz, vals, w.as<double>());
-            HALA_CHECK_LAUNCH();
-            load_values32(c, p, w.as<double>());
-            HALA_HIP(hipStreamSynchronize(c->stream));
-        }
+        tri_plan &p = trans_checked(trans, "hala_trsv_f32") ? T->T : T->N;
+        load_narrow(T, p, vals);
         tri_exec<float, float, float>(c, p, TRI_SUM, alpha, b, x);
         if (c->opt.sync_checks) check_wait_error(c);
     });
 }
 
+// B <- op(T)^-1 (alpha B): the values into the plan once, then every column
+// (64^3 lower triangle, 8 columns: values, copies, sweep and a host wait per
+// column took 1030 us).
 int hala_trsm_f64(hala_tri T, char transa, char transb, int nrhs, double alpha, const double *vals, double *B,
                   int ldb) {
     HALA_RANGE();
     return guard([&] {
         HALA_REQUIRE(T && vals, HALA_ERR_ARG, "hala_trsm_f64: null argument");
-        set_device(T->ctx);
-        tri_trsm_cols(T, transb, nrhs, sizeof(double), B, ldb, [&](const void *in, void *out) {
-            const int rc = hala_trsv_f64(T, transa, alpha, vals, (const double *)in, (double *)out);
-            if (rc != HALA_OK) throw status_error{rc, hala_last_error()};
-        });
+        hala_ctx c = T->ctx;
+        set_device(c);
+        const trsm_layout l = tri_trsm_layout(T, transb, nrhs, B, ldb);
+        if (nrhs == 0) return;
+        tri_plan &p = trans_checked(transa, "hala_trsm_f64") ? T->T : T->N;
+        load_values64(c, p, vals);
+        tri_exec_cols<double>(c, p, TRI_SUM, alpha, B, l.ldb, l.inc, nrhs);
+        if (c->opt.sync_checks) check_wait_error(c);
     });
 }
 
@@ -208,11 +202,14 @@ int hala_trsm_f32(hala_tri T, char transa, char transb, int nrhs, float alpha, c
     HALA_RANGE();
     return guard([&] {
         HALA_REQUIRE(T && vals, HALA_ERR_ARG, "hala_trsm_f32: null argument");
-        set_device(T->ctx);
-        tri_trsm_cols(T, transb, nrhs, sizeof(float), B, ldb, [&](const void *in, void *out) {
-            const int rc = hala_trsv_f32(T, transa, alpha, vals, (const float *)in, (float *)out);
-            if (rc != HALA_OK) throw status_error{rc, hala_last_error()};
-        });
+        hala_ctx c = T->ctx;
+        set_device(c);
+        const trsm_layout l = tri_trsm_layout(T, transb, nrhs, B, ldb);
+        if (nrhs == 0) return;
+        tri_plan &p = trans_checked(transa, "hala_trsm_f32") ? T->T : T->N;
+        load_narrow(T, p, vals);
+        tri_exec_cols<float>(c, p, TRI_SUM, alpha, B, l.ldb, l.inc, nrhs);
+        if (c->opt.sync_checks) check_wait_error(c);
     });
 }
 

@@ -50,6 +50,8 @@ struct tri_colplan {
     dbuf spar;                   // per slot: parity of its level within its column (which external buffer it reads)
     dbuf val64, val32;           // packed row records (see col_pack)
     dbuf xs64, xs32;             // input, gathered into slot order per sweep
+    dbuf mxs, mout;              // the same and the polled output for several right-hand sides at once
+    bool upward = false;         // some column waits on a higher-numbered one (every column then needs a CU)
     bool hand64 = false;         // val64 carries hand-off slots (col_set_handoff)
 };
 
@@ -132,12 +134,20 @@ void load_values32(hala_ctx c, tri_plan &p, const double *factor);
 // gate (nullable, device): when *gate != 0 at launch the solve does nothing.
 template <class T, class TIN, class TOUT>
 void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *out_nat, const int *gate = nullptr);
+// The same for nrhs vectors in place: element r of vector k at b[k ldb + r inc].
+// Grid and column sweeps take many vectors in one launch (they are bound by
+// latency: more of them in flight cost little more than one); other plans go
+// vector by vector through a contiguous copy.
+template <class T>
+void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs);
 
 // Column-blocked layout (trcol.hip): built after build_schedule when the
 // pattern allows it (returns false and leaves p.col.ok unset otherwise);
 // ncol_req = 0 picks the column count.  tri_exec uses it when present and
 // enabled (option tri_col).
 bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req);
+template <class T>
+void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs);
 void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
 bool col_usable(hala_ctx c, const tri_plan &p, bool is64);
 // next (nullable; FP64, TRI_SUB, unit p with hand-off slots, see

@@ -1,0 +1,156 @@
+"""Several vectors at once: the fused sparse-times-dense product around its
+group sizes and tiles, triangular solves with many right-hand sides on the
+grid, column and level-pool sweeps, and multi-right-hand-side ILU-PCG -- every
+column bit for bit what the oracle (or the one-column call, pinned elsewhere)
+gives."""
+import numpy as np
+import pytest
+import torch
+
+import hala_amd as H
+import oracle
+from hala_amd import stencils as st
+from tests.conftest import bits
+
+pytestmark = pytest.mark.gpu
+
+
+def host(t):
+    return t.detach().cpu().numpy()
+
+
+def raw(a):
+    a = np.ascontiguousarray(a)
+    return bits(a.view(np.float64 if a.dtype in (np.complex128, np.float64) else np.float32))
+
+
+def ragged(nr, nc, seed, longest):
+    """Rows of 0 .. longest entries, one row with all nc columns."""
+    rng = np.random.default_rng(seed)
+    p, i = [0], []
+    for r in range(nr):
+        k = nc if r == nr // 3 else int(rng.integers(0, longest + 1))
+        i.extend(np.sort(rng.choice(nc, size=min(k, nc), replace=False)))
+        p.append(len(i))
+    return np.array(p, np.int32), np.array(i, np.int32)
+
+
+MATS = {
+    "band": lambda: (lambda p, i, v: (p, i, len(p) - 1))(*st.laplace3d(9, 8, 8)),  # int16 offsets, tile remainders
+    "ragged": lambda: (*ragged(517, 3000, 3, 9), 3000),  # a row and a tile longer than the staging
+    "wide": lambda: (*ragged(260, 70000, 4, 5), 70000),  # int32 columns
+    "one": lambda: (np.array([0, 1], np.int32), np.array([0], np.int32), 1),
+    "empty": lambda: (np.zeros(301, np.int32), np.zeros(0, np.int32), 40),
+}
+
+
+@pytest.mark.parametrize("mat", sorted(MATS))
+@pytest.mark.parametrize("ct", [np.float64, np.float32, np.complex128, np.complex64])
+def test_spmm_columns(engine, mat, ct):
+    p, i, nc = MATS[mat]()
+    nr = len(p) - 1
+    rng = np.random.default_rng(9)
+    cplx = np.issubdtype(ct, np.complexfloating)
+
+    def rnd(*shape):
+        a = rng.uniform(-1, 1, shape)
+        return (a + 1j * rng.uniform(-1, 1, shape) if cplx else a).astype(ct)
+
+    v = rnd(len(i))
+    A = H.make_sparse_matrix(engine, nc, engine.load(p), engine.load(i), engine.load(v))
+    z = np.zeros(0)
+    for ta in ("N", "T", "C") if cplx else ("N", "T"):
+        k, m = (nc, nr) if ta == "N" else (nr, nc)
+        for tb, cols, beta in (("N", 1, 0.0), ("N", 2, 0.5), ("N", 3, 0.0), ("N", 5, 0.5), ("N", 8, 0.0), ("N", 9, 0.5),
+                               ("T", 5, 0.0), ("C", 9, 0.5)):
+            ldb, ldc = (k + 3 if tb == "N" else cols + 1), m + 2
+            B = rnd(cols if tb == "N" else k, ldb)  # column-major: row q of this array is column q of B
+            C0 = rnd(cols, ldc)
+            gC = engine.load(C0)
+            A.gemm(ta, tb, k if tb == "N" else cols, cols if tb == "N" else k, 1.5, engine.load(B), ldb, beta, gC, ldc)
+            got = host(gC)
+            assert np.array_equal(raw(got[:, m:]), raw(C0[:, m:]))  # nothing written past a column
+            for c in sorted({0, cols - 1}):
+                x = np.ascontiguousarray(B[c, :k] if tb == "N" else (B[:, c].conj() if tb == "C" else B[:, c]))
+                y = np.ascontiguousarray(C0[c, :m])
+                if ct == np.float64:
+                    y = oracle.spmv(ta, nr, nc, 1.5, p, i, v, x, beta, y)
+                elif ct == np.float32 and ta == "N":
+                    y = oracle.spmv_f32(p, i, v, x, alpha=1.5, beta=beta, y=y)
+                else:  # FP32 'T': the complex product with zero imaginary parts, term by term
+                    w = ct if cplx else np.complex64
+                    yc = y.astype(w)
+                    oracle.zspmv(ta, nr, nc, 1.5 + 0j, p, i, v.astype(w), x.astype(w), complex(beta), yc)
+                    y = yc if cplx else yc.real.astype(np.float32)
+                assert np.array_equal(raw(got[c, :m]), raw(y)), (ta, tb, cols, c)
+
+
+TRI = {
+    "grid3": lambda: st.laplace3d(21, 9, 10),
+    "grid2": lambda: st.laplace2d(30, 66),
+    "column": lambda: st.convdiff27(12, seed=3),
+    "pool": lambda: st.laplace2d(10, 6),
+}
+
+
+@pytest.mark.parametrize("name", sorted(TRI))
+@pytest.mark.parametrize("uplo", ["L", "U"])
+def test_trsm_many_columns(engine, name, uplo):
+    p, i, v = TRI[name]()
+    n = len(p) - 1
+    row = np.repeat(np.arange(n), np.diff(p))
+    keep = i <= row if uplo == "L" else i >= row
+    q = np.zeros(n + 1, np.int32)
+    q[1:] = np.cumsum(np.bincount(row[keep], minlength=n))
+    i, v = i[keep].copy(), v[keep] * np.linspace(0.2, 0.3, keep.sum())
+    T = H.make_triangular_matrix(engine, uplo, "N", engine.load(q), engine.load(i), engine.load(v))
+    T32 = H.make_triangular_matrix(engine, uplo, "N", T.pntr, T.indx, T.vals.float())
+    Tz = H.make_triangular_matrix(engine, uplo, "N", T.pntr, T.indx, engine.load(v * (1 + 0.25j)))
+    saved = engine.get_option("tri_grid"), engine.get_option("tri_col")
+    try:
+        if name == "pool":
+            engine.set_option("tri_col", 0)
+        for ta in "NT":
+            for tb, nrhs, pad in (("N", 1, 0), ("N", 3, 5), ("T", 4, 2), ("N", 9, 0)):
+                rng = np.random.default_rng(nrhs)
+                shape = (nrhs, n + pad) if tb == "N" else (n, nrhs + pad)
+                B = rng.uniform(-1, 1, shape)
+                for M, w in ((T, np.float64), (T32, np.float32), (Tz, np.complex128)):
+                    g = engine.load(B.astype(w))
+                    M.trsm(ta, tb, nrhs, 1.5, g, shape[1])
+                    got = host(g)
+                    assert np.array_equal(raw(got[:, shape[1] - pad:]), raw(B.astype(w)[:, shape[1] - pad:]))
+                    for c in range(nrhs):
+                        b = np.ascontiguousarray((B[c, :n] if tb == "N" else B[:, c]).astype(w))
+                        ref = {np.float64: lambda: oracle.trsv(uplo, ta, "N", 1.5, q, i, v, b),
+                               np.float32: lambda: oracle.trsv_f32(uplo, ta, "N", 1.5, q, i, v.astype(w), b),
+                               np.complex128: lambda: oracle.ztrsv(uplo, ta, "N", 1.5, q, i, v * (1 + 0.25j), b)}[w]()
+                        col = got[c, :n] if tb == "N" else got[:, c]
+                        assert np.array_equal(raw(col), raw(ref)), (name, ta, tb, nrhs, w, c)
+    finally:
+        engine.set_option("tri_grid", saved[0])
+        engine.set_option("tri_col", saved[1])
+
+
+@pytest.mark.parametrize("name", ["grid3", "column"])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 8, 9])
+def test_multirhs_pcg_grid_and_columns(engine, name, nrhs):
+    p, i, v = TRI["grid3"]()
+    n = len(p) - 1
+    gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+    saved = engine.get_option("tri_grid")
+    try:
+        engine.set_option("tri_grid", 1 if name == "grid3" else 0)
+        M = H.make_ilu(engine, gp, gi, gv)
+        B = np.stack([st.uniform(40 + k, n) for k in range(nrhs)])
+        tol = 1e-9 * max(oracle.cnrm2(b) for b in B)
+        X = torch.zeros(nrhs, n, dtype=torch.float64, device="cuda")
+        it = H.solve_batch_cg_ilu(engine, tol, gp, gi, gv, M, engine.load(B), X)
+        dg, _ = oracle.diag(p, i)
+        f = oracle.ilu0(p, i, v, dg)
+        for k in range(nrhs):  # each column is the single solve stopped after the same number of passes
+            _, x, _ = oracle.cg(p, i, v, B[k], tol=0.0, max_iter=it, prec=oracle.PREC_ILU, mpntr=p, mindx=i, mdiag=dg,
+                                mdata=f)
+            assert np.array_equal(bits(host(X[k])), bits(x)), k
+    finally:
+        engine.set_option("tri_grid", saved)
