@@ -13,6 +13,7 @@
 #include <cmath>
 
 #include "blas1.hpp"
+#include "cgsmall.hpp"
 #include "solvers.hpp"
 
 namespace hala_amd {
@@ -492,6 +493,12 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
     int batch = 4;
     int it = 1, done = 0, status = 0;
     double rn = 0.0;
+    if (!w && c->opt.cg_small && (P.prec == PREC_ID || P.prec == PREC_JAC) && !P.transposed && cg_small_fits(P.A)) {
+        cg_small_passes(c, P.A, P.vals, P.prec == PREC_JAC ? P.pdiag : nullptr, x, r, p, st, [&] {
+            cg_read(c, &it, &done, &status, &rn);
+            return done;
+        });
+    }
     while (!done) {
         for (int k = 0; k < batch; k++) one_pass();
         cg_read(c, &it, &done, &status, &rn);
