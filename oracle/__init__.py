@@ -363,9 +363,9 @@ def cg_batch(pntr, indx, vals, B, tol=0.0, max_iter=2**31 - 1, prec=PREC_IDENTIT
     return it, X, hist[: max(it - 1, 0)].copy()
 
 
-def cg_team(pntr, indx, vals, dvals, b, tol, team, max_iter=2**31 - 1, max_hist=100000):
+def cg_team(pntr, indx, vals, dvals, b, tol, team, max_iter=2**31 - 1, max_hist=100000, x0=None):
     n = len(pntr) - 1
-    x = np.zeros(n)
+    x = np.zeros(n) if x0 is None else c64(x0).copy()
     hist = np.zeros(max_hist)
     it = lib().hala_or_cg_team(n, P(ci32(pntr)), P(ci32(indx)), P(c64(vals)), P(c64(dvals)), P(c64(b)), P(x), tol,
                                max_iter, team, P(hist), max_hist)

@@ -1,0 +1,67 @@
+"""Batched PCG with the systems held in registers: solutions and iteration
+counts bit for bit the oracle's for every team size, at the edges of the rows
+per thread (one row, a full and a just started last round, the two register
+classes and the step to the general loop), rows of up to 5, 7 and 8 entries,
+ragged rows, a start that is not zero and an iteration cap."""
+import numpy as np
+import pytest
+import torch
+
+import hala_amd as H
+import oracle
+from tests.conftest import bits
+
+pytestmark = pytest.mark.gpu
+
+
+def banded(n, longest, rng):
+    """Symmetric, diagonally dominant, rows of 1 .. longest entries at a few offsets."""
+    offs = [1, max(2, int(n ** 0.5)), max(3, n // 2)][: (longest - 1) // 2]
+    row, col = [np.arange(n)], [np.arange(n)]
+    for o in offs:
+        a = np.nonzero(rng.random(max(n - o, 0)) < 0.9)[0]
+        row += [a, a + o]
+        col += [a + o, a]
+    row, col = np.concatenate(row), np.concatenate(col)
+    key = np.unique(row * n + col)
+    row, col = key // n, key % n
+    v = np.where(row == col, longest + 0.25 * (row % 5), -0.5 - 0.125 * ((row + col) % 4))
+    p = np.zeros(n + 1, np.int64)
+    p[1:] = np.cumsum(np.bincount(row, minlength=n))
+    return p, col, v
+
+
+def sizes_of(team, longest):
+    rounds = {64: (4, 10), 128: (4, 10), 256: (4, 10), 512: (4, 10), 1024: (3, 3)}[team] if longest <= 5 else (3, 8)
+    s = [1, 2, 63, 65, team - 1, team, team + 1, rounds[0] * team - 5, rounds[0] * team, rounds[0] * team + 1,
+         rounds[1] * team]
+    return s
+
+
+@pytest.mark.parametrize("longest,past", [(5, False), (5, True), (7, False), (9, False)])
+@pytest.mark.parametrize("team", [64, 128, 256, 512, 1024])
+def test_batch_resident_bitexact(engine, team, longest, past):
+    rng = np.random.default_rng(team + longest)
+    sizes = [min(n, 6000) for n in sizes_of(team, longest)] + ([min(sizes_of(team, longest)[-1] + 1, 6000)] if past else [])
+    sizes = [int(n) for n in rng.permutation(sizes)]
+    systems = [banded(n, longest, rng) for n in sizes]
+    ro = np.concatenate([[0], np.cumsum(sizes)])
+    nz = np.concatenate([[0], np.cumsum([len(s[1]) for s in systems])])
+    p = np.concatenate([s[0][:-1] + z for s, z in zip(systems, nz)] + [nz[-1:]])
+    i, v = np.concatenate([s[1] for s in systems]), np.concatenate([s[2] for s in systems])
+    d = rng.uniform(2.0, 9.0, ro[-1])
+    b, x0 = rng.uniform(-1, 1, ro[-1]), rng.uniform(-1, 1, ro[-1])
+    i32 = lambda a: engine.load(np.ascontiguousarray(a, np.int32))
+    bs = H.batch_solver(engine, i32(ro), i32(p), i32(i))
+    bs.set_shape(team, 1)
+    gv, gd, gb = engine.load(v), engine.load(d), engine.load(b)
+    for rtol, cap in ((1e-9, 100000), (1e-30, 6)):
+        gx = engine.load(x0)
+        iters = torch.zeros(len(sizes), dtype=torch.int32, device="cuda")
+        bs.solve(gv, gd, gb, gx, rtol=rtol, max_iter=cap, iters=iters)
+        for s, (sp, si, sv) in enumerate(systems):
+            r = slice(ro[s], ro[s + 1])
+            tol = rtol * np.sqrt(oracle.team_dot(b[r], b[r], team))
+            it, x, _ = oracle.cg_team(sp, si, sv, d[r], b[r], tol, team, x0=x0[r], max_iter=cap)
+            assert int(iters[s]) == it, (s, sizes[s])
+            assert np.array_equal(bits(gx[r].cpu().numpy()), bits(x)), (s, sizes[s])
