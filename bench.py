@@ -9,10 +9,9 @@ numeric factorisation, then device-resident PCG until ||r|| < 1e-10 ||b||.
 value = mean seconds per step (lower is better).
 
 roofline:      what dominates a step's time -- the triangular sweep of the
-               ILU(0) apply (two per PCG pass: the input gathered into L's
-               slot order, the column-blocked L sweep, L's output handed to
-               U's slot order, the U sweep, U's output scattered to natural
-               order), one triangle = half an apply, timed live with HIP
+               ILU(0) apply (two per PCG pass: the input gathered into the
+               tiles' order, the L sweep, the U sweep, its output scattered
+               to natural order), one triangle = half an apply, timed live with HIP
                events on the engine stream;
 roofline_spmv: the CSR SpMV (the bandwidth kernel of the path), with the
                rate of a plain 256 MiB device copy measured beside it
@@ -519,15 +518,13 @@ def main():
         "solve_ms": round(1e3 * float(np.mean(solves)), 3),
         "iters_per_s": round((it - 1) / float(np.mean(solves)), 2),
         "final_relres": relres,
-        "roofline": {"kernel": "ILU(0) triangular sweep, one triangle = half an apply: col_gather_in + "
-                               "tri_col_kernel<f64> (L, also storing U's slot-order input) + "
-                               "tri_col_kernel<f64> (U) + col_scatter_out",
+        "roofline": {"kernel": "ILU(0) triangular sweep, one triangle = half an apply: grid_gather + "
+                               "grid_sweep_kernel<f64> (L) + grid_sweep_kernel<f64> (U) + grid_scatter",
                      "bound": "hbm", "achieved": round(ach_sweep, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(ach_sweep / HBM_PEAK_GBS, 4), "traffic": traffic.get("tri_sweep_bytes"),
                      "bytes_per_launch": by_sweep, "avg_launch_ms": round(ms_sweep, 5),
                      "note": f"latency-bound: {ilu.info()['nlev_lower']} dependency levels per triangle, "
-                             f"{ilu.sweep_info(False)['ncol']} columns "
-                             f"({ilu.sweep_info(False)['split']} per slab of planes)"},
+                             "swept as register wavefronts over tiles of 64 grid lines"},
         "roofline_spmv": {"kernel": "spmv_rows_kernel<f64> (CSR, LDS-staged 256-row blocks"
                                     + (", columns streamed as int16 offsets from the block's first row)" if ib == 2
                                        else ")"),
