@@ -165,12 +165,14 @@ void jac_pattern(hala_ilu M) {
     // banded triangles: the sweeps stream int16 block offsets instead (6 instead of 8 bytes per FP32 entry)
     if (!build_block_offsets(c, n, nl, M->jl_ptr.as<int>(), M->jl_idx.as<int>(), M->jl_off)) M->jl_off.release();
     if (!build_block_offsets(c, n, nu, M->ju_ptr.as<int>(), M->ju_idx.as<int>(), M->ju_off)) M->ju_off.release();
-    // columns of 256 rows where padding every row to the longest adds at most a quarter: what the
-    // sweep gains there (21 -> 16 us), the padding's bytes would take back
+    // columns of 256 rows where padding every row to the longest adds at most a quarter (what the
+    // sweep gains, more padding would take back) and rows have at least five entries.  Applies with 3
+    // sweeps, packed -> columns: 27-point 96^3 132 -> 107 us FP32, 172 -> 160 FP64; 40^3 41 -> 34, 46 -> 36;
+    // rows of two (5-point 500^2) 38 -> 37, 40 -> 44; of three (7-point 96^3) 71 -> 59, 84 -> 84
     auto columns = [&](const dbuf &len, int nnz, const dbuf &ptr, dbuf &off) {
         if (!off.p || nnz == 0) return 0;
         const int w = reduce_max_i32(c, len.as<int>(), n);
-        if ((int64_t)g * 256 * w * 4 > (int64_t)nnz * 5) return 0;
+        if (w < 5 || (int64_t)g * 256 * w * 4 > (int64_t)nnz * 5) return 0;
         dbuf out;
         out.reserve((size_t)g * 256 * w * sizeof(short));
         jac_columns<<<g, 256, 0, c->stream>>>(n, w, ptr.as<int>(), off.as<short>(), out.as<short>());

@@ -26,7 +26,7 @@ def band(n, half, keep, seed):
 
 
 @pytest.mark.parametrize("prec", ["f32", "f64"])
-@pytest.mark.parametrize("n,half,keep", [(1, 1, 1), (255, 1, 1), (256, 6, 1), (257, 7, 1), (1000, 8, 1), (770, 13, 1),
+@pytest.mark.parametrize("n,half,keep", [(1, 1, 1), (255, 4, 1), (256, 5, 1), (256, 6, 1), (257, 7, 1), (1000, 8, 1), (770, 13, 1),
                                          (513, 14, 1), (600, 15, 1), (700, 5, 9)])
 def test_jacobi_columns_bitexact(engine, n, half, keep, prec):
     p, i, v = band(n, half, keep, n + half)
