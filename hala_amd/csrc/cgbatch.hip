@@ -97,14 +97,14 @@ __global__ __launch_bounds__(256) void cgb_start(int n, const double *__restrict
 // once; fused <p_k, Ap_k>, and block k forms a_k = zr_k / <p_k, Ap_k> (a
 // collector per column: one block collecting eight in turn costs eight
 // reduction latencies).
-template <int G, class TI>
+template <int G, class TI, class TO>
 __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int *__restrict__ pntr,
                                                 const TI *__restrict__ indx, const double *__restrict__ vals,
                                                 const double *__restrict__ Pv, double *__restrict__ AP, double *part,
                                                 const double *zr, double *al, cgb_state *st, int *err) {
     if (st->done) return;
     __shared__ double sv[spmm_tile<double>::value];
-    __shared__ unsigned so[spmm_tile<double>::value];
+    __shared__ TO so[spmm_tile<double>::value];
     const int64_t nb = ((int64_t)n + CB - 1) / CB;
     const int row = blockIdx.x * SPMV_ROWS + threadIdx.x;
     const char *xb[G];
@@ -113,8 +113,8 @@ __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int
     double acc[G];
 #pragma unroll
     for (int k = 0; k < G; k++) acc[k] = 0.0;
-    csr_block_rowsums<double, G, TI, false, unsigned>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false,
-                                                      false, sv, so, acc);
+    csr_block_rowsums<double, G, TI, false, TO>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false, false,
+                                                sv, so, acc);
     static_assert(G * CB <= spmm_tile<double>::value, "tree scratch");
 #pragma unroll
     for (int k = 0; k < G; k++) {
@@ -279,20 +279,21 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
     auto one_pass = [&]() {
         for (int c0 = 0; c0 < nrhs; c0 += CGB_GROUP) {
             const int nc = std::min(CGB_GROUP, nrhs - c0);
-            const short *bo = A->boff.as<short>();
-#define HALA_CGB(GG)                                                                                          \
-    if (bo)                                                                                                   \
-        cgb_spmm<GG, short><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, bo, vals, Pv, AP, part, zr, al, st,  \
-                                                       wait_error_flag(c));                                   \
+#define HALA_CGB(GG, TO)                                                                                       \
+    if (A->boff.p)                                                                                            \
+        cgb_spmm<GG, short, TO><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->boff.as<short>(), vals, Pv, AP, \
+                                                           part, zr, al, st, wait_error_flag(c));              \
     else                                                                                                      \
-        cgb_spmm<GG, int><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->indx, vals, Pv, AP, part, zr, al,   \
-                                                     st, wait_error_flag(c))
-            if (nc > 4) {
-                HALA_CGB(8);
+        cgb_spmm<GG, int, TO><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->indx, vals, Pv, AP, part, zr, al, \
+                                                         st, wait_error_flag(c))
+            if (gather_wide(n, sizeof(double))) {
+                HALA_CGB(8, uint64_t);
+            } else if (nc > 4) {
+                HALA_CGB(8, unsigned);
             } else if (nc > 2) {
-                HALA_CGB(4);
+                HALA_CGB(4, unsigned);
             } else {
-                HALA_CGB(2);
+                HALA_CGB(2, unsigned);
             }
 #undef HALA_CGB
         }

@@ -1,0 +1,17 @@
+// gather.hpp -- integer arithmetic of the products' gathers
+// (plain C++: tested on the host at sizes no test matrix has).
+#pragma once
+#include <cstdint>
+
+namespace hala_amd {
+
+// Byte offset of element c of a vector whose elements lie step bytes apart.
+template <class TO>
+constexpr TO gather_offset(int c, TO step) {
+    return (TO)c * step;
+}
+
+// Whether the offsets of an n-element vector need 64 bits.
+constexpr bool gather_wide(int64_t n, int64_t step) { return n * step > (int64_t)UINT32_MAX; }
+
+}  // namespace hala_amd

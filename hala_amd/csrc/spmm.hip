@@ -137,7 +137,7 @@ void spmm_columns(hala_csr A, char trans, S alpha, const S *vals, const S *x, in
     const int g = (nrows + SPMV_ROWS - 1) / SPMV_ROWS;
     const int conjv = is_c(trans) ? 1 : 0;
     const int64_t step = sc * (int64_t)sizeof(S);
-    const bool wide = ncin * step > (int64_t)UINT32_MAX;  // 32-bit offsets into a vector otherwise
+    const bool wide = gather_wide(ncin, step);
     const int gmax = wide ? 1 : 8;
     for (int c0 = 0; c0 < ncols; c0 += gmax) {
         const int nc = std::min(gmax, ncols - c0);

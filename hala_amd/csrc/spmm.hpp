@@ -8,6 +8,7 @@
 // neighbouring elements of the vectors wherever neighbouring rows have
 // neighbouring columns.
 #pragma once
+#include "gather.hpp"
 #include "scalar.hpp"
 #include "spmv.hpp"
 
@@ -19,7 +20,7 @@ struct spmm_tile {
 };
 
 // acc[k] = op over the row's entries, k < G: acc + v * x_k (N), acc + (alpha * x_k) * v (TRANS).
-// x_k(c) is at xb[k] + c * step bytes (TO: 32- or 64-bit offsets).  TI = short: columns as offsets from
+// x_k(c) is at xb[k] + c * step bytes (TO: uint64_t where gather_wide() of the vector, else unsigned).  TI = short: columns as offsets from
 // the block's first row.
 // Must be called by all 256 threads of the block; sv, so: spmm_tile entries of LDS each.
 template <class S, int G, class TI, bool TRANS, class TO>
@@ -45,7 +46,7 @@ __device__ __forceinline__ void csr_block_rowsums(int nrows, const int *__restri
             S v = vals[TRANS ? tmap[j] : j];
             if (is_complex<S>::value && conjv) v = cconj(v);
             sv[e] = v;
-            so[e] = (TO)(cb + (int)indx[j]) * step;
+            so[e] = gather_offset<TO>(cb + (int)indx[j], step);
         }
         __syncthreads();
         const int a = max(rs, base) - base, b = min(re, base + cnt) - base;
