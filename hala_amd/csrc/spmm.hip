@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void spmv_t_rows_kernel(int nrows, const int *
         re = tpntr[row + 1];
         if (beta != T(0)) acc = beta * y[row];
     }
-    for (int base = bstart; base < bend; base += TILE) {
+    for (int base = bstart; base < bend; base = tile_next(base, bend, TILE)) {
         const int cnt = min(TILE, bend - base);
         int e = threadIdx.x;
         for (; e + 3 * SPMV_ROWS < cnt; e += 4 * SPMV_ROWS) {

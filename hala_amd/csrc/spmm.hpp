@@ -8,7 +8,6 @@
 // neighbouring elements of the vectors wherever neighbouring rows have
 // neighbouring columns.
 #pragma once
-#include "gather.hpp"
 #include "scalar.hpp"
 #include "spmv.hpp"
 
@@ -38,7 +37,7 @@ __device__ __forceinline__ void csr_block_rowsums(int nrows, const int *__restri
         rs = pntr[row];
         re = pntr[row + 1];
     }
-    for (int base = bstart; base < bend; base += TILE) {
+    for (int base = bstart; base < bend; base = tile_next(base, bend, TILE)) {
         const int cnt = min(TILE, bend - base);
 #pragma unroll 4
         for (int e = threadIdx.x; e < cnt; e += SPMV_ROWS) {

@@ -174,11 +174,13 @@ __global__ __launch_bounds__(256) void spmv_wave_kernel(int nrows, const int *__
         const int s = pntr[row], e = pntr[row + 1];
         TA acc = TA(0);
         TA p = TA(0);
-        if (s + lane < e) p = (TA)vals[s + lane] * (TA)x[indx[s + lane]];
-        for (int base = s; base < e; base += 64) {
-            const int jn = base + 64 + lane;
+        if (lane < e - s) p = (TA)vals[s + lane] * (TA)x[indx[s + lane]];
+        for (int base = s; base < e; base = tile_next(base, e, 64)) {
             TA pn = TA(0);
-            if (jn < e) pn = (TA)vals[jn] * (TA)x[indx[jn]];
+            if (lane < e - base - 64) {
+                const int jn = base + 64 + lane;
+                pn = (TA)vals[jn] * (TA)x[indx[jn]];
+            }
             const int cnt = min(64, e - base);
             for (int k = 0; k < cnt; k++) acc = acc + lane_value(p, k);
             p = pn;

@@ -1,5 +1,6 @@
 // spmv.hpp -- CSR matrix handle and the sparse matrix-vector product cores.
 #pragma once
+#include "gather.hpp"
 #include "util.hpp"
 
 struct hala_csr_s {
@@ -68,7 +69,7 @@ __device__ __forceinline__ TA csr_block_rowsum(int nrows, const int *__restrict_
         re = pntr[row + 1];
     }
     TA acc = init;
-    for (int base = bstart; base < bend; base += TILE) {
+    for (int base = bstart; base < bend; base = tile_next(base, bend, TILE)) {
         const int cnt = min(TILE, bend - base);
         int e = threadIdx.x;
         for (; e + 3 * SPMV_ROWS < cnt; e += 4 * SPMV_ROWS) {

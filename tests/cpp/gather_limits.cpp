@@ -1,4 +1,4 @@
-// Gathers at the largest sizes the entry points accept
+// Gathers and tile loops at the largest sizes the entry points accept
 // (hala_amd/csrc/gather.hpp); prints one line per check, exits 1 on a failure.
 #include <climits>
 #include <cstdio>
@@ -23,6 +23,20 @@ static bool reaches(int64_t n, int64_t step) {
     return got == want;
 }
 
+// a tile loop visits every entry of [begin, end) once and ends
+static bool covers(int begin, int end, int tile) {
+    int64_t seen = 0;
+    int at = begin;
+    for (int base = begin; base < end; base = tile_next(base, end, tile)) {
+        if (base != at) return false;
+        const int cnt = end - base < tile ? end - base : tile;
+        seen += cnt;
+        at = base + cnt;
+        if (seen > (int64_t)end - begin) return false;
+    }
+    return seen == (int64_t)end - begin && at == end;
+}
+
 int main() {
     const int64_t lim = int64_t(1) << 29;  // 2^29 doubles are 2^32 bytes
     for (int64_t step : {4, 8, 16})
@@ -30,5 +44,9 @@ int main() {
     check(!gather_wide(lim - 1, 8) && gather_wide(lim + 1, 8), "doubles need 64-bit offsets past 2^29");
     check(reaches(INT_MAX, 8) && reaches(INT_MAX, 16) && reaches(1, 8), "extremes");
     check(reaches(1000, int64_t(8) * 3000000), "a row of a wide dense matrix");
+    for (int tile : {64, 1024, 2048, 4096})
+        for (int end : {0, 1, tile - 1, tile, tile + 1, 3 * tile + 5, INT_MAX - 1, INT_MAX})
+            for (int len : {0, 1, tile - 1, tile, tile + 1, 5 * tile - 3})
+                if (len <= end) check(covers(end - len, end, tile), "tile loop");
     return failures ? 1 : 0;
 }

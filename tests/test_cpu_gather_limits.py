@@ -1,8 +1,9 @@
 """Index arithmetic of the sparse products at the limits of int32 sizes: the
 offset type chosen for a vector's gathers reaches its last element (a
-multi-right-hand-side CG of more than 2^29 rows gathers past 4 GiB).  Host build
-of hala_amd/csrc/gather.hpp under UndefinedBehaviorSanitizer; every product that
-gathers by byte offsets takes its choice from there."""
+multi-right-hand-side CG of more than 2^29 rows gathers past 4 GiB), and
+loops over a block's entries end and stay in bounds for entry counts up to
+INT_MAX - 1.  Host build of hala_amd/csrc/gather.hpp under
+UndefinedBehaviorSanitizer; the products take both from there."""
 import os
 import re
 import shutil
@@ -38,3 +39,10 @@ def test_offset_products_choose_the_width():
         assert "gather_wide(" in text, f
         for call in re.findall(r"csr_block_rowsums<([^;]*?)>\(", text):
             assert call.rstrip().endswith("TO"), (f, call)
+
+
+def test_tile_loops_step_in_bounds():
+    # a loop over int entry positions steps by tile_next: base += TILE overflows within a tile of INT_MAX
+    for f in ("spmv.hpp", "spmv.hip", "spmm.hpp", "spmm.hip"):
+        for loop in re.findall(r"for \(int base = [^;]*;[^;]*;([^)]*\)?)\)", open(os.path.join(CSRC, f)).read()):
+            assert "tile_next(base" in loop, (f, loop)
