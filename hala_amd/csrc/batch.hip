@@ -27,6 +27,7 @@ struct hala_batch_s {
     const int *row_off = nullptr, *pntr = nullptr, *indx = nullptr;  // device, not owned
     hala_amd::dbuf order, work, iters, ctl;
     int team = 256, wg_per_cu = 2;
+    int path = -1;  // what launch_batch last chose (hala_path)
     // graph cache
     hipStream_t cap = nullptr;
     hipGraph_t graph = nullptr;
@@ -402,6 +403,7 @@ static bool resident(hala_batch B, hipStream_t s, int wg, const double *vals, co
     const int big = (int)(std::partition_point(B->sizes.begin(), B->sizes.end(), [](int n) { return n > R1 * T; }) -
                           B->sizes.begin());
     unsigned *ctl = B->ctl.as<unsigned>();
+    B->path = (big ? 4 : 0) + (big < B->nsys ? 2 : 0);
     auto grid = [&](int k) { return std::max(1, std::min(k, c->num_cus * wg)); };
     if (big)
         batch_resident_kernel<T, R2, LEN, 2><<<grid(big), T, resident_lds<T, LEN>(B->sizes[0]), s>>>(
@@ -443,6 +445,7 @@ static void launch_batch(hala_batch B, hipStream_t s, int team, int wg, const do
     size_t lds = batch_lds(team, B->max_n);
     batch_reset_kernel<<<1, 1, 0, s>>>(ctl);
     if (launch_resident(B, s, team, wg, vals, dvals, b, x, rtol, max_iter)) return;
+    B->path = 1;
 #define HALA_BATCH(TT)                                                                                          \
     batch_pcg_kernel<TT><<<grid, TT, lds, s>>>(B->nsys, B->n_total, B->max_n, B->order.as<int>(), B->row_off,    \
                                                B->pntr, B->indx, vals, dvals, b, x, B->work.as<double>(), rtol,  \
@@ -498,6 +501,7 @@ static void run_batch(hala_batch B, const double *vals, const double *dvals, con
         B->key_team = B->team;
         B->key_wg = B->wg_per_cu;
     }
+    c->path[PATH_BATCH] = B->path;
     HALA_HIP(hipGraphLaunch(B->exec, c->stream));
 }
 

@@ -409,6 +409,7 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
     const int *gate = &st->done;
     ilu_ends ends{};
     const bool fused = P.prec == PREC_ILU && c->opt.cg_fuse && ilu_fused64(P.M, P.transposed, ends);
+    if (P.prec == PREC_ILU) c->path[PATH_PCG] = !fused ? 0 : ends.axpy ? 1 : 2;
     auto precond = [&](const double *in, double *out, const int *g) {
         if (P.transposed) ilu_apply_t64(P.M, in, out, g);
         else ilu_apply64(P.M, in, out, g);
@@ -426,6 +427,7 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
 
     // small identity/Jacobi systems: the direction update rides in the next product (p and z's slot alternate)
     const bool pz = (P.prec == PREC_ID || P.prec == PREC_JAC) && !P.transposed && n <= PZ_MAX_ROWS;
+    if (P.prec != PREC_ILU) c->path[PATH_CG] = pz ? 1 : 0;
     int pass = 0;
     auto one_pass = [&]() {
         if (pz) {
@@ -494,6 +496,7 @@ static void run_cg(hala_ctx c, const cg_problem &P, const double *b, double *x, 
     int it = 1, done = 0, status = 0;
     double rn = 0.0;
     if (!w && c->opt.cg_small && (P.prec == PREC_ID || P.prec == PREC_JAC) && !P.transposed && cg_small_fits(P.A)) {
+        c->path[PATH_CG] = 2;
         cg_small_passes(c, P.A, P.vals, P.prec == PREC_JAC ? P.pdiag : nullptr, x, r, p, st, [&] {
             cg_read(c, &it, &done, &status, &rn);
             return done;

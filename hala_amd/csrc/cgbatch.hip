@@ -269,6 +269,7 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
     ilu_ends ends{};
     int64_t N_ = 0;
     const bool fused = !ident && c->opt.cg_fuse && ilu_fused64_cols(M, nrhs, ends, N_);
+    if (!ident) c->path[PATH_PCG] = fused ? 2 : 0;
     if (ident) {
         cgb_start<true><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, nullptr, Pv, part, zr, wait_error_flag(c));
     } else {

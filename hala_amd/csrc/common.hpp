@@ -218,8 +218,21 @@ struct hala_options {
                                // by the next call that synchronises the context (hala_ctx_sync included)
 };
 
+// Which of its kernels the last call of a family ran (hala_ctx_get_option("path_..."), meanings in
+// include/hala_amd.h): noted at the dispatch, so that a test can tell a path from its fallback.
+enum hala_path : int {
+    PATH_SWEEP,    // triangular sweep
+    PATH_PCG,      // ILU-preconditioned CG, one or several right-hand sides
+    PATH_CG,       // identity / Jacobi CG
+    PATH_BATCH,    // batched systems
+    PATH_JACOBI,   // Jacobi-applied ILU
+    PATH_PRODUCT,  // sparse times dense, transposed and complex products
+    PATH_COUNT
+};
+
 struct hala_ctx_s {
     hala_options opt;
+    int path[PATH_COUNT] = {-1, -1, -1, -1, -1, -1};
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;

@@ -225,6 +225,14 @@ static int *option_slot(hala_ctx c, const char *name) {
     return nullptr;
 }
 
+static const int *path_slot(hala_ctx c, const char *name) {
+    static const char *const names[PATH_COUNT] = {"path_sweep",  "path_pcg",    "path_cg",
+                                                  "path_batch", "path_jacobi", "path_product"};
+    for (int k = 0; k < PATH_COUNT; k++)
+        if (name && std::strcmp(name, names[k]) == 0) return &c->path[k];
+    return nullptr;
+}
+
 int hala_ctx_set_option(hala_ctx c, const char *name, int value) {
     return guard([&] {
         HALA_REQUIRE(c, HALA_ERR_ARG, "null context");
@@ -240,7 +248,8 @@ int hala_ctx_set_option(hala_ctx c, const char *name, int value) {
 int hala_ctx_get_option(hala_ctx c, const char *name, int *value) {
     return guard([&] {
         HALA_REQUIRE(c && value, HALA_ERR_ARG, "null argument");
-        int *slot = option_slot(c, name);
+        const int *slot = option_slot(c, name);
+        if (!slot) slot = path_slot(c, name);
         HALA_REQUIRE(slot, HALA_ERR_ARG, std::string("unknown option ") + (name ? name : "(null)"));
         *value = *slot;
     });

@@ -227,6 +227,7 @@ void jac_apply(hala_ilu M, const double *x, double *r, const int *gate, int k, c
             else sweep<V, double, V, V, true, false>(c, n, lp, li, lo, M->jl_w, lv, dv, x, yo, yn, nullptr, gate);
         }
     }
+    c->path[PATH_JACOBI] = (M->jl_w ? 2 : lo ? 1 : 0) + 4 * (M->ju_w ? 2 : uo ? 1 : 0);
     // U sweeps: z(m+1) = (y - (U - D) z(m)) / d; the last writes the FP64 result
     const V *y = ybuf[(k - 1) & 1];
     for (int m = 0; m < k; m++) {

@@ -133,6 +133,7 @@ void spmm_columns(hala_csr A, char trans, S alpha, const S *vals, const S *x, in
     const bool tr = !is_n(trans);
     const int nrows = tr ? A->ncols : A->nrows, ncin = tr ? A->nrows : A->ncols;
     if (tr) ensure_transpose(A);
+    c->path[PATH_PRODUCT] = 1;
     if (nrows == 0 || ncols == 0) return;
     const int g = (nrows + SPMV_ROWS - 1) / SPMV_ROWS;
     const int conjv = is_c(trans) ? 1 : 0;
@@ -188,6 +189,7 @@ void spmm(hala_csr A, char transa, char transb, int b_rows, int b_cols, S alpha,
     if constexpr (!is_complex<S>::value) {
         if ((bn && N == 1) || (is_n(transa) && A->kernel == 1)) {
             hala_ctx c = A->ctx;
+            c->path[PATH_PRODUCT] = 0;
             tmp_scope ts(c);
             dbuf &t = ts.get();
             if (!bn) t.reserve((size_t)std::max(K, 1) * sizeof(S));

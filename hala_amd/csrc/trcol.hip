@@ -1032,6 +1032,7 @@ void col_sweep(hala_ctx c, tri_plan &p, int mode, T alpha, const int *gate, tri_
                const col_axpy *ax = nullptr, int nrhs = 0) {
     constexpr bool is64 = sizeof(T) == 8;
     tri_colplan &q = p.col;
+    c->path[PATH_SWEEP] = 1;
     col_args<T, TOUT> a;
     a.nlev = p.nlev;
     a.K = q.K;

@@ -192,6 +192,7 @@ void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *o
         tri_col_exec<T, TOUT>(c, p, mode, alpha, in, out_nat, gate);
         return;
     }
+    c->path[PATH_SWEEP] = 0;
     tri_rearm_prec(c, p, is64);
     tri_args<T, TIN, TOUT> a;
     a.out = is64 ? reinterpret_cast<T *>(p.out64.p) : reinterpret_cast<T *>(p.out32.p);

@@ -635,6 +635,7 @@ void sweep(hala_ctx c, const tri_plan &p, int mode, V alpha, const V *in, V *out
     const tri_gridplan &q = p.grid;
     const grid_geom &g = q.g;
     const int dim = g.nz > 1 ? 3 : 2, TJ = dim == 3 ? 8 : 64, TK = dim == 3 ? 8 : 1;
+    c->path[PATH_SWEEP] = 2;
     gsweep_args<V> a;
     a.nx = g.nx;
     a.ntj = g.ntj;

@@ -867,6 +867,7 @@ void stencil_load(hala_ilu_s *M, bool f32) {
 
 template <class V, class TIN, class TOUT>
 void stencil_apply(hala_ilu_s *M, const TIN *x, TOUT *r, const int *gate) {
+    M->ctx->path[PATH_SWEEP] = 3;
     switch (M->sp->kind) {
     case SK_5: sweep_pair<SK_5, V, TIN, TOUT>(M, x, r, gate); break;
     case SK_9: sweep_pair<SK_9, V, TIN, TOUT>(M, x, r, gate); break;

@@ -72,7 +72,18 @@ int hala_ctx_device(hala_ctx ctx, int *device);
  * of the exact apply, inside GMRES and the standalone applies).  Errors:
  * "sync_checks" (1: standalone sweeps wait for the device and report a
  * dependency wait that gave up; 0: the report is deferred to the next
- * synchronising call).  Unknown names return HALA_ERR_ARG. */
+ * synchronising call).  Unknown names return HALA_ERR_ARG.
+ *
+ * hala_ctx_get_option also reads which kernels the context's last call of a
+ * family ran (-1: none yet): "path_sweep" (0 level pool, 1 columns, 2 grid
+ * wavefronts, 3 pencils), "path_pcg" (ILU-PCG; 0 separate applies, 1 fused
+ * column sweeps, 2 fused grid sweeps), "path_cg" (identity and Jacobi CG; 0
+ * launched passes, 1 with the direction update in the product, 2 one
+ * workgroup), "path_batch" (sum of 1: general loop, 2 and 4: resident systems
+ * of the small and the large size class), "path_jacobi" (Jacobi-applied ILU,
+ * L + 4 U; 0 packed rows, 1 with int16 offsets, 2 columns of 256 rows),
+ * "path_product" (sparse times dense, transposed, complex; 0 the single
+ * product per column, 1 several columns at once). */
 int hala_ctx_set_option(hala_ctx ctx, const char *name, int value);
 int hala_ctx_get_option(hala_ctx ctx, const char *name, int *value);
 

@@ -1,7 +1,7 @@
 """Batched PCG with the systems held in registers: solutions and iteration
 counts bit for bit the oracle's for every team size, at the edges of the rows
 per thread (one row, a full and a just started last round, the two register
-classes and the step to the general loop), rows of up to 5, 7 and 8 entries,
+classes and the step to the general loop), rows of up to 5, 7 and 9 entries,
 ragged rows, a start that is not zero and an iteration cap."""
 import numpy as np
 import pytest
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 def banded(n, longest, rng):
     """Symmetric, diagonally dominant, rows of 1 .. longest entries at a few offsets."""
-    offs = [1, max(2, int(n ** 0.5)), max(3, n // 2)][: (longest - 1) // 2]
+    offs = [1, max(2, int(n ** 0.5)), max(3, n // 2), max(4, n // 3)][: (longest - 1) // 2]
     row, col = [np.arange(n)], [np.arange(n)]
     for o in offs:
         a = np.nonzero(rng.random(max(n - o, 0)) < 0.9)[0]
@@ -55,10 +55,17 @@ def test_batch_resident_bitexact(engine, team, longest, past):
     bs = H.batch_solver(engine, i32(ro), i32(p), i32(i))
     bs.set_shape(team, 1)
     gv, gd, gb = engine.load(v), engine.load(d), engine.load(b)
+    # which kernels: resident, by rows per thread, where every system and row fits; else the general loop
+    small, large = ((4, 10) if team < 1024 else (3, 3)) if longest <= 5 else ((3, 8) if team < 1024 else (0, 0))
+    if longest > 7 or max(sizes) > large * team:
+        want = 1
+    else:
+        want = (4 if max(sizes) > small * team else 0) + (2 if min(sizes) <= small * team else 0)
     for rtol, cap in ((1e-9, 100000), (1e-30, 6)):
         gx = engine.load(x0)
         iters = torch.zeros(len(sizes), dtype=torch.int32, device="cuda")
         bs.solve(gv, gd, gb, gx, rtol=rtol, max_iter=cap, iters=iters)
+        assert engine.get_option("path_batch") == want
         for s, (sp, si, sv) in enumerate(systems):
             r = slice(ro[s], ro[s + 1])
             tol = rtol * np.sqrt(oracle.team_dot(b[r], b[r], team))

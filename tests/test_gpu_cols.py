@@ -24,12 +24,12 @@ def raw(a):
     return bits(a.view(np.float64 if a.dtype in (np.complex128, np.float64) else np.float32))
 
 
-def ragged(nr, nc, seed, longest):
-    """Rows of 0 .. longest entries, one row with all nc columns."""
+def ragged(nr, nc, seed, longest, full=True):
+    """Rows of 0 .. longest entries, with `full` one row with all nc columns."""
     rng = np.random.default_rng(seed)
     p, i = [0], []
     for r in range(nr):
-        k = nc if r == nr // 3 else int(rng.integers(0, longest + 1))
+        k = nc if full and r == nr // 3 else int(rng.integers(0, longest + 1))
         i.extend(np.sort(rng.choice(nc, size=min(k, nc), replace=False)))
         p.append(len(i))
     return np.array(p, np.int32), np.array(i, np.int32)
@@ -38,7 +38,8 @@ def ragged(nr, nc, seed, longest):
 MATS = {
     "band": lambda: (lambda p, i, v: (p, i, len(p) - 1))(*st.laplace3d(9, 8, 8)),  # int16 offsets, tile remainders
     "ragged": lambda: (*ragged(517, 3000, 3, 9), 3000),  # a row and a tile longer than the staging
-    "wide": lambda: (*ragged(260, 70000, 4, 5), 70000),  # int32 columns
+    "wide": lambda: (*ragged(260, 70000, 4, 5), 70000),  # int32 columns, a row for the wavefront kernel
+    "wide short": lambda: (*ragged(260, 70000, 6, 5, full=False), 70000),
     "one": lambda: (np.array([0, 1], np.int32), np.array([0], np.int32), 1),
     "empty": lambda: (np.zeros(301, np.int32), np.zeros(0, np.int32), 40),
 }
@@ -70,7 +71,9 @@ def test_spmm_columns(engine, mat, ct):
             A.gemm(ta, tb, k if tb == "N" else cols, cols if tb == "N" else k, 1.5, engine.load(B), ldb, beta, gC, ldc)
             got = host(gC)
             assert np.array_equal(raw(got[:, m:]), raw(C0[:, m:]))  # nothing written past a column
-            for c in sorted({0, cols - 1}):
+            single = (tb == "N" and cols == 1) or (ta == "N" and A.info()["kernel"] == 1)
+            assert engine.get_option("path_product") == (0 if single and not cplx else 1)
+            for c in range(cols):
                 x = np.ascontiguousarray(B[c, :k] if tb == "N" else (B[:, c].conj() if tb == "C" else B[:, c]))
                 y = np.ascontiguousarray(C0[c, :m])
                 if ct == np.float64:

@@ -31,6 +31,9 @@ GRIDS = {
 }
 
 
+GRID_SWEEP = 2  # path_sweep of the kernels tested here
+
+
 def host(t):
     return t.detach().cpu().numpy()
 
@@ -51,8 +54,10 @@ def test_grid_apply_bitexact(engine, name):
         x = st.uniform(seed, n)
         gx = engine.load(x)
         M.apply(gx, gr)
+        assert engine.get_option("path_sweep") == GRID_SWEEP
         assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(p, i, dg, f, x)))
         M.apply_t(gx, gr)
+        assert engine.get_option("path_sweep") == GRID_SWEEP
         assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply_t(p, i, dg, f, x)))
         ref32 = oracle.ilu_apply_f32(p, i, dg, f.astype(np.float32), x.astype(np.float32))
         M.apply_f32x64(gx, gr)
@@ -85,6 +90,7 @@ def test_grid_trsv_bitexact(engine, name, uplo, diag):
         for _ in range(2):
             x, x32 = engine.vector(n), engine.vector(n, dtype=torch.float32)
             T.trsv(trans, 1.5, engine.load(b), x)
+            assert engine.get_option("path_sweep") == GRID_SWEEP
             assert np.array_equal(bits(host(x)), bits(oracle.trsv(uplo, trans, diag, 1.5, q, i, v, b)))
             T32.trsv(trans, 1.5, engine.load(b.astype(np.float32)), x32)
             ref = oracle.trsv_f32(uplo, trans, diag, 1.5, q, i, v.astype(np.float32), b.astype(np.float32))
@@ -107,6 +113,7 @@ def test_grid_incomplete_pattern(engine, name):
     x = st.uniform(3, n)
     gr = engine.vector(n)
     M.apply(engine.load(x), gr)
+    assert engine.get_option("path_sweep") != GRID_SWEEP
     assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(q, i[keep].copy(), dg, f, x)))
 
 

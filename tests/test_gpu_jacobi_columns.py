@@ -32,6 +32,11 @@ def test_jacobi_columns_bitexact(engine, n, half, keep, prec):
     p, i, v = band(n, half, keep, n + half)
     opt = "ilu32_jacobi" if prec == "f32" else "ilu64_jacobi"
     saved = engine.get_option(opt)
+    # columns for triangles of rows of five and more entries, padded by at most a quarter
+    row = np.repeat(np.arange(n), np.diff(p))
+    low = np.bincount(row[i < row], minlength=n)
+    width, blocks = int(low.max()), (n + 255) // 256
+    columns = width >= 5 and blocks * 256 * width * 4 <= int(low.sum()) * 5
     try:
         dg, _ = oracle.diag(p, i)
         f = oracle.ilu0(p, i, v, dg)
@@ -49,5 +54,6 @@ def test_jacobi_columns_bitexact(engine, n, half, keep, prec):
                 M.apply(engine.load(x), gr)
                 ref = oracle.ilu_apply_jacobi(p, i, dg, f, x, k)
             assert np.array_equal(bits(gr.cpu().numpy()), bits(ref))
+            assert (engine.get_option("path_jacobi") % 4 == 2) == columns
     finally:
         engine.set_option(opt, saved)
