@@ -1,0 +1,139 @@
+"""Solver paths that the grid sweeps and the one-workgroup CG took over from on
+the other tests' complete grids, and that every other matrix still runs: the
+column sweeps fused into PCG (hand-off, x updated on the helper workgroups, the
+stopping pass's own update), the column and level-pool sweeps, and CG whose
+direction update rides in the product.  Bit for bit the oracle's, with the path
+checked."""
+import numpy as np
+import pytest
+import torch
+
+import hala_amd as H
+import oracle
+from hala_amd import stencils as st
+from tests.conftest import bits
+
+pytestmark = pytest.mark.gpu
+
+
+def host(t):
+    return t.detach().cpu().numpy()
+
+
+class options:
+    def __init__(self, engine, **kw):
+        self.engine, self.kw = engine, kw
+
+    def __enter__(self):
+        self.saved = {k: self.engine.get_option(k) for k in self.kw}
+        for k, v in self.kw.items():
+            self.engine.set_option(k, v)
+
+    def __exit__(self, *a):
+        for k, v in self.saved.items():
+            self.engine.set_option(k, v)
+
+
+def holes(p, i, v, every):
+    """The matrix without the symmetric pairs of couplings (r, r + 1) of every `every`-th row r."""
+    n = len(p) - 1
+    row = np.repeat(np.arange(n), np.diff(p))
+    gone = ((i == row + 1) & (row % every == 0)) | ((row == i + 1) & (i % every == 0))
+    q = np.zeros(n + 1, np.int32)
+    q[1:] = np.cumsum(np.bincount(row[~gone], minlength=n))
+    return q, i[~gone].copy(), v[~gone].copy()
+
+
+PCG = {  # name: (matrix, options, path_pcg)
+    "grid": (lambda: st.laplace3d(32, 32, 32), {}, 2),
+    "columns": (lambda: st.laplace3d(32, 32, 32), {"tri_grid": 0}, 1),
+    "columns ragged": (lambda: st.laplace3d(30, 31, 29), {"tri_grid": 0}, 1),
+    "columns ragged, dispatch order": (lambda: st.laplace3d(30, 31, 29), {"tri_grid": 0, "cg_xcd": 0}, 1),
+    "columns separate": (lambda: st.laplace3d(32, 32, 32), {"tri_grid": 0, "cg_fuse": 0}, 0),
+    "columns, grid-stride product": (lambda: st.laplace3d(40, 40, 40), {"tri_grid": 0, "spmv_blocks_per_cu": 2}, 1),
+    "mesh with holes": (lambda: holes(*st.laplace3d(30, 31, 29), 97), {}, 1),
+    "mesh with holes, separate": (lambda: holes(*st.laplace3d(30, 31, 29), 97), {"cg_fuse": 0}, 0),
+    "level pool": (lambda: st.laplace3d(20, 21, 19), {"tri_col": 0}, 0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(PCG))
+def test_pcg_paths_bitexact(engine, name):
+    mat, opts, path = PCG[name]
+    p, i, v = mat()
+    n = len(p) - 1
+    b = st.uniform(202, n)
+    tol = 1e-10 * oracle.cnrm2(b)
+    dg, _ = oracle.diag(p, i)
+    it, x, hist = oracle.cg(p, i, v, b, tol=tol, prec=oracle.PREC_ILU, mpntr=p, mindx=i, mdiag=dg,
+                            mdata=oracle.ilu0(p, i, v, dg))
+    with options(engine, **opts):
+        gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+        M = H.make_ilu(engine, gp, gi, gv)
+        for _ in range(2):  # the polled outputs re-arm themselves
+            gx, gh = engine.vector(n), torch.zeros(2000, dtype=torch.float64, device="cuda")
+            git = H.solve_cg_ilu(engine, tol, gp, gi, gv, M, engine.load(b), gx, hist=gh)
+            assert engine.get_option("path_pcg") == path
+            assert git == it
+            assert np.array_equal(bits(host(gh)[: it - 1]), bits(hist))
+            assert np.array_equal(bits(host(gx)), bits(x))
+
+
+SWEEPS = {  # name: (matrix, options, path_sweep)
+    "columns of a grid": (lambda: st.laplace3d(24, 24, 24), {"tri_grid": 0}, 1),
+    "mesh with holes": (lambda: holes(*st.laplace3d(24, 23, 22), 50), {}, 1),
+    "2-D mesh with holes": (lambda: holes(*st.laplace2d(90, 71), 64), {}, 1),
+    "27-point": (lambda: st.convdiff27(16, seed=3), {}, 1),
+    "level pool": (lambda: st.laplace3d(24, 24, 24), {"tri_col": 0}, 0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SWEEPS))
+def test_sweep_paths_bitexact(engine, name):
+    mat, opts, path = SWEEPS[name]
+    p, i, v = mat()
+    n = len(p) - 1
+    dg, _ = oracle.diag(p, i)
+    f = oracle.ilu0(p, i, v, dg)
+    x = st.uniform(22, n)
+    with options(engine, **opts):
+        M = H.make_ilu(engine, engine.load(p), engine.load(i), engine.load(v), want_f32=True)
+        gx, gr = engine.load(x), engine.vector(n)
+        for _ in range(2):
+            M.apply(gx, gr)
+            assert engine.get_option("path_sweep") == path
+            assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(p, i, dg, f, x)))
+            M.apply_f32x64(gx, gr)
+            assert engine.get_option("path_sweep") == path
+            ref = oracle.ilu_apply_f32(p, i, dg, f.astype(np.float32), x.astype(np.float32)).astype(np.float64)
+            assert np.array_equal(bits(host(gr)), bits(ref))
+            M.apply_t(gx, gr)
+            assert engine.get_option("path_sweep") == path
+            assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply_t(p, i, dg, f, x)))
+
+
+@pytest.mark.parametrize("prec", ["identity", "jacobi"])
+@pytest.mark.parametrize("side,opts,path", [(64, {"cg_small": 0}, 1), (65, {}, 1), (64, {}, 2), (520, {}, 0)])
+def test_cg_paths_bitexact(engine, prec, side, opts, path):
+    p, i, v = st.laplace2d(side, side, diag=4.3)
+    n = len(p) - 1
+    d = np.full(n, 4.3)
+    b = st.uniform(404 + side, n)
+    kind = oracle.PREC_JACOBI if prec == "jacobi" else oracle.PREC_IDENTITY
+    it, x, hist = oracle.cg(p, i, v, b, tol=0.0, max_iter=40, prec=kind, mdata=d)
+    gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+    gx, gh = engine.vector(n), torch.zeros(64, dtype=torch.float64, device="cuda")
+    pre = ("jacobi", engine.load(d)) if prec == "jacobi" else None
+    with options(engine, **opts):
+        git = H.solve_cg(engine, H.stop_criteria(0.0, 40), gp, gi, gv, pre, engine.load(b), gx, hist=gh)
+    assert engine.get_option("path_cg") == path
+    assert git == it == 40
+    assert np.array_equal(bits(host(gh)[: it - 1]), bits(hist[: it - 1]))
+    assert np.array_equal(bits(host(gx)), bits(x))
+
+
+def test_path_names_are_read_only(engine):
+    with pytest.raises(H.HalaError, match="unknown option"):
+        engine.set_option("path_cg", 1)
+    with pytest.raises(H.HalaError, match="unknown option"):
+        engine.get_option("path_none")
