@@ -113,8 +113,8 @@ __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int
     double acc[G];
 #pragma unroll
     for (int k = 0; k < G; k++) acc[k] = 0.0;
-    csr_block_rowsums<double, G, TI, false, TO>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false, false,
-                                                sv, so, acc);
+    csr_block_rowsums<double, G, TI, false, TO, false>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false,
+                                                       false, sv, so, acc);
     static_assert(G * CB <= spmm_tile<double>::value, "tree scratch");
 #pragma unroll
     for (int k = 0; k < G; k++) {

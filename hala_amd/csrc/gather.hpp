@@ -14,6 +14,25 @@ constexpr TO gather_offset(int c, TO step) {
 // Whether the offsets of an n-element vector need 64 bits.
 constexpr bool gather_wide(int64_t n, int64_t step) { return n * step > (int64_t)UINT32_MAX; }
 
+// Whether the threads of a product walk their rows in memory instead of in staged tiles.  A staged block
+// keeps only the rows of the present tile at work: with more entries than a tile (`tile`) it waits for
+// one tile after the other, which other workgroups of the CU hide if there are any.  So the rows are
+// walked where the CUs hold at most per_cu of them (walk_per_cu), and where one row alone (max_row, 0: not
+// known) takes a good part of a tile.  Walking many blocks per CU loses the lines that neighbouring rows
+// share.  Staged -> walked (us), x vectors:
+//   27-point complex FP64, 250 blocks x1 35 -> 11, 432 x1 41 -> 18, 1024 x1 44 -> 61; transposed 432 57 -> 43, 1024 78 -> 133
+//   27-point FP64, 250 blocks x8 31 -> 20, 420 x8 34 -> 27, 762 x8 47 -> 54
+//   30 random entries FP64 per row, 235 blocks x8 83 -> 70, 293 x8 117 -> 142
+//   rows of 2 .. 3000 FP64, 391 blocks x2 325 -> 207
+constexpr bool walk_rows(int64_t entries, int blocks, int max_row, int tile, int num_cus, int per_cu) {
+    return (blocks <= num_cus * per_cu && entries > (int64_t)blocks * tile) || max_row > tile / 4;
+}
+// One, but two for 16-byte values, whose tiles are half as long; not for a transposed product of more than
+// two vectors (313 blocks of 15 entries a row, x1 33 -> 28, x3 50 -> 58).
+constexpr int walk_per_cu(int elem_bytes, bool trans, int ncols) {
+    return elem_bytes >= 16 && (!trans || ncols <= 2) ? 2 : 1;
+}
+
 // Where a loop over the entries [.., end) in tiles goes after base (never past
 // end: entry counts reach INT_MAX - 1).
 constexpr int tile_next(int base, int end, int tile) { return end - base > tile ? base + tile : end; }

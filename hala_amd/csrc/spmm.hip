@@ -5,8 +5,11 @@
 // columns, the vectors once): 64^3 27-point FP64 times 16 vectors 121 us, one
 // product per column 333 us; 701^2 5-point complex FP64 times 5 vectors 38 us,
 // one product per column (a thread per row, no staging) 184 us.  Groups of 8:
-// the row sums and the operands of two entries then fit 96 registers.
+// the row sums and the operands of two entries then fit 96 registers.  Few
+// workgroups of long rows are not staged (walk_rows): 2000 rows of 45 random
+// entries, complex FP64, 66 -> 10 us (19 us with a thread per row before).
 #include <algorithm>
+#include <type_traits>
 
 #include "spmm.hpp"
 
@@ -14,14 +17,14 @@ namespace hala_amd {
 
 namespace {
 
-template <class S, int G, class TI, bool TRANS, class TO>
+template <class S, int G, class TI, bool TRANS, class TO, bool WALK>
 __global__ __launch_bounds__(256) void spmm_rows_kernel(int nrows, const int *__restrict__ pntr,
                                                         const TI *__restrict__ indx, const int *__restrict__ tmap,
                                                         const S *__restrict__ vals, const S *__restrict__ x, int64_t sg,
                                                         TO step, S alpha, S beta, int conjv, int conjx, S *y,
                                                         int64_t ldy, int nc) {
-    __shared__ S sv[spmm_tile<S>::value];
-    __shared__ TO so[spmm_tile<S>::value];
+    __shared__ S sv[WALK ? 1 : spmm_tile<S>::value];
+    __shared__ TO so[WALK ? 1 : spmm_tile<S>::value];
     const int row = blockIdx.x * SPMV_ROWS + threadIdx.x;
     const char *xb[G];  // columns past nc repeat the last one (its loads hit in the cache); nothing is stored for them
 #pragma unroll
@@ -33,8 +36,8 @@ __global__ __launch_bounds__(256) void spmm_rows_kernel(int nrows, const int *__
         acc[k] = S{};
         if (TRANS && !bz && k < nc && row < nrows) acc[k] = cmul(beta, y[k * ldy + row]);
     }
-    csr_block_rowsums<S, G, TI, TRANS, TO>(nrows, pntr, indx, tmap, vals, xb, step, alpha, conjv != 0, conjx != 0, sv, so,
-                                       acc);
+    csr_block_rowsums<S, G, TI, TRANS, TO, WALK>(nrows, pntr, indx, tmap, vals, xb, step, alpha, conjv != 0, conjx != 0,
+                                                 sv, so, acc);
     if (row >= nrows) return;
 #pragma unroll
     for (int k = 0; k < G; k++) {
@@ -106,17 +109,22 @@ __global__ __launch_bounds__(256) void spmv_t_rows_kernel(int nrows, const int *
 template <class S, class TI, bool TRANS>
 void launch_group(hala_ctx c, int g, int nrows, const int *pntr, const TI *indx, const int *tmap, const S *vals,
                   const S *x, int64_t sg, int64_t step, S alpha, S beta, int conjv, int conjx, S *y, int64_t ldy,
-                  int nc, bool wide) {
-#define HALA_G(GG, TO)                                                                                     \
-    spmm_rows_kernel<S, GG, TI, TRANS, TO><<<g, SPMV_ROWS, 0, c->stream>>>(nrows, pntr, indx, tmap, vals, x, sg, \
-                                                                           (TO)step, alpha, beta, conjv, conjx, y, \
-                                                                           ldy, nc)
-    if (wide) HALA_G(1, uint64_t);
-    else if (nc > 6) HALA_G(8, unsigned);
-    else if (nc > 4) HALA_G(6, unsigned);
-    else if (nc > 2) HALA_G(4, unsigned);
-    else if (nc > 1) HALA_G(2, unsigned);
-    else HALA_G(1, unsigned);
+                  int nc, bool wide, bool walk) {
+#define HALA_G(GG, TO, WALK)                                                                                    \
+    spmm_rows_kernel<S, GG, TI, TRANS, TO, WALK><<<g, SPMV_ROWS, 0, c->stream>>>(nrows, pntr, indx, tmap, vals, x, sg, \
+                                                                                 (TO)step, alpha, beta, conjv,   \
+                                                                                 conjx, y, ldy, nc)
+    auto group = [&](auto w) {
+        constexpr bool WALK = decltype(w)::value;
+        if (nc > 6) HALA_G(8, unsigned, WALK);
+        else if (nc > 4) HALA_G(6, unsigned, WALK);
+        else if (nc > 2) HALA_G(4, unsigned, WALK);
+        else if (nc > 1) HALA_G(2, unsigned, WALK);
+        else HALA_G(1, unsigned, WALK);
+    };
+    if (wide) HALA_G(1, uint64_t, false);
+    else if (walk) group(std::true_type());
+    else group(std::false_type());
 #undef HALA_G
     HALA_CHECK_LAUNCH();
 }
@@ -133,12 +141,14 @@ void spmm_columns(hala_csr A, char trans, S alpha, const S *vals, const S *x, in
     const bool tr = !is_n(trans);
     const int nrows = tr ? A->ncols : A->nrows, ncin = tr ? A->nrows : A->ncols;
     if (tr) ensure_transpose(A);
-    c->path[PATH_PRODUCT] = 1;
-    if (nrows == 0 || ncols == 0) return;
     const int g = (nrows + SPMV_ROWS - 1) / SPMV_ROWS;
     const int conjv = is_c(trans) ? 1 : 0;
     const int64_t step = sc * (int64_t)sizeof(S);
     const bool wide = gather_wide(ncin, step);
+    const bool walk = !wide && walk_rows(A->nnz, g, tr ? 0 : A->max_row, spmm_tile<S>::value, c->num_cus,
+                                         walk_per_cu(sizeof(S), tr, ncols));
+    c->path[PATH_PRODUCT] = walk ? 2 : 1;
+    if (nrows == 0 || ncols == 0) return;
     const int gmax = wide ? 1 : 8;
     for (int c0 = 0; c0 < ncols; c0 += gmax) {
         const int nc = std::min(gmax, ncols - c0);
@@ -146,13 +156,13 @@ void spmm_columns(hala_csr A, char trans, S alpha, const S *vals, const S *x, in
         S *yc = y + c0 * ldy;
         if (tr)
             launch_group<S, int, true>(c, g, nrows, A->tp.tpntr.as<int>(), A->tp.trow.as<int>(), A->tp.tmap.as<int>(),
-                                       vals, xc, sg, step, alpha, beta, conjv, conjx, yc, ldy, nc, wide);
+                                       vals, xc, sg, step, alpha, beta, conjv, conjx, yc, ldy, nc, wide, walk);
         else if (A->boff.p)
             launch_group<S, short, false>(c, g, nrows, A->pntr, A->boff.as<short>(), nullptr, vals, xc, sg, step, alpha,
-                                          beta, 0, conjx, yc, ldy, nc, wide);
+                                          beta, 0, conjx, yc, ldy, nc, wide, walk);
         else
             launch_group<S, int, false>(c, g, nrows, A->pntr, A->indx, nullptr, vals, xc, sg, step, alpha, beta, 0,
-                                        conjx, yc, ldy, nc, wide);
+                                        conjx, yc, ldy, nc, wide, walk);
     }
 }
 
@@ -161,6 +171,13 @@ void spmv_trans(hala_csr A, T alpha, const T *vals, const T *x, T beta, T *y) {
     ensure_transpose(A);
     hala_ctx c = A->ctx;
     if (A->ncols == 0) return;
+    // a few workgroups of rows of several tiles each: walked (2000 x 2000, 45 random entries per row in
+    // FP64: 26 us staged, 23 us with a thread per row before there were tiles)
+    const int blocks = (A->ncols + SPMV_ROWS - 1) / SPMV_ROWS;
+    if (blocks <= c->num_cus && A->nnz > (int64_t)blocks * 4 * spmv_tile<T>::value) {
+        spmm_columns<T>(A, 'T', alpha, vals, x, 0, 1, false, beta, y, 0, 1);
+        return;
+    }
     spmv_t_rows_kernel<T><<<(A->ncols + SPMV_ROWS - 1) / SPMV_ROWS, SPMV_ROWS, 0, c->stream>>>(
         A->ncols, A->tp.tpntr.as<int>(), A->tp.trow.as<int>(), A->tp.tmap.as<int>(), vals, x, alpha, beta, y);
     HALA_CHECK_LAUNCH();

@@ -6,7 +6,8 @@
 // vectors at once: a matrix entry is read once per G vectors instead of once
 // per vector, and a wavefront's gathers of one entry position go to
 // neighbouring elements of the vectors wherever neighbouring rows have
-// neighbouring columns.
+// neighbouring columns.  A few workgroups of long rows, and rows that fill
+// tiles by themselves, are walked in memory instead (walk_rows in gather.hpp).
 #pragma once
 #include "scalar.hpp"
 #include "spmv.hpp"
@@ -21,8 +22,9 @@ struct spmm_tile {
 // acc[k] = op over the row's entries, k < G: acc + v * x_k (N), acc + (alpha * x_k) * v (TRANS).
 // x_k(c) is at xb[k] + c * step bytes (TO: uint64_t where gather_wide() of the vector, else unsigned).  TI = short: columns as offsets from
 // the block's first row.
-// Must be called by all 256 threads of the block; sv, so: spmm_tile entries of LDS each.
-template <class S, int G, class TI, bool TRANS, class TO>
+// WALK: each thread reads its row's entries from memory itself (walk_rows), nothing is staged.
+// Must be called by all 256 threads of the block; sv, so: spmm_tile entries of LDS each (WALK: unused).
+template <class S, int G, class TI, bool TRANS, class TO, bool WALK>
 __device__ __forceinline__ void csr_block_rowsums(int nrows, const int *__restrict__ pntr, const TI *__restrict__ indx,
                                                   const int *__restrict__ tmap, const S *__restrict__ vals,
                                                   const char *const (&xb)[G], TO step, S alpha, bool conjv,
@@ -37,6 +39,26 @@ __device__ __forceinline__ void csr_block_rowsums(int nrows, const int *__restri
         rs = pntr[row];
         re = pntr[row + 1];
     }
+    // one entry into the G sums
+    auto add = [&](const S v, const TO o) {
+        S x[G];
+#pragma unroll
+        for (int k = 0; k < G; k++) x[k] = *reinterpret_cast<const S *>(xb[k] + o);
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            if (is_complex<S>::value && conjx) x[k] = cconj(x[k]);
+            acc[k] = cadd(acc[k], TRANS ? cmul(cmul(alpha, x[k]), v) : cmul(v, x[k]));
+        }
+    };
+    if constexpr (WALK) {
+#pragma unroll 4
+        for (int j = rs; j < re; j++) {
+            S v = vals[TRANS ? tmap[j] : j];
+            if (is_complex<S>::value && conjv) v = cconj(v);
+            add(v, gather_offset<TO>(cb + (int)indx[j], step));
+        }
+        return;
+    }
     for (int base = bstart; base < bend; base = tile_next(base, bend, TILE)) {
         const int cnt = min(TILE, bend - base);
 #pragma unroll 4
@@ -50,18 +72,7 @@ __device__ __forceinline__ void csr_block_rowsums(int nrows, const int *__restri
         __syncthreads();
         const int a = max(rs, base) - base, b = min(re, base + cnt) - base;
 #pragma unroll 2
-        for (int j = a; j < b; j++) {
-            const S v = sv[j];
-            const TO o = so[j];
-            S x[G];
-#pragma unroll
-            for (int k = 0; k < G; k++) x[k] = *reinterpret_cast<const S *>(xb[k] + o);
-#pragma unroll
-            for (int k = 0; k < G; k++) {
-                if (is_complex<S>::value && conjx) x[k] = cconj(x[k]);
-                acc[k] = cadd(acc[k], TRANS ? cmul(cmul(alpha, x[k]), v) : cmul(v, x[k]));
-            }
-        }
+        for (int j = a; j < b; j++) add(sv[j], so[j]);
         __syncthreads();
     }
 }

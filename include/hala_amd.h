@@ -83,7 +83,7 @@ int hala_ctx_device(hala_ctx ctx, int *device);
  * of the small and the large size class), "path_jacobi" (Jacobi-applied ILU,
  * L + 4 U; 0 packed rows, 1 with int16 offsets, 2 columns of 256 rows),
  * "path_product" (sparse times dense, transposed, complex; 0 the single
- * product per column, 1 several columns at once). */
+ * product per column, 1 several columns at once, 2 the same without staging). */
 int hala_ctx_set_option(hala_ctx ctx, const char *name, int value);
 int hala_ctx_get_option(hala_ctx ctx, const char *name, int *value);
 

@@ -48,5 +48,11 @@ int main() {
         for (int end : {0, 1, tile - 1, tile, tile + 1, 3 * tile + 5, INT_MAX - 1, INT_MAX})
             for (int len : {0, 1, tile - 1, tile, tile + 1, 5 * tile - 3})
                 if (len <= end) check(covers(end - len, end, tile), "tile loop");
+    check(walk_rows(257 * 2048, 256, 9, 2048, 256, 1) && !walk_rows(257 * 2048, 257, 9, 2048, 256, 1) &&
+              walk_rows(513 * 1024, 512, 9, 1024, 256, 2) && !walk_rows(100 * 2048, 100, 9, 2048, 256, 1) &&
+              walk_rows(100, 1000, 513, 2048, 256, 1) && walk_rows(INT_MAX, 200, 0, 2048, 256, 1) &&
+              walk_per_cu(16, false, 8) == 2 && walk_per_cu(16, true, 2) == 2 && walk_per_cu(16, true, 3) == 1 &&
+              walk_per_cu(8, false, 1) == 1,
+          "walked rows");
     return failures ? 1 : 0;
 }

@@ -71,8 +71,7 @@ def test_spmm_columns(engine, mat, ct):
             A.gemm(ta, tb, k if tb == "N" else cols, cols if tb == "N" else k, 1.5, engine.load(B), ldb, beta, gC, ldc)
             got = host(gC)
             assert np.array_equal(raw(got[:, m:]), raw(C0[:, m:]))  # nothing written past a column
-            single = (tb == "N" and cols == 1) or (ta == "N" and A.info()["kernel"] == 1)
-            assert engine.get_option("path_product") == (0 if single and not cplx else 1)
+            assert engine.get_option("path_product") == product_path(A, ct, nr, nc, len(i), ta, tb, cols)
             for c in range(cols):
                 x = np.ascontiguousarray(B[c, :k] if tb == "N" else (B[:, c].conj() if tb == "C" else B[:, c]))
                 y = np.ascontiguousarray(C0[c, :m])
@@ -86,6 +85,85 @@ def test_spmm_columns(engine, mat, ct):
                     oracle.zspmv(ta, nr, nc, 1.5 + 0j, p, i, v.astype(w), x.astype(w), complex(beta), yc)
                     y = yc if cplx else yc.real.astype(np.float32)
                 assert np.array_equal(raw(got[c, :m]), raw(y)), (ta, tb, cols, c)
+
+
+def product_path(A, ct, nr, nc, nnz, ta, tb, cols):
+    """The product's dispatch: 0 single products, 1 staged tiles, 2 rows walked in memory."""
+    es = np.dtype(ct).itemsize
+    cplx = np.issubdtype(ct, np.complexfloating)
+    if not cplx and ((tb == "N" and cols == 1) or (ta == "N" and A.info()["kernel"] == 1)):
+        return 0
+    blocks = ((nr if ta == "N" else nc) + 255) // 256
+    tile = 1024 if es == 16 else 2048
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    few = blocks <= cus * (2 if es == 16 and (ta == "N" or cols <= 2) else 1) and nnz > blocks * tile
+    return 2 if few or (ta == "N" and A.info()["max_row"] > tile // 4) else 1
+
+
+MANY = {  # more workgroups than the rule walks, and more than a tile of entries in each; one fewer than it stages
+    "27-point 41^3": (lambda: st.convdiff27(41), (np.float64, np.float32)),
+    "27-point 40^3": (lambda: st.convdiff27(40), (np.float64, np.float32)),
+    "7-point 51^3": (lambda: st.laplace3d(51, 51, 51), (np.complex128,)),
+    "7-point 50^3": (lambda: st.laplace3d(50, 50, 50), (np.complex128,)),
+}
+
+
+@pytest.mark.parametrize("mat", sorted(MANY))
+def test_spmm_many_tiles(engine, mat):
+    gen, types = MANY[mat]
+    p, i, v = gen()
+    n = len(p) - 1
+    rng = np.random.default_rng(2)
+    for ct in types:
+        cplx = ct == np.complex128
+        w = (v * (1 + 0.5j) if cplx else v).astype(ct)
+        A = H.make_sparse_matrix(engine, n, engine.load(p), engine.load(i), engine.load(w))
+        paths = set()
+        for ta in ("N", "T"):
+            for cols in (1, 2, 8):
+                B = (rng.uniform(-1, 1, (cols, n)) + (1j * rng.uniform(-1, 1, (cols, n)) if cplx else 0)).astype(ct)
+                gC = torch.zeros(cols, n, dtype=torch.from_numpy(B).dtype, device="cuda")
+                A.gemm(ta, "N", n, cols, 1.5, engine.load(B), n, 0.0, gC, n)
+                path = engine.get_option("path_product")
+                if ta == "N" or cols > 1:  # (a single real transposed product picks by rules of its own)
+                    assert path == product_path(A, ct, n, n, len(i), ta, "N", cols)
+                    paths.add(path)
+                got = host(gC)
+                for c in {0, cols - 1}:
+                    if ct == np.float64:
+                        ref = oracle.spmv(ta, n, n, 1.5, p, i, w, B[c], 0.0, np.zeros(n))
+                    elif ct == np.float32 and ta == "N":
+                        ref = oracle.spmv_f32(p, i, w, B[c], alpha=1.5, beta=0.0, y=np.zeros(n, ct))
+                    else:
+                        z = ct if cplx else np.complex64
+                        ref = np.zeros(n, z)
+                        oracle.zspmv(ta, n, n, 1.5 + 0j, p, i, w.astype(z), B[c].astype(z), 0j, ref)
+                        ref = ref if cplx else ref.real.astype(np.float32)
+                    assert np.array_equal(raw(got[c]), raw(ref)), (ct, ta, cols, c)
+        assert (1 if mat in ("27-point 41^3", "7-point 51^3") else 2) in paths
+
+
+def test_transposed_product_of_few_long_rows(engine):
+    # a few workgroups of rows of several tiles: the single transposed product walks them too
+    rng = np.random.default_rng(11)
+    n, k = 600, 45
+    i = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for _ in range(n)]).astype(np.int32)
+    p = np.arange(0, n * k + 1, k, dtype=np.int32)
+    for ct in (np.float64, np.float32):
+        v = rng.uniform(-1, 1, n * k).astype(ct)
+        A = H.make_sparse_matrix(engine, n, engine.load(p), engine.load(i), engine.load(v))
+        x, y = rng.uniform(-1, 1, n).astype(ct), rng.uniform(-1, 1, n).astype(ct)
+        for beta in (0.0, 0.5):
+            gy = engine.load(y)
+            A.gemv("T", 1.5, engine.load(x), beta, gy)
+            if ct == np.float64:
+                assert engine.get_option("path_product") == 2
+                ref = oracle.spmv("T", n, n, 1.5, p, i, v, x, beta, y.copy())
+            else:
+                ref = y.astype(np.complex64)
+                oracle.zspmv("T", n, n, 1.5 + 0j, p, i, v.astype(np.complex64), x.astype(np.complex64), complex(beta), ref)
+                ref = ref.real.astype(ct)
+            assert np.array_equal(raw(host(gy)), raw(ref))
 
 
 TRI = {
