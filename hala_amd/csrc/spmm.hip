@@ -149,7 +149,8 @@ void spmm_columns(hala_csr A, char trans, S alpha, const S *vals, const S *x, in
                                          walk_per_cu(sizeof(S), tr, ncols));
     c->path[PATH_PRODUCT] = walk ? 2 : 1;
     if (nrows == 0 || ncols == 0) return;
-    const int gmax = wide ? 1 : 8;
+    const bool apart = A->spread && !tr && !walk && !is_complex<S>::value && sc == 1;
+    const int gmax = wide ? 1 : apart ? gather_group(ncin * (int64_t)sizeof(S)) : 8;
     for (int c0 = 0; c0 < ncols; c0 += gmax) {
         const int nc = std::min(gmax, ncols - c0);
         const S *xc = x + c0 * sg;
@@ -200,11 +201,13 @@ void spmm(hala_csr A, char transa, char transb, int b_rows, int b_cols, S alpha,
     HALA_REQUIRE(N == 0 || vals || A->nnz == 0, HALA_ERR_ARG, "spmm: null pointer");
     const bool bn = is_n(transb);
     // one column of a real product (its products are formed in entry order:
-    // more gathers in flight), and rows too long for a thread each (one
-    // wavefront per row), run the single product's kernels
+    // more gathers in flight), vectors too long for a group of them
+    // (gather_group), and rows too long for a thread each (one wavefront per
+    // row), run the single product's kernels
     const int64_t sg = bn ? ldb : 1, sc = bn ? 1 : ldb;
     if constexpr (!is_complex<S>::value) {
-        if ((bn && N == 1) || (is_n(transa) && A->kernel == 1)) {
+        const bool alone = bn && is_n(transa) && A->spread && gather_group(K * (int64_t)sizeof(S)) == 1;
+        if ((bn && N == 1) || alone || (is_n(transa) && A->kernel == 1)) {
             hala_ctx c = A->ctx;
             c->path[PATH_PRODUCT] = 0;
             tmp_scope ts(c);

@@ -10,13 +10,31 @@ namespace hala_amd {
 // ---------------------------------------------------------------------------
 // row statistics and validation
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void row_stats_kernel(int nrows, const int *__restrict__ pntr, int *out) {
-    __shared__ int smax[256], smin[256];
+// out[0], out[1]: longest and shortest row.  out[5], out[6]: entries of the sampled rows (about 2048 rows, at
+// most SPREAD_LEN entries of each), and those of them one column right of an entry of the row above.
+constexpr int SPREAD_LEN = 64;
+__global__ __launch_bounds__(256) void row_stats_kernel(int nrows, const int *__restrict__ pntr,
+                                                        const int *__restrict__ indx, int *out) {
+    __shared__ int smax[256], smin[256], ssum[2];
+    if (threadIdx.x < 2) ssum[threadIdx.x] = 0;
+    __syncthreads();
+    const int step = max(64, nrows / 2048);
     int mx = 0, mn = INT_MAX;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < nrows; i += gridDim.x * 256) {
-        int l = pntr[i + 1] - pntr[i];
+        const int s = pntr[i], l = pntr[i + 1] - s;
         mx = max(mx, l);
         mn = min(mn, l);
+        if (i % step == 1) {
+            const int above = pntr[i - 1], m = min(l, SPREAD_LEN);
+            int next = 0;
+            for (int k = 0, q = above; k < m; k++) {
+                const int c = indx[s + k] - 1;
+                while (q < s && indx[q] < c) q++;
+                next += q < s && indx[q] == c;
+            }
+            atomicAdd(ssum, m);
+            atomicAdd(ssum + 1, next);
+        }
     }
     smax[threadIdx.x] = mx;
     smin[threadIdx.x] = mn;
@@ -31,10 +49,14 @@ __global__ __launch_bounds__(256) void row_stats_kernel(int nrows, const int *__
     if (threadIdx.x == 0) {
         atomicMax(out, smax[0]);
         atomicMin(out + 1, smin[0]);
+        if (ssum[0]) atomicAdd(out + 5, ssum[0]);
+        if (ssum[1]) atomicAdd(out + 6, ssum[1]);
     }
 }
 
 __global__ void init_stats(int *out) {
+    out[5] = 0;
+    out[6] = 0;
     out[0] = 0;
     out[1] = INT_MAX;
     out[2] = INT_MAX;
@@ -79,7 +101,7 @@ bool build_block_offsets(hala_ctx c, int nrows, int64_t nnz, const int *ptr, con
     if (nrows <= 0 || nnz <= 0) return false;
     tmp_scope ts(c);
     dbuf &st = ts.get();
-    st.reserve(5 * sizeof(int));
+    st.reserve(7 * sizeof(int));
     init_stats<<<1, 1, 0, c->stream>>>(st.as<int>());
     block_offset_kernel<<<(nrows + 255) / 256, 256, 0, c->stream>>>(nrows, ptr, idx, st.as<int>());
     HALA_CHECK_LAUNCH();
@@ -279,11 +301,11 @@ int hala_csr_create(hala_ctx c, int nrows, int ncols, int64_t nnz, const int *pn
             }
             int *st = reinterpret_cast<int *>(c->scal.as<double>() + S_DOT + 2);
             init_stats<<<1, 1, 0, c->stream>>>(st);
-            row_stats_kernel<<<grid_for(nrows, 256 * 8, 1024), 256, 0, c->stream>>>(nrows, pntr, st);
+            row_stats_kernel<<<grid_for(nrows, 256 * 8, 1024), 256, 0, c->stream>>>(nrows, pntr, indx, st);
             block_offset_kernel<<<(nrows + 255) / 256, 256, 0, c->stream>>>(nrows, pntr, indx, st);
-            int h[5];
+            int h[7];
             hipError_t e1 = hipGetLastError();
-            if (e1 == hipSuccess) e1 = hipMemcpyAsync(c->host_pinned, st, 5 * sizeof(int), hipMemcpyDeviceToHost, c->stream);
+            if (e1 == hipSuccess) e1 = hipMemcpyAsync(c->host_pinned, st, 7 * sizeof(int), hipMemcpyDeviceToHost, c->stream);
             if (e1 == hipSuccess) e1 = hipStreamSynchronize(c->stream);
             if (e1 != hipSuccess) {
                 delete A;
@@ -293,6 +315,7 @@ int hala_csr_create(hala_ctx c, int nrows, int ncols, int64_t nnz, const int *pn
             A->max_row = h[0];
             A->min_row = h[1];
             A->mean_row = (double)nnz / nrows;
+            A->spread = 2 * (int64_t)h[6] < h[5];
             // Short rows (every stencil here): LDS-staged blocks keep the
             // index/value streams fully coalesced and sum each row in CSR
             // order.  Long rows waste the per-row thread there: one

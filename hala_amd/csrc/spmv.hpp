@@ -17,6 +17,9 @@ struct hala_csr_s {
     // row, when every offset fits (banded patterns: every stencil here); null
     // otherwise.  The LDS-staged products stream it instead of indx.
     hala_amd::dbuf boff;
+    // neighbouring rows seldom hold neighbouring columns (random and ragged
+    // patterns; stencils do), by a sample of the rows
+    bool spread = false;
 };
 
 namespace hala_amd {

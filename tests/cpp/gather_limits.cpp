@@ -54,5 +54,9 @@ int main() {
               walk_per_cu(16, false, 8) == 2 && walk_per_cu(16, true, 2) == 2 && walk_per_cu(16, true, 3) == 1 &&
               walk_per_cu(8, false, 1) == 1,
           "walked rows");
+    check(gather_group(1) == 8 && gather_group(1 << 19) == 8 && gather_group((1 << 19) + 1) == 4 &&
+              gather_group((1 << 20) + 1) == 2 && gather_group((1 << 21) + 1) == 1 &&
+              gather_group(int64_t(INT_MAX) * 16) == 1,
+          "vectors at once");
     return failures ? 1 : 0;
 }

@@ -40,6 +40,8 @@ MATS = {
     "ragged": lambda: (*ragged(517, 3000, 3, 9), 3000),  # a row and a tile longer than the staging
     "wide": lambda: (*ragged(260, 70000, 4, 5), 70000),  # int32 columns, a row for the wavefront kernel
     "wide short": lambda: (*ragged(260, 70000, 6, 5, full=False), 70000),
+    "wide pairs": lambda: (*ragged(260, 140000, 7, 5, full=False), 140000),  # FP64 two columns at once, FP32 four
+    "wide alone": lambda: (*ragged(260, 540000, 8, 5, full=False), 540000),  # FP64 one, FP32 one
     "one": lambda: (np.array([0, 1], np.int32), np.array([0], np.int32), 1),
     "empty": lambda: (np.zeros(301, np.int32), np.zeros(0, np.int32), 40),
 }
@@ -91,7 +93,9 @@ def product_path(A, ct, nr, nc, nnz, ta, tb, cols):
     """The product's dispatch: 0 single products, 1 staged tiles, 2 rows walked in memory."""
     es = np.dtype(ct).itemsize
     cplx = np.issubdtype(ct, np.complexfloating)
-    if not cplx and ((tb == "N" and cols == 1) or (ta == "N" and A.info()["kernel"] == 1)):
+    # vectors past half an XCD's L2 on a pattern without parallel rows: one by one
+    alone = ta == "N" and tb == "N" and nc > nr and 2 * nc * es > 4 << 20
+    if not cplx and ((tb == "N" and cols == 1) or alone or (ta == "N" and A.info()["kernel"] == 1)):
         return 0
     blocks = ((nr if ta == "N" else nc) + 255) // 256
     tile = 1024 if es == 16 else 2048
@@ -103,6 +107,7 @@ def product_path(A, ct, nr, nc, nnz, ta, tb, cols):
 MANY = {  # more workgroups than the rule walks, and more than a tile of entries in each; one fewer than it stages
     "27-point 41^3": (lambda: st.convdiff27(41), (np.float64, np.float32)),
     "27-point 40^3": (lambda: st.convdiff27(40), (np.float64, np.float32)),
+    "5-point 530^2": (lambda: st.laplace2d(530, 530), (np.float64,)),  # long vectors, parallel rows: not one by one
     "7-point 51^3": (lambda: st.laplace3d(51, 51, 51), (np.complex128,)),
     "7-point 50^3": (lambda: st.laplace3d(50, 50, 50), (np.complex128,)),
 }
@@ -140,7 +145,7 @@ def test_spmm_many_tiles(engine, mat):
                         oracle.zspmv(ta, n, n, 1.5 + 0j, p, i, w.astype(z), B[c].astype(z), 0j, ref)
                         ref = ref if cplx else ref.real.astype(np.float32)
                     assert np.array_equal(raw(got[c]), raw(ref)), (ct, ta, cols, c)
-        assert (1 if mat in ("27-point 41^3", "7-point 51^3") else 2) in paths
+        assert (1 if mat in ("27-point 41^3", "5-point 530^2", "7-point 51^3") else 2) in paths
 
 
 def test_transposed_product_of_few_long_rows(engine):
