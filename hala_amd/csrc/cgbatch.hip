@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "blas1.hpp"
 #include "solvers.hpp"
@@ -93,18 +94,46 @@ __global__ __launch_bounds__(256) void cgb_start(int n, const double *__restrict
     }
 }
 
+// The row sum of thread threadIdx.x of the block: the block's products formed in entry order by all threads
+// tile by tile, each row's added in order by its thread, several LDS reads ahead of the chain of sums.
+template <class TI>
+__device__ __forceinline__ double cgb_products(int n, const int *__restrict__ pntr, const TI *__restrict__ indx,
+                                               const double *__restrict__ vals, const double *__restrict__ p,
+                                               double *prod) {
+    constexpr int TILE = spmm_tile<double>::value;
+    const int r0 = blockIdx.x * SPMV_ROWS, row = r0 + threadIdx.x, cb = sizeof(TI) == 2 ? r0 : 0;
+    const int bstart = pntr[r0], bend = pntr[min(r0 + SPMV_ROWS, n)];
+    const int rs = row < n ? pntr[row] : 0, re = row < n ? pntr[row + 1] : 0;
+    double acc = 0.0;
+    for (int base = bstart; base < bend; base = tile_next(base, bend, TILE)) {
+        const int cnt = min(TILE, bend - base);
+#pragma unroll 4
+        for (int e = threadIdx.x; e < cnt; e += SPMV_ROWS) prod[e] = vals[base + e] * p[cb + (int)indx[base + e]];
+        __syncthreads();
+        const int a = max(rs, base) - base, b = min(re, base + cnt) - base;
+#pragma unroll 8
+        for (int j = a; j < b; j++) acc = acc + prod[j];
+        __syncthreads();
+    }
+    return acc;
+}
+
 // Ap_k = A p_k for columns c0 .. c0+nc-1 (nc <= G), each matrix entry read
 // once; fused <p_k, Ap_k>, and block k forms a_k = zr_k / <p_k, Ap_k> (a
 // collector per column: one block collecting eight in turn costs eight
 // reduction latencies).
-template <int G, class TI, class TO>
+// MODE: the rows' entries staged, walked in memory (walk_rows), or (one column) their products formed in
+// entry order by all threads, so that a row that fills tiles by itself is summed out of LDS.
+enum cgb_mode { CGB_STAGED, CGB_WALK, CGB_PRODUCTS };
+template <int G, class TI, class TO, cgb_mode MODE>
 __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int *__restrict__ pntr,
                                                 const TI *__restrict__ indx, const double *__restrict__ vals,
                                                 const double *__restrict__ Pv, double *__restrict__ AP, double *part,
                                                 const double *zr, double *al, cgb_state *st, int *err) {
     if (st->done) return;
-    __shared__ double sv[spmm_tile<double>::value];
-    __shared__ TO so[spmm_tile<double>::value];
+    static_assert(MODE != CGB_PRODUCTS || G == 1, "one column");
+    __shared__ double sv[MODE == CGB_WALK ? G * CB : spmm_tile<double>::value];
+    __shared__ TO so[MODE == CGB_STAGED ? spmm_tile<double>::value : 1];
     const int64_t nb = ((int64_t)n + CB - 1) / CB;
     const int row = blockIdx.x * SPMV_ROWS + threadIdx.x;
     const char *xb[G];
@@ -113,8 +142,11 @@ __global__ __launch_bounds__(256) void cgb_spmm(int n, int c0, int nc, const int
     double acc[G];
 #pragma unroll
     for (int k = 0; k < G; k++) acc[k] = 0.0;
-    csr_block_rowsums<double, G, TI, false, TO, false>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0, false,
-                                                       false, sv, so, acc);
+    if constexpr (MODE == CGB_PRODUCTS)
+        acc[0] = cgb_products<TI>(n, pntr, indx, vals, reinterpret_cast<const double *>(xb[0]), sv);
+    else
+        csr_block_rowsums<double, G, TI, false, TO, MODE == CGB_WALK>(n, pntr, indx, nullptr, vals, xb, sizeof(double), 1.0,
+                                                                      false, false, sv, so, acc);
     static_assert(G * CB <= spmm_tile<double>::value, "tree scratch");
 #pragma unroll
     for (int k = 0; k < G; k++) {
@@ -239,6 +271,43 @@ void cgb_read(hala_ctx c, cgb_state *st, int *it, int *done, double *rn) {
     if (rn) *rn = h.rn;
 }
 
+// Whether the product walks its rows.
+bool cgb_walks(hala_csr A) {
+    const int blocks = (A->nrows + SPMV_ROWS - 1) / SPMV_ROWS;
+    return walk_rows(A->nnz, blocks, A->max_row, spmm_tile<double>::value, A->ctx->num_cus, 1);
+}
+
+// The product of columns c0 .. c0+nc-1.  One column with a row that fills a good part of a tile: products
+// (arrow matrix of 8000 rows, 11 passes: 1.4 ms, walked 5.0, staged 5.8).
+template <class TI>
+void cgb_spmm_of(hala_csr A, const TI *indx, const double *vals, int c0, int nc, const double *Pv, double *AP,
+                 double *part, const double *zr, double *al, cgb_state *st) {
+    hala_ctx c = A->ctx;
+    const int n = A->nrows, gs = (n + SPMV_ROWS - 1) / SPMV_ROWS;
+    const bool walk = cgb_walks(A);
+#define HALA_CGB(G, TO, MODE)                                                                                   \
+    cgb_spmm<G, TI, TO, MODE><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, indx, vals, Pv, AP, part, zr, al, st, \
+                                                         wait_error_flag(c))
+    auto run = [&](auto w) {
+        constexpr cgb_mode MODE = decltype(w)::value ? CGB_WALK : CGB_STAGED;
+        if (nc > 4) HALA_CGB(8, unsigned, MODE);
+        else if (nc > 2) HALA_CGB(4, unsigned, MODE);
+        else if (nc > 1) HALA_CGB(2, unsigned, MODE);
+        else HALA_CGB(1, unsigned, MODE);
+    };
+    if (nc == 1 && A->max_row > spmm_tile<double>::value / 4) HALA_CGB(1, unsigned, CGB_PRODUCTS);
+    else if (gather_wide(n, sizeof(double))) HALA_CGB(8, uint64_t, CGB_STAGED);
+    else if (walk) run(std::true_type());
+    else run(std::false_type());
+#undef HALA_CGB
+    c->path[PATH_PRODUCT] = nc == 1 && A->max_row > spmm_tile<double>::value / 4 ? 0 : walk ? 2 : 1;
+}
+void launch_cgb_spmm(hala_csr A, const double *vals, int c0, int nc, const double *Pv, double *AP, double *part,
+                     const double *zr, double *al, cgb_state *st) {
+    if (A->boff.p) cgb_spmm_of(A, A->boff.as<short>(), vals, c0, nc, Pv, AP, part, zr, al, st);
+    else cgb_spmm_of(A, A->indx, vals, c0, nc, Pv, AP, part, zr, al, st);
+}
+
 }  // namespace
 
 void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nrhs, const double *B, double *X,
@@ -277,27 +346,11 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
         cgb_start<false><<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, R, Z, Pv, part, zr, wait_error_flag(c));
     }
     HALA_CHECK_LAUNCH();
+    // columns per product launch: pairs at least (a launch and its reductions per column cost more than the
+    // gathers save: 600 000 rows of 10 random entries, 8 columns, 9.9 ms by eight, 7.0 by two)
+    const int group = A->spread && !cgb_walks(A) ? std::max(2, gather_group(n * (int64_t)sizeof(double))) : CGB_GROUP;
     auto one_pass = [&]() {
-        for (int c0 = 0; c0 < nrhs; c0 += CGB_GROUP) {
-            const int nc = std::min(CGB_GROUP, nrhs - c0);
-#define HALA_CGB(GG, TO)                                                                                       \
-    if (A->boff.p)                                                                                            \
-        cgb_spmm<GG, short, TO><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->boff.as<short>(), vals, Pv, AP, \
-                                                           part, zr, al, st, wait_error_flag(c));              \
-    else                                                                                                      \
-        cgb_spmm<GG, int, TO><<<gs, 256, 0, c->stream>>>(n, c0, nc, A->pntr, A->indx, vals, Pv, AP, part, zr, al, \
-                                                         st, wait_error_flag(c))
-            if (gather_wide(n, sizeof(double))) {
-                HALA_CGB(8, uint64_t);
-            } else if (nc > 4) {
-                HALA_CGB(8, unsigned);
-            } else if (nc > 2) {
-                HALA_CGB(4, unsigned);
-            } else {
-                HALA_CGB(2, unsigned);
-            }
-#undef HALA_CGB
-        }
+        for (int c0 = 0; c0 < nrhs; c0 += group) launch_cgb_spmm(A, vals, c0, std::min(group, nrhs - c0), Pv, AP, part, zr, al, st);
         cgb_update<<<dim3(ge, nrhs), 256, 0, c->stream>>>(n, Pv, AP, X, R, part, al, rr, st, wait_error_flag(c),
                                                           fused ? ends.in_slot : nullptr, ends.in, N_);
         cgb_stop<<<1, 1, 0, c->stream>>>(nrhs, rr, st);

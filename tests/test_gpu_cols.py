@@ -240,3 +240,48 @@ def test_multirhs_pcg_grid_and_columns(engine, name, nrhs):
             assert np.array_equal(bits(host(X[k])), bits(x)), k
     finally:
         engine.set_option("tri_grid", saved)
+
+
+def spd(n, extra, full_row, seed):
+    """Symmetric, diagonally dominant: `extra` random couplings per row, with full_row one row coupled to all."""
+    rng = np.random.default_rng(seed)
+    a, b = rng.integers(0, n, n * extra // 2), rng.integers(0, n, n * extra // 2)
+    if full_row:
+        a, b = np.concatenate([a, np.full(n, n // 3)]), np.concatenate([b, np.arange(n)])
+    d = np.arange(n, dtype=np.int64)
+    key = np.unique(np.concatenate([a * np.int64(n) + b, b * np.int64(n) + a, d * n + d]))
+    row, col = key // n, (key % n).astype(np.int32)
+    p = np.zeros(n + 1, np.int32)
+    p[1:] = np.cumsum(np.bincount(row, minlength=n))
+    v = np.where(row == col, 2.0 * np.diff(p)[row], -1.0 / (1 + (row + col) % 5))
+    return p, col, v
+
+
+MULTI = {  # name: (matrix, path of the product of several columns, of one column)
+    "grid": (lambda: st.laplace3d(17, 18, 19), 1, 1),
+    "a long row": (lambda: spd(3000, 3, True, 5), 2, 0),
+    "few workgroups of long rows": (lambda: spd(700, 30, False, 6), 2, 2),
+    "random, groups of four": (lambda: spd(70000, 4, False, 7), 1, 1),
+    "random, pairs": (lambda: spd(270000, 4, False, 8), 1, 1),
+}
+
+
+@pytest.mark.parametrize("name", sorted(MULTI))
+def test_multirhs_cg_products(engine, name):
+    mat, path, path1 = MULTI[name]
+    p, i, v = mat()
+    n = len(p) - 1
+    gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+    A = H.make_sparse_matrix(engine, n, gp, gi, gv)
+    passes = 5
+    for nrhs in (1, 2, 3, 5, 8, 9):
+        B = np.stack([st.uniform(60 + k, n) for k in range(nrhs)])
+        X = torch.zeros(nrhs, n, dtype=torch.float64, device="cuda")
+        it = H.solve_batch_cg(engine, H.stop_criteria(0.0, passes), gp, gi, gv, None, engine.load(B), X, matrix=A)
+        # of the last group: nine columns leave one over a group of eight, four or two, three one over two
+        last = nrhs == 1 or nrhs == 9 or (name.endswith("pairs") and nrhs in (3, 5)) or (name.endswith("four") and nrhs == 5)
+        assert engine.get_option("path_product") == (path1 if last else path)
+        assert it == passes
+        for k in sorted({0, nrhs // 2, nrhs - 1}):
+            _, x, _ = oracle.cg(p, i, v, B[k], tol=0.0, max_iter=passes)
+            assert np.array_equal(bits(host(X[k])), bits(x)), (nrhs, k)
