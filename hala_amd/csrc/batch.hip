@@ -417,8 +417,19 @@ static bool resident(hala_batch B, hipStream_t s, int wg, const double *vals, co
     return true;
 }
 
+// A CU's registers hold 16 wavefronts of them, the general loop up to 32: a shape that asks for more on
+// systems with few rows per thread, where barriers are all there is to hide, runs faster on the loop.  Team
+// 1024, 2 per CU, general -> resident (us, 12 passes): 256 rows 307 -> 447, 512 204 -> 254, 1024 167 -> 159;
+// team 512, 4 per CU: 64 rows 476 -> 594, 128 286 -> 311, 200 214 -> 223, 256 185 -> 178; smaller teams gain
+// at any size.  (The systems' mean decides: the small ones are the many.)
+static bool resident_crowded(hala_batch B, int team, int wg) {
+    const int rows = team == 1024 ? 1024 : team == 512 ? 205 : 0;
+    return team * wg > 1024 && (int64_t)B->n_total < (int64_t)B->nsys * rows;
+}
+
 static bool launch_resident(hala_batch B, hipStream_t s, int team, int wg, const double *vals, const double *dvals,
                             const double *b, double *x, double rtol, int max_iter) {
+    if (resident_crowded(B, team, wg)) return false;
 #define HALA_RES(T, LEN, R1, R2) resident<T, LEN, R1, R2>(B, s, wg, vals, dvals, b, x, rtol, max_iter)
     if (B->max_row <= 5) switch (team) {
         case 64: return HALA_RES(64, 5, 4, 10);

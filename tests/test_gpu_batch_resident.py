@@ -72,3 +72,27 @@ def test_batch_resident_bitexact(engine, team, longest, past):
             it, x, _ = oracle.cg_team(sp, si, sv, d[r], b[r], tol, team, x0=x0[r], max_iter=cap)
             assert int(iters[s]) == it, (s, sizes[s])
             assert np.array_equal(bits(gx[r].cpu().numpy()), bits(x)), (s, sizes[s])
+
+
+@pytest.mark.parametrize("team,wg,n,path", [(512, 4, 204, 1), (512, 4, 205, 2), (512, 2, 60, 2), (1024, 2, 1023, 1),
+                                            (1024, 2, 1024, 2), (1024, 1, 40, 2), (256, 8, 20, 2)])
+def test_batch_crowded_shapes(engine, team, wg, n, path):
+    # more wavefronts per CU than the resident kernels' registers hold, on systems small for the team: the loop
+    rng = np.random.default_rng(team + n)
+    systems = [banded(n, 5, rng) for _ in range(3)]
+    nz = np.concatenate([[0], np.cumsum([len(s[1]) for s in systems])])
+    p = np.concatenate([s[0][:-1] + z for s, z in zip(systems, nz)] + [nz[-1:]])
+    i, v = np.concatenate([s[1] for s in systems]), np.concatenate([s[2] for s in systems])
+    d, b = rng.uniform(2.0, 9.0, 3 * n), rng.uniform(-1, 1, 3 * n)
+    i32 = lambda a: engine.load(np.ascontiguousarray(a, np.int32))
+    bs = H.batch_solver(engine, i32(np.arange(4) * n), i32(p), i32(i))
+    bs.set_shape(team, wg)
+    gx, iters = engine.vector(3 * n), torch.zeros(3, dtype=torch.int32, device="cuda")
+    bs.solve(engine.load(v), engine.load(d), engine.load(b), gx, rtol=1e-9, max_iter=100000, iters=iters)
+    assert engine.get_option("path_batch") == path
+    for s, (sp, si, sv) in enumerate(systems):
+        r = slice(s * n, (s + 1) * n)
+        tol = 1e-9 * np.sqrt(oracle.team_dot(b[r], b[r], team))
+        it, x, _ = oracle.cg_team(sp, si, sv, d[r], b[r], tol, team)
+        assert int(iters[s]) == it
+        assert np.array_equal(bits(gx[r].cpu().numpy()), bits(x))
