@@ -231,8 +231,8 @@ __global__ void set_int(int *p, int v) { *p = v; }
 static bool use_stencil(hala_ilu M) { return M->sp && M->ctx->opt.tri_stencil; }
 
 // both triangles on the grid sweeps, in one packed order
-static bool use_grid(hala_ilu M, bool is64) {
-    return !use_stencil(M) && grid_pair_usable(M->ctx, M->L, M->U, is64);
+static bool use_grid(hala_ilu M, bool is64, int nrhs = 1) {
+    return !use_stencil(M) && grid_pair_usable(M->ctx, M->L, M->U, is64, nrhs);
 }
 
 static bool use_columns(hala_ilu M) {
@@ -303,7 +303,7 @@ void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const in
     hala_ctx c = M->ctx;
     HALA_REQUIRE(M->factored, HALA_ERR_ARG, "ILU apply before factorisation");
     const int64_t n = M->n;
-    const bool grid = use_grid(M, true);
+    const bool grid = use_grid(M, true, nrhs);
     const int step = grid ? cols_at_once(M->L.grid.g.N, nrhs) : 1;
     for (int k = 0; k < nrhs; k += step) {
         const int m = std::min(step, nrhs - k);
@@ -313,7 +313,7 @@ void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const in
 }
 
 bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
-    if (!use_grid(M, true)) return false;
+    if (!use_grid(M, true, nrhs)) return false;
     N = M->L.grid.g.N;
     if (cols_at_once(N, nrhs) < nrhs) return false;
     grid_reserve(M->ctx, M->L, true, nrhs);
@@ -617,6 +617,7 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         col_set_handoff(c, M->L, M->U);
         // the grid sweeps' vectors come from the context's cache, as the rest of the factor
         for (tri_plan *p : {&M->L, &M->U}) {
+            if (p->grid.thin) continue;
             if (p->grid.ok) grid_reserve(c, *p, true, 1);
             if (p->grid.ok && want_f32) grid_reserve(c, *p, false, 1);
         }

@@ -231,7 +231,7 @@ template <class T>
 void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
     constexpr bool is64 = sizeof(T) == 8;
     constexpr int64_t ELEMS = 1ll << 28;  // elements of one packed copy at most
-    const bool grid = grid_usable(c, p, is64), col = !grid && col_usable(c, p, is64) && !p.col.upward;
+    const bool grid = grid_usable(c, p, is64, nrhs), col = !grid && col_usable(c, p, is64) && !p.col.upward;
     const int64_t per = grid ? p.grid.g.N : (int64_t)p.nchunk * WAVE + SLOT_PAD;
     const int at_once = (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, ELEMS / per, 4096}));
     if (grid || (col && at_once > 1)) {

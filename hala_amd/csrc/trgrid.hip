@@ -719,6 +719,12 @@ void build_grid_plan(hala_ctx c, tri_plan &p) {
     if (g.N > 3 * (int64_t)n && g.N > (1 << 20)) return;
     if (g.N > (1 << 28)) return;  // 32-bit byte offsets into a vector's frames
     q.g = g;
+    // A hop from tile to tile takes as long as about ten levels of a few rows of the column sweep (1.8 us
+    // against 0.19): 3-D grids of short lines, a hop every eight levels, run one vector there.  Applies, column
+    // -> grid: 8 x 8 x 4000 1538 -> 1823 us, 9 x 1000 x 9 425 -> 476, 2 x 2 x 2000 775 -> 846; wider levels
+    // take the column sweep longer: 3 x 100 x 100 127 -> 124, 5 x 200 x 200 238 -> 227, 12 x 200 x 200 334 -> 237.
+    // (Several vectors hide each other's hops.)
+    q.thin = dim == 3 && p.col.ok && (int64_t)(g.ntj + g.ntk - 2) * 10 > p.nlev && n < 128 * (int64_t)p.nlev;
     const gdims d = dims_of(p);
     int *flag = reinterpret_cast<int *>(c->scal.as<double>() + S_DOT + 9);
     HALA_HIP(hipMemsetAsync(flag, 0, sizeof(int), c->stream));
@@ -769,15 +775,16 @@ void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {
     }
 }
 
-bool grid_usable(hala_ctx c, const tri_plan &p, bool is64) {
+bool grid_usable(hala_ctx c, const tri_plan &p, bool is64, int nrhs) {
     const hala_options &o = c->opt;
     // the column options, where given, ask for the column sweeps
     if (!p.grid.ok || !o.tri_grid || !o.tri_col || o.tri_col_cols || o.tri_col_split) return false;
+    if (p.grid.thin && nrhs == 1) return false;
     return is64 ? p.grid.has64 : p.grid.has32;
 }
 
-bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64) {
-    return grid_usable(c, first, is64) && grid_usable(c, second, is64) && first.grid.g.same(second.grid.g) &&
+bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64, int nrhs) {
+    return grid_usable(c, first, is64, nrhs) && grid_usable(c, second, is64, nrhs) && first.grid.g.same(second.grid.g) &&
            first.backward != second.backward;
 }
 

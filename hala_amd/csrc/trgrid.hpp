@@ -33,6 +33,7 @@ struct grid_geom {
 // The grid side of a plan (member of tri_plan).
 struct tri_gridplan {
     bool ok = false;
+    bool thin = false;  // one vector runs faster on the column sweep (see build_grid_plan)
     bool zyx = true;  // a row's terms in the order k-1, j-1, i-1 (else i-1, j-1, k-1)
     grid_geom g;
     dbuf order;         // tile per ticket, in dependency order
@@ -50,10 +51,10 @@ struct tri_gridplan {
 void build_grid_plan(hala_ctx c, tri_plan &p);
 // The factor's values into the step records of one precision.
 void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
-// The plan runs on the grid sweep in this precision (pattern, values, options).
-bool grid_usable(hala_ctx c, const tri_plan &p, bool is64);
+// The plan runs nrhs vectors on the grid sweep in this precision (pattern, values, options).
+bool grid_usable(hala_ctx c, const tri_plan &p, bool is64, int nrhs = 1);
 // ... and so does second, in first's packed order (an ILU's two triangles).
-bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64);
+bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64, int nrhs = 1);
 // Packed vectors for nrhs right-hand sides.
 void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs);
 

@@ -112,6 +112,45 @@ def test_sweep_paths_bitexact(engine, name):
             assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply_t(p, i, dg, f, x)))
 
 
+THIN = {  # name: (matrix, path_sweep of one vector); complete grids, on the columns where a hop comes every few levels
+    "8x8x400": (lambda: st.laplace3d(8, 8, 400), 1),
+    "9x400x9": (lambda: st.laplace3d(9, 400, 9), 1),
+    "400x9x9": (lambda: st.laplace3d(400, 9, 9), 2),
+    "3x60x60": (lambda: st.laplace3d(3, 60, 60), 1),
+    "12x60x60": (lambda: st.laplace3d(12, 60, 60), 2),
+    "2x500": (lambda: st.laplace2d(2, 500), 2),
+}
+
+
+@pytest.mark.parametrize("name", sorted(THIN))
+def test_thin_grids(engine, name):
+    mat, path = THIN[name]
+    p, i, v = mat()
+    n = len(p) - 1
+    dg, _ = oracle.diag(p, i)
+    f = oracle.ilu0(p, i, v, dg)
+    gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+    M = H.make_ilu(engine, gp, gi, gv)
+    x = st.uniform(31, n)
+    gx, gr = engine.load(x), engine.vector(n)
+    for _ in range(2):
+        M.apply(gx, gr)
+        assert engine.get_option("path_sweep") == path
+        assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(p, i, dg, f, x)))
+        M.apply_t(gx, gr)
+        assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply_t(p, i, dg, f, x)))
+        # several vectors take the grid sweeps in every case
+        B = np.stack([st.uniform(40 + k, n) for k in range(3)])
+        X = torch.zeros(3, n, dtype=torch.float64, device="cuda")
+        H.solve_batch_cg_ilu(engine, H.stop_criteria(0.0, 6), gp, gi, gv, M, engine.load(B), X)
+        assert engine.get_option("path_sweep") == engine.get_option("path_pcg") == 2
+        gx1 = engine.vector(n)
+        H.solve_cg_ilu(engine, H.stop_criteria(0.0, 6), gp, gi, gv, M, engine.load(B[1]), gx1)
+        assert engine.get_option("path_pcg") == path
+        _, ref, _ = oracle.cg(p, i, v, B[1], tol=0.0, max_iter=6, prec=oracle.PREC_ILU, mpntr=p, mindx=i, mdiag=dg, mdata=f)
+        assert np.array_equal(bits(host(X[1])), bits(ref)) and np.array_equal(bits(host(gx1)), bits(ref))
+
+
 @pytest.mark.parametrize("prec", ["identity", "jacobi"])
 @pytest.mark.parametrize("side,opts,path", [(64, {"cg_small": 0}, 1), (65, {}, 1), (64, {}, 2), (520, {}, 0)])
 def test_cg_paths_bitexact(engine, prec, side, opts, path):
