@@ -231,12 +231,40 @@ __global__ void set_int(int *p, int v) { *p = v; }
 static bool use_stencil(hala_ilu M) { return M->sp && M->ctx->opt.tri_stencil; }
 
 // both triangles on the grid sweeps, in one packed order
-static bool use_grid(hala_ilu M, bool is64, int nrhs = 1) {
-    return !use_stencil(M) && grid_pair_usable(M->ctx, M->L, M->U, is64, nrhs);
+static bool use_grid(hala_ilu M, int nrhs = 1) {
+    return !use_stencil(M) && grid_pair_usable(M->ctx, M->L, M->U, nrhs);
 }
 
+// both triangles on the column sweeps, L handing its results to U in slot order
 static bool use_columns(hala_ilu M) {
-    return !use_stencil(M) && col_usable(M->ctx, M->L, true) && col_usable(M->ctx, M->U, true) && M->L.col.hand64;
+    return !use_stencil(M) && col_usable(M->ctx, M->L) && col_usable(M->ctx, M->U);
+}
+
+// The factor's values in a layout: packed by the factorisation for the sweeps that run by the options
+// of that time, here on another layout's first use.  A pack that a capture recorded has not run: every
+// later call packs again until one does so outside a capture.
+static void need(hala_ilu M, tri_plan &p, bool is64, tri_layout layout) {
+    int &loaded = is64 ? p.loaded64 : p.loaded32, &rec = is64 ? p.rec64 : p.rec32;
+    if ((loaded & layout) && !(rec & layout)) return;
+    hala_ctx c = M->ctx;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HALA_HIP(hipStreamIsCapturing(c->stream, &capture));
+    if (is64) load_values64(c, p, M->factor.as<double>(), layout);
+    else load_values32(c, p, M->factor.as<double>(), layout);
+    rec = capture != hipStreamCaptureStatusNone ? rec | layout : rec & ~layout;
+}
+static void need_pair(hala_ilu M, bool is64, tri_layout layout) {
+    need(M, M->L, is64, layout);
+    need(M, M->U, is64, layout);
+}
+static void need_columns(hala_ilu M) {
+    need_pair(M, true, LAYOUT_COLUMNS);
+    if (!M->L.col.hand64) col_set_handoff(M->ctx, M->L, M->U);
+}
+// each triangle by itself
+static void need_routes(hala_ilu M, bool is64) {
+    need(M, M->L, is64, tri_route(M->ctx, M->L));
+    need(M, M->U, is64, tri_route(M->ctx, M->U));
 }
 
 bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
@@ -244,7 +272,9 @@ bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
     if (!M->factored) return false;
     if (transposed) ilu_prepare_adjoint(M);
     tri_plan &first = transposed ? M->Ut : M->L, &second = transposed ? M->Lt : M->U;
-    if (transposed ? grid_pair_usable(c, first, second, true) : use_grid(M, true)) {
+    if (transposed ? grid_pair_usable(c, first, second) : use_grid(M)) {
+        need(M, first, true, LAYOUT_GRID);
+        need(M, second, true, LAYOUT_GRID);
         grid_reserve(c, first, true, 1);
         grid_reserve(c, second, true, 1);
         e = ilu_ends{first.grid.slot.as<int>(), first.grid.in64.as<double>(), first.grid.slot.as<int>(),
@@ -252,6 +282,7 @@ bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
         return true;
     }
     if (!transposed && use_columns(M)) {
+        need_columns(M);
         e = ilu_ends{first.slot_of_row.as<int>(), first.col.xs64.as<double>(), second.slot_of_row.as<int>(),
                      second.out64.as<double>(), true};
         return true;
@@ -265,7 +296,7 @@ void ilu_apply64_mid(hala_ilu M, bool transposed, const int *gate, const col_axp
         grid_pair_mid64(c, M->Ut, M->Lt, 1, gate);
         return;
     }
-    if (use_grid(M, true)) {
+    if (use_grid(M)) {
         grid_pair_mid64(c, M->L, M->U, 1, gate);
         return;
     }
@@ -281,16 +312,19 @@ void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate) {
         stencil_apply<double, double, double>(M, x, r, gate);
         return;
     }
-    if (use_grid(M, true)) {
+    if (use_grid(M)) {
+        need_pair(M, true, LAYOUT_GRID);
         grid_exec_pair<double, double>(c, M->L, M->U, x, 0, r, 0, 1, gate);
         return;
     }
     if (use_columns(M)) {  // L's output handed to U in slot order
+        need_columns(M);
         tri_col_exec<double, double>(c, M->L, TRI_SUB, 1.0, x, nullptr, gate, &M->U);
         col_sweep64(c, M->U, TRI_SUB, 1.0, gate, nullptr, &M->L);
         col_scatter64(c, M->U, r, gate);
         return;
     }
+    need_routes(M, true);
     tri_exec<double, double, double>(c, M->L, TRI_SUB, 1.0, x, M->tmp64.as<double>(), gate);
     tri_exec<double, double, double>(c, M->U, TRI_SUB, 1.0, M->tmp64.as<double>(), r, gate);
 }
@@ -303,7 +337,8 @@ void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const in
     hala_ctx c = M->ctx;
     HALA_REQUIRE(M->factored, HALA_ERR_ARG, "ILU apply before factorisation");
     const int64_t n = M->n;
-    const bool grid = use_grid(M, true, nrhs);
+    const bool grid = use_grid(M, nrhs);
+    if (grid) need_pair(M, true, LAYOUT_GRID);
     const int step = grid ? cols_at_once(M->L.grid.g.N, nrhs) : 1;
     for (int k = 0; k < nrhs; k += step) {
         const int m = std::min(step, nrhs - k);
@@ -313,7 +348,8 @@ void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const in
 }
 
 bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
-    if (!use_grid(M, true, nrhs)) return false;
+    if (!use_grid(M, nrhs)) return false;
+    need_pair(M, true, LAYOUT_GRID);
     N = M->L.grid.g.N;
     if (cols_at_once(N, nrhs) < nrhs) return false;
     grid_reserve(M->ctx, M->L, true, nrhs);
@@ -338,10 +374,12 @@ void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate) {
         stencil_apply<float, double, double>(M, x, r, gate);
         return;
     }
-    if (use_grid(M, false)) {
+    if (use_grid(M)) {
+        need_pair(M, false, LAYOUT_GRID);
         grid_exec_pair<float, double>(c, M->L, M->U, x, 0, r, 0, 1, gate);
         return;
     }
+    need_routes(M, false);
     tri_exec<float, double, double>(c, M->L, TRI_SUB, 1.0f, x, M->tmp64.as<double>(), gate);
     tri_exec<float, double, double>(c, M->U, TRI_SUB, 1.0f, M->tmp64.as<double>(), r, gate);
 }
@@ -358,18 +396,16 @@ void ilu_prepare_adjoint(hala_ilu M) {
         build_schedule(c, M->Lt, false);
         M->adjoint = true;
     }
-    if (!M->adjoint_loaded) {
-        load_values64(c, M->Ut, M->factor.as<double>());
-        load_values64(c, M->Lt, M->factor.as<double>());
-        M->adjoint_loaded = true;
-    }
+    const bool pair = grid_pair_usable(c, M->Ut, M->Lt);
+    need(M, M->Ut, true, pair ? LAYOUT_GRID : tri_route(c, M->Ut));
+    need(M, M->Lt, true, pair ? LAYOUT_GRID : tri_route(c, M->Lt));
 }
 
 void ilu_apply_t64(hala_ilu M, const double *x, double *r, const int *gate) {
     hala_ctx c = M->ctx;
     HALA_REQUIRE(M->factored, HALA_ERR_ARG, "ILU apply before factorisation");
     ilu_prepare_adjoint(M);
-    if (grid_pair_usable(c, M->Ut, M->Lt, true)) {
+    if (grid_pair_usable(c, M->Ut, M->Lt)) {
         grid_exec_pair<double, double>(c, M->Ut, M->Lt, x, 0, r, 0, 1, gate);
         return;
     }
@@ -580,7 +616,7 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         pivot_check<<<(M->n + 255) / 256, 256, 0, c->stream>>>(M->n, M->diag.as<int>(), f, bad);
         HALA_CHECK_LAUNCH();
         M->factored = false;
-        M->adjoint_loaded = false;
+        for (tri_plan *p : {&M->L, &M->U, &M->Lt, &M->Ut}) p->loaded64 = p->loaded32 = p->rec64 = p->rec32 = 0;
         M->jac_values = false;
         M->jac_values64 = false;
         // The values are packed without waiting for the host; the
@@ -589,7 +625,16 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         // stays unfactored).
         // the two triangles' values are packed side by side: U's on the
         // auxiliary context's stream, joined back before anything reads them
-        // (scattered gathers from the factor, mostly latency)
+        // (scattered gathers from the factor, mostly latency), in the layout
+        // that the options now choose (128^3: 1.78 ms, all three 2.24)
+        for (tri_plan *p : {&M->L, &M->U}) {
+            reserve_values(c, *p, false);
+            if (want_f32) reserve_values(c, *p, true);
+        }
+        const bool grid = use_grid(M), columns = !grid && use_columns(M);
+        auto layout = [&](const tri_plan &p) {
+            return grid ? LAYOUT_GRID : columns ? LAYOUT_COLUMNS : tri_route(c, p);
+        };
         hala_ctx a = aux_ctx(c);
         hipEvent_t ev[2] = {nullptr, nullptr};
         HALA_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
@@ -600,11 +645,11 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         try {
             HALA_HIP(hipEventRecord(ev[0], c->stream));
             HALA_HIP(hipStreamWaitEvent(a->stream, ev[0], 0));
-            load_values64(a, M->U, f);
-            if (want_f32) load_values32(a, M->U, f);
+            load_values64(a, M->U, f, layout(M->U));
+            if (want_f32) load_values32(a, M->U, f, layout(M->U));
             HALA_HIP(hipEventRecord(ev[1], a->stream));
-            load_values64(c, M->L, f);
-            if (want_f32) load_values32(c, M->L, f);
+            load_values64(c, M->L, f, layout(M->L));
+            if (want_f32) load_values32(c, M->L, f, layout(M->L));
             HALA_HIP(hipStreamWaitEvent(c->stream, ev[1], 0));
         } catch (...) {
             (void)hipStreamSynchronize(a->stream);
@@ -614,7 +659,7 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         }
         (void)hipEventDestroy(ev[0]);
         (void)hipEventDestroy(ev[1]);
-        col_set_handoff(c, M->L, M->U);
+        if (columns) col_set_handoff(c, M->L, M->U);
         // the grid sweeps' vectors come from the context's cache, as the rest of the factor
         for (tri_plan *p : {&M->L, &M->U}) {
             if (p->grid.thin) continue;
@@ -652,9 +697,11 @@ int hala_ilu_apply_f32(hala_ilu M, const float *x, float *r) {
         set_device(c);
         if (use_stencil(M)) {
             stencil_apply<float, float, float>(M, x, r, nullptr);
-        } else if (use_grid(M, false)) {
+        } else if (use_grid(M)) {
+            need_pair(M, false, LAYOUT_GRID);
             grid_exec_pair<float, float>(c, M->L, M->U, x, 0, r, 0, 1, nullptr);
         } else {
+            need_routes(M, false);
             M->tmp32.reserve((size_t)M->n * sizeof(float));
             tri_exec<float, float, float>(c, M->L, TRI_SUB, 1.0f, x, M->tmp32.as<float>());
             tri_exec<float, float, float>(c, M->U, TRI_SUB, 1.0f, M->tmp32.as<float>(), r);

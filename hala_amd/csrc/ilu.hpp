@@ -20,7 +20,7 @@ struct hala_ilu_s {
     hala_amd::tri_plan Ut, Lt; // adjoint: U^T forward, L^T backward (built on demand)
     hala_amd::csr_transpose tp;
     hala_amd::dbuf tmp64, tmp32;  // natural-order hand-off between the two solves
-    bool factored = false, has32 = false, adjoint = false, adjoint_loaded = false;
+    bool factored = false, has32 = false, adjoint = false;
     // Jacobi-applied factor (ilujac.hip): packed strict-L / strict-U parts with
     // FP32 (and, for FP64 applies, FP64) values and diagonal, four iterates of
     // each precision (built on first use)

@@ -615,6 +615,14 @@ bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req) {
     return false;
 }
 
+void col_reserve_values(tri_plan &p, bool f32) {
+    tri_colplan &q = p.col;
+    if (!q.ok) return;
+    const int npad = p.nchunk * WAVE + BTMAX;
+    (f32 ? q.val32 : q.val64).reserve((size_t)npad * rec_bytes(q.L, f32 ? sizeof(float) : sizeof(double)));
+    if (f32) q.xs32.reserve((size_t)npad * sizeof(float));
+}
+
 void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {
     tri_colplan &q = p.col;
     if (!q.ok) return;
@@ -622,14 +630,13 @@ void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {
     const int RB = rec_bytes(q.L, f32 ? sizeof(float) : sizeof(double));
     const int kcp = q.K * q.CP, xc = WAVE * q.EL;
     dbuf &dst = f32 ? q.val32 : q.val64;
-    dst.reserve((size_t)npad * RB);
+    col_reserve_values(p, f32);
     if (!f32) q.hand64 = false;  // rewritten below: hand-off slots gone
     const int g = (int)(((int64_t)npad * (RB / 16) + 255) / 256);  // a thread per 16-byte quad
     if (f32) {
         col_pack<float><<<g, 256, 0, c->stream>>>(nslots, npad, q.L, RB, kcp, xc, q.code.as<int>(), q.spar.as<int>(),
                                                  q.src.as<int>(),
                                                  p.dg_src.as<int>(), factor, dst.as<unsigned char>());
-        if (!q.xs32.p) q.xs32.reserve((size_t)npad * sizeof(float));
     } else {
         col_pack<double><<<g, 256, 0, c->stream>>>(nslots, npad, q.L, RB, kcp, xc, q.code.as<int>(), q.spar.as<int>(),
                                                   q.src.as<int>(),
@@ -1011,14 +1018,13 @@ void launch_col(hala_ctx c, tri_plan &p, col_args<T, TOUT> &a, size_t lds) {
 
 }  // namespace
 
-bool col_usable(hala_ctx c, const tri_plan &p, bool is64) {
+bool col_usable(hala_ctx c, const tri_plan &p) {
     const tri_colplan &q = p.col;
     if (!q.ok || !c->opt.tri_col) return false;
     if (q.CP > (q.L == 4 ? CPMAX : CPMAX_LONG)) return false;
     // the kernel addresses records, inputs and outputs by 32-bit byte offsets
     const int64_t npad = (int64_t)p.nchunk * WAVE + BTMAX;
-    if (npad * rec_bytes(q.L, sizeof(double)) > INT_MAX) return false;
-    return is64 ? (q.val64.p != nullptr) : (q.val32.p != nullptr);
+    return npad * rec_bytes(q.L, sizeof(double)) <= INT_MAX;
 }
 
 namespace {
@@ -1169,7 +1175,7 @@ __global__ void col_set_hand(int nslots, const int *__restrict__ chunk_row, cons
 void col_set_handoff(hala_ctx c, tri_plan &src, tri_plan &dst) {
     tri_colplan &q = src.col;
     q.hand64 = false;
-    if (!q.ok || !dst.col.ok || !src.unit || !q.val64.p || !dst.col.xs64.p) return;
+    if (!q.ok || !dst.col.ok || !src.unit || !(src.loaded64 & LAYOUT_COLUMNS) || !dst.col.xs64.p) return;
     const int nslots = src.nchunk * WAVE;
     col_set_hand<<<(nslots + 255) / 256, 256, 0, c->stream>>>(nslots, src.chunk_row.as<int>(),
                                                              dst.slot_of_row.as<int>(), dst.nchunk * WAVE,

@@ -179,16 +179,22 @@ __global__ __launch_bounds__(256) void tri_exec_kernel(tri_args<T, TIN, TOUT> a)
 }
 
 
+tri_layout tri_route(hala_ctx c, const tri_plan &p, int nrhs) {
+    return grid_usable(c, p, nrhs) ? LAYOUT_GRID : col_usable(c, p) ? LAYOUT_COLUMNS : LAYOUT_POOL;
+}
+
 template <class T, class TIN, class TOUT>
 void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *out_nat, const int *gate) {
     constexpr bool is64 = sizeof(T) == 8;
-    HALA_REQUIRE(is64 ? p.has64 : p.has32, HALA_ERR_ARG, "triangular solve: values not loaded for this precision");
+    const tri_layout route = tri_route(c, p);
+    HALA_REQUIRE((is64 ? p.loaded64 : p.loaded32) & route, HALA_ERR_ARG,
+                 "triangular solve: values not loaded for this precision");
     static_assert(std::is_same<TIN, TOUT>::value, "input and output share a type");
-    if (grid_usable(c, p, is64)) {
+    if (route == LAYOUT_GRID) {
         grid_exec<T, TIN>(c, p, mode, alpha, in, 0, out_nat, 0, 1, gate);
         return;
     }
-    if (col_usable(c, p, is64)) {  // (its gather pass re-arms the polled output)
+    if (route == LAYOUT_COLUMNS) {  // (its gather pass re-arms the polled output)
         tri_col_exec<T, TOUT>(c, p, mode, alpha, in, out_nat, gate);
         return;
     }
@@ -225,13 +231,16 @@ void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *o
     HALA_CHECK_LAUNCH();
 }
 
-// 64^3 lower triangle, 8 vectors: 155 us, of which the values' packing is 45;
-// one solve per vector took 926 us.
+// 64^3 lower triangle, 8 vectors: 105 us with the values' packing; one solve
+// per vector took 1050 us.
 template <class T>
 void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
     constexpr bool is64 = sizeof(T) == 8;
     constexpr int64_t ELEMS = 1ll << 28;  // elements of one packed copy at most
-    const bool grid = grid_usable(c, p, is64, nrhs), col = !grid && col_usable(c, p, is64) && !p.col.upward;
+    const tri_layout route = tri_route(c, p, nrhs);
+    HALA_REQUIRE((is64 ? p.loaded64 : p.loaded32) & route, HALA_ERR_ARG,
+                 "triangular solve: values not loaded for this precision");
+    const bool grid = route == LAYOUT_GRID, col = route == LAYOUT_COLUMNS && !p.col.upward;
     const int64_t per = grid ? p.grid.g.N : (int64_t)p.nchunk * WAVE + SLOT_PAD;
     const int at_once = (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, ELEMS / per, 4096}));
     if (grid || (col && at_once > 1)) {

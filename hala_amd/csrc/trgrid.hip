@@ -757,7 +757,6 @@ void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {
     const int nstep = (int)(q.g.N / WAVE), g = (nstep + 3) / 4;
     auto pack = [&](auto zero, dbuf &rec) {
         using V = decltype(zero);
-        rec.reserve(rec_values<V>(p) * sizeof(V));
         if (q.g.nz > 1)
             grid_pack<3, V><<<g, 256, 0, c->stream>>>(d, q.zyx, p.unit, nstep, p.dptr.as<int>(), p.dsrc.as<int>(),
                                                       p.diag_src.as<int>(), factor, rec.as<V>());
@@ -766,25 +765,26 @@ void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {
                                                       p.diag_src.as<int>(), factor, rec.as<V>());
         HALA_CHECK_LAUNCH();
     };
-    if (f32) {
-        pack(0.0f, q.rec32);
-        q.has32 = true;
-    } else {
-        pack(0.0, q.rec64);
-        q.has64 = true;
-    }
+    grid_reserve_values(p, f32);
+    if (f32) pack(0.0f, q.rec32);
+    else pack(0.0, q.rec64);
 }
 
-bool grid_usable(hala_ctx c, const tri_plan &p, bool is64, int nrhs) {
+void grid_reserve_values(tri_plan &p, bool f32) {
+    if (!p.grid.ok) return;
+    if (f32) p.grid.rec32.reserve(rec_values<float>(p) * sizeof(float));
+    else p.grid.rec64.reserve(rec_values<double>(p) * sizeof(double));
+}
+
+bool grid_usable(hala_ctx c, const tri_plan &p, int nrhs) {
     const hala_options &o = c->opt;
     // the column options, where given, ask for the column sweeps
     if (!p.grid.ok || !o.tri_grid || !o.tri_col || o.tri_col_cols || o.tri_col_split) return false;
-    if (p.grid.thin && nrhs == 1) return false;
-    return is64 ? p.grid.has64 : p.grid.has32;
+    return !(p.grid.thin && nrhs == 1);
 }
 
-bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64, int nrhs) {
-    return grid_usable(c, first, is64, nrhs) && grid_usable(c, second, is64, nrhs) && first.grid.g.same(second.grid.g) &&
+bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, int nrhs) {
+    return grid_usable(c, first, nrhs) && grid_usable(c, second, nrhs) && first.grid.g.same(second.grid.g) &&
            first.backward != second.backward;
 }
 

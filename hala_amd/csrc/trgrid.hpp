@@ -39,7 +39,6 @@ struct tri_gridplan {
     dbuf order;         // tile per ticket, in dependency order
     dbuf slot;          // packed element (forward order) of every natural row
     dbuf rec64, rec32;  // per (tile, step) the step's coefficients and diagonal (see grid_pack)
-    bool has64 = false, has32 = false;
     // packed input, output and frames (boundary results the tiles poll; sentinels
     // before a sweep) of `rhs64` / `rhs32` vectors, made on first use
     dbuf in64, in32, out64, out32, fr64, fr32;
@@ -51,10 +50,11 @@ struct tri_gridplan {
 void build_grid_plan(hala_ctx c, tri_plan &p);
 // The factor's values into the step records of one precision.
 void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
-// The plan runs nrhs vectors on the grid sweep in this precision (pattern, values, options).
-bool grid_usable(hala_ctx c, const tri_plan &p, bool is64, int nrhs = 1);
+void grid_reserve_values(tri_plan &p, bool f32);
+// The plan runs nrhs vectors on the grid sweep (pattern, options).
+bool grid_usable(hala_ctx c, const tri_plan &p, int nrhs = 1);
 // ... and so does second, in first's packed order (an ILU's two triangles).
-bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, bool is64, int nrhs = 1);
+bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, int nrhs = 1);
 // Packed vectors for nrhs right-hand sides.
 void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs);
 

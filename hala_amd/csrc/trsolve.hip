@@ -432,10 +432,15 @@ __global__ void gather_vals(int64_t nent, const int *__restrict__ src, const dou
 }
 
 template <class T>
-static void load_values(hala_ctx c, tri_plan &p, const double *factor, dbuf &ent, dbuf &dg) {
-    int64_t nslots = (int64_t)p.nchunk * WAVE;
+static void reserve_pool(tri_plan &p, dbuf &ent, dbuf &dg) {
     ent.reserve((size_t)(p.nent > 0 ? p.nent : 1) * sizeof(T));
-    dg.reserve((size_t)(nslots + SLOT_PAD) * sizeof(T));
+    dg.reserve((size_t)((int64_t)p.nchunk * WAVE + SLOT_PAD) * sizeof(T));
+}
+
+template <class T>
+static void load_pool(hala_ctx c, tri_plan &p, const double *factor, dbuf &ent, dbuf &dg) {
+    int64_t nslots = (int64_t)p.nchunk * WAVE;
+    reserve_pool<T>(p, ent, dg);
     if (p.nent > 0) {
         gather_vals<T><<<(int)((p.nent + 255) / 256), 256, 0, c->stream>>>(p.nent, p.ent_src.as<int>(), factor,
                                                                           ent.as<T>());
@@ -446,21 +451,32 @@ static void load_values(hala_ctx c, tri_plan &p, const double *factor, dbuf &ent
     HALA_CHECK_LAUNCH();
 }
 
-void load_values64(hala_ctx c, tri_plan &p, const double *factor) {
-    load_values<double>(c, p, factor, p.ent_val64, p.dg_val64);
-    col_load_values(c, p, factor, false);
-    grid_load_values(c, p, factor, false);
-    p.has64 = true;
-}
-void load_values32(hala_ctx c, tri_plan &p, const double *factor) {
-    load_values<float>(c, p, factor, p.ent_val32, p.dg_val32);
-    col_load_values(c, p, factor, true);
-    grid_load_values(c, p, factor, true);
-    if (!p.out32.p) {
+void reserve_values(hala_ctx c, tri_plan &p, bool f32) {
+    if (f32) reserve_pool<float>(p, p.ent_val32, p.dg_val32);
+    else reserve_pool<double>(p, p.ent_val64, p.dg_val64);
+    col_reserve_values(p, f32);
+    grid_reserve_values(p, f32);
+    if (f32 && !p.out32.p) {
         p.out32.reserve((size_t)p.nchunk * WAVE * sizeof(float));
         tri_rearm(c, p);
     }
-    p.has32 = true;
+}
+
+void load_values64(hala_ctx c, tri_plan &p, const double *factor, tri_layout layout) {
+    if (layout == LAYOUT_POOL) load_pool<double>(c, p, factor, p.ent_val64, p.dg_val64);
+    else if (layout == LAYOUT_COLUMNS) col_load_values(c, p, factor, false);
+    else grid_load_values(c, p, factor, false);
+    p.loaded64 |= layout;
+}
+void load_values32(hala_ctx c, tri_plan &p, const double *factor, tri_layout layout) {
+    if (layout == LAYOUT_POOL) load_pool<float>(c, p, factor, p.ent_val32, p.dg_val32);
+    else if (layout == LAYOUT_COLUMNS) col_load_values(c, p, factor, true);
+    else grid_load_values(c, p, factor, true);
+    if (layout != LAYOUT_GRID && !p.out32.p) {
+        p.out32.reserve((size_t)p.nchunk * WAVE * sizeof(float));
+        tri_rearm(c, p);
+    }
+    p.loaded32 |= layout;
 }
 
 }  // namespace hala_amd

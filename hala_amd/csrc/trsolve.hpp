@@ -75,7 +75,8 @@ struct tri_plan {
     dbuf ent_dep, ent_src, dg_src;
     // values
     dbuf ent_val64, ent_val32, dg_val64, dg_val32;
-    bool has64 = false, has32 = false;
+    int loaded64 = 0, loaded32 = 0;  // layouts (tri_layout bits) that hold the present values,
+    int rec64 = 0, rec32 = 0;        // ... of them those whose pack a stream capture recorded (it runs on replay only)
     // polled outputs in slot order (re-armed to sentinels at the start of every sweep)
     dbuf out64, out32;
     tri_colplan col;
@@ -125,8 +126,15 @@ void sort_level_keys(hala_ctx c, const tri_plan &p, const int *key, int nkey, in
 void apply_level_order(hala_ctx c, tri_plan &p, const int *order);
 
 // Gathers plan values from a factor value array (positions ent_src / diag_src).
-void load_values64(hala_ctx c, tri_plan &p, const double *factor);
-void load_values32(hala_ctx c, tri_plan &p, const double *factor);
+// The values (of a new factor: clear loaded64 / loaded32 first) into one of the layouts: each costs a
+// scattered pass over the factor, and a sweep reads one of them.
+enum tri_layout : int { LAYOUT_POOL = 1, LAYOUT_COLUMNS = 2, LAYOUT_GRID = 4 };
+void load_values64(hala_ctx c, tri_plan &p, const double *factor, tri_layout layout);
+void load_values32(hala_ctx c, tri_plan &p, const double *factor, tri_layout layout);
+// The value buffers of every layout the plan has, so that loading one later allocates nothing.
+void reserve_values(hala_ctx c, tri_plan &p, bool f32);
+// The layout on which tri_exec (nrhs 1) and tri_exec_cols run the plan, by its patterns and the options.
+tri_layout tri_route(hala_ctx c, const tri_plan &p, int nrhs = 1);
 
 // Solves with plan p.  in: natural-order input (TIN), out_nat: natural-order
 // output (TOUT).  The plan's polled output of this precision is re-armed first,
@@ -149,7 +157,8 @@ bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req);
 template <class T>
 void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs);
 void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
-bool col_usable(hala_ctx c, const tri_plan &p, bool is64);
+void col_reserve_values(tri_plan &p, bool f32);
+bool col_usable(hala_ctx c, const tri_plan &p);  // pattern and options
 // next (nullable; FP64, TRI_SUB, unit p with hand-off slots, see
 // col_set_handoff): the sweep also writes next's input in next's slot order,
 // and its helper workgroups re-arm next's polled output.

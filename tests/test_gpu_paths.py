@@ -176,3 +176,77 @@ def test_path_names_are_read_only(engine):
         engine.set_option("path_cg", 1)
     with pytest.raises(H.HalaError, match="unknown option"):
         engine.get_option("path_none")
+
+
+def test_layouts_follow_options_and_factorisations(engine):
+    # the factor's values are packed for the sweeps that run: every other layout on its first use, and
+    # none of them survives a new factorisation (FP32 ones too, where it asked for FP64 only)
+    p, i, v = st.laplace3d(13, 12, 11)
+    n = len(p) - 1
+    dg, _ = oracle.diag(p, i)
+    w = v * np.where(i == np.repeat(np.arange(n), np.diff(p)), 1.25, 1.0)
+    x = st.uniform(9, n)
+    M = H.make_ilu(engine, engine.load(p), engine.load(i), engine.load(v), want_f32=True)
+    gx, gr = engine.load(x), engine.vector(n)
+
+    def check(vals, path):
+        f = oracle.ilu0(p, i, vals, dg)
+        M.apply(gx, gr)
+        assert engine.get_option("path_sweep") == path
+        assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(p, i, dg, f, x)))
+        M.apply_f32x64(gx, gr)
+        ref = oracle.ilu_apply_f32(p, i, dg, f.astype(np.float32), x.astype(np.float32)).astype(np.float64)
+        assert np.array_equal(bits(host(gr)), bits(ref))
+        M.apply_t(gx, gr)
+        assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply_t(p, i, dg, f, x)))
+        gs = engine.vector(n)
+        H.solve_cg_ilu(engine, H.stop_criteria(0.0, 5), M.pntr, M.indx, engine.load(vals), M, gx, gs)
+        _, ref, _ = oracle.cg(p, i, vals, x, tol=0.0, max_iter=5, prec=oracle.PREC_ILU, mpntr=p, mindx=i, mdiag=dg, mdata=f)
+        assert np.array_equal(bits(host(gs)), bits(ref))
+
+    ways = [({}, 2), ({"tri_grid": 0}, 1), ({"tri_col": 0}, 0), ({}, 2), ({"tri_col_cols": 4}, 1)]
+    for opts, path in ways:
+        with options(engine, **opts):
+            check(v, path)
+    for first, _ in ways[:3]:
+        with options(engine, **first):
+            M.factor(engine.load(w))  # FP64 only
+        for opts, path in ways:
+            with options(engine, **opts):
+                check(w, path)
+        with options(engine, **first):
+            M.factor(engine.load(v), want_f32=True)
+        for opts, path in ways:
+            with options(engine, **opts):
+                check(v, path)
+
+
+def test_layout_first_used_under_capture():
+    # a pack that a capture recorded has not run: the next eager call packs again, and replays give the same bits
+    p, i, v = st.laplace3d(13, 12, 11)
+    n = len(p) - 1
+    dg, _ = oracle.diag(p, i)
+    f = oracle.ilu0(p, i, v, dg)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        eng = H.gpu_engine(0, stream=s)
+        eng.set_option("sync_checks", 0)
+        M = H.make_ilu(eng, eng.load(p), eng.load(i), eng.load(v))
+        gx, gr, ge = eng.load(st.uniform(1, n)), eng.vector(n), eng.vector(n)
+        M.apply(gx, ge)  # the grid sweeps
+        eng.set_option("tri_grid", 0)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            M.apply(gx, gr)
+        for seed in (1, 2, 3):
+            x = st.uniform(seed, n)
+            ref = bits(oracle.ilu_apply(p, i, dg, f, x))
+            gx.copy_(eng.load(x))
+            M.apply(gx, ge)
+            assert eng.get_option("path_sweep") == 1
+            assert np.array_equal(bits(host(ge)), ref)
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(bits(host(gr)), ref)
+            eng.synchronize()
