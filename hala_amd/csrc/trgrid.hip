@@ -14,8 +14,8 @@
 // of the same length: 272 us on 128^3 when the lag of one took 241).
 #include <algorithm>
 #include <climits>
-#include <numeric>
 
+#include "tile_order.hpp"
 #include "trsolve.hpp"
 
 namespace hala_amd {
@@ -75,14 +75,19 @@ struct gdims {
 __device__ __forceinline__ int padded(int m, int t) { return (m + t - 1) / t * t; }
 
 // flag bit 0 / 1: some row's dependencies are not its in-grid neighbours in
-// the order k, j, i / i, j, k
+// the order k, j, i / i, j, k.  The packed element (forward order) of every
+// natural row, and behind them the tile of every ticket.
 __global__ __launch_bounds__(256) void grid_check(gdims d, int n, const int *__restrict__ dptr,
-                                                  const int *__restrict__ ddep, int *__restrict__ flag) {
+                                                  const int *__restrict__ ddep, int *__restrict__ flag,
+                                                  int *__restrict__ slot) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < d.ntj * d.ntk) slot[n + tile_ticket(r % d.ntj, r / d.ntj, d.ntj, d.ntk)] = r;
     unsigned bad = 0;
     if (r < n) {
         const int P = d.nx * d.ny;
         const int i = r % d.nx, j = (r / d.nx) % d.ny, k = r / P;
+        const int ta = j % d.TJ, tb = k % d.TK;
+        slot[r] = (((k / d.TK) * d.ntj + j / d.TJ) * d.S + i + ta + tb) * WAVE + lane_of(d.nz > 1 ? 3 : 2, ta, tb);
         const int s = d.backward ? 1 : -1;
         const bool hx = d.backward ? i < d.nx - 1 : i > 0;
         const bool hy = d.backward ? j < d.ny - 1 : j > 0;
@@ -104,15 +109,6 @@ __global__ __launch_bounds__(256) void grid_check(gdims d, int n, const int *__r
     // at most one atomic per wavefront and bit, none once the flag holds it
     const unsigned w = (__any(bad & 1) ? 1u : 0u) | (__any(bad & 2) ? 2u : 0u);
     if ((threadIdx.x & (WAVE - 1)) == 0 && w && (w & ~(unsigned)ld_agent(flag))) atomicOr(flag, (int)w);
-}
-
-// packed element (forward order) of every natural row
-__global__ void grid_slots(gdims d, int n, int *__restrict__ slot) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    const int i = r % d.nx, j = (r / d.nx) % d.ny, k = r / (d.nx * d.ny);
-    const int tile = (k / d.TK) * d.ntj + j / d.TJ, a = j % d.TJ, b = k % d.TK;
-    slot[r] = ((tile * d.S) + i + a + b) * WAVE + lane_of(d.nz > 1 ? 3 : 2, a, b);
 }
 
 // Step records, processing order: per (tile, step) the terms' coefficients as
@@ -648,7 +644,7 @@ void sweep(hala_ctx c, const tri_plan &p, int mode, V alpha, const V *in, V *out
     a.klo = p.backward ? g.ntk * TK - g.nz : 0;
     a.khi = p.backward ? g.ntk * TK : g.nz;
     a.N = g.N;
-    a.order = q.order.as<int>();
+    a.order = q.slot.as<int>() + p.n;
     a.rec = sizeof(V) == 8 ? reinterpret_cast<const V *>(q.rec64.p) : reinterpret_cast<const V *>(q.rec32.p);
     a.in = in;
     a.out = out;
@@ -680,34 +676,53 @@ V *buf(const dbuf &b64, const dbuf &b32) {
 
 }  // namespace
 
-void build_grid_plan(hala_ctx c, tri_plan &p) {
-    tri_gridplan &q = p.grid;
-    q.ok = false;
-    const int n = p.n;
-    if (n < 4) return;
+// What grid_probe reads back: dependency count of the row swept last, their distances, a word of the
+// caller's; then the check's flag (host side: at PROBE_HOST doubles into the landing zone, past what other
+// read-backs use).
+constexpr int PROBE_WORDS = 5, PROBE_HOST = 1000;
+static int *probe_dev(hala_ctx c) { return reinterpret_cast<int *>(c->scal.as<double>() + S_DOT + 10); }
+
+static __global__ void grid_probe_kernel(int corner, const int *__restrict__ dptr, const int *__restrict__ ddep,
+                                         const int *__restrict__ word, int *__restrict__ out) {
+    const int a = dptr[corner], m = dptr[corner + 1] - a;
+    out[0] = m;
+    for (int k = 0; k < 3; k++) out[1 + k] = k < m ? abs(ddep[a + k] - corner) : 0;
+    out[4] = *word;
+    out[PROBE_WORDS] = 0;
+}
+
+int grid_probe(hala_ctx c, tri_plan &p, const int *word) {
+    p.grid.ok = false;
     // the last row swept has every neighbour: its offsets are 1, nx (and nx ny)
-    const int corner = p.backward ? 0 : n - 1;
-    int h[2];
-    HALA_HIP(hipMemcpyAsync(c->host_pinned, p.dptr.as<int>() + corner, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-    HALA_HIP(hipStreamSynchronize(c->stream));
-    std::memcpy(h, c->host_pinned, sizeof(h));
-    const int m = h[1] - h[0];
-    if (m != 2 && m != 3) return;
-    int o[3];
-    HALA_HIP(hipMemcpyAsync(c->host_pinned, p.ddep.as<int>() + h[0], m * sizeof(int), hipMemcpyDeviceToHost,
+    grid_probe_kernel<<<1, 1, 0, c->stream>>>(p.backward ? 0 : p.n - 1, p.dptr.as<int>(), p.ddep.as<int>(), word,
+                                                probe_dev(c));
+    HALA_CHECK_LAUNCH();
+    HALA_HIP(hipMemcpyAsync(c->host_pinned + PROBE_HOST, probe_dev(c), PROBE_WORDS * sizeof(int), hipMemcpyDeviceToHost,
                             c->stream));
     HALA_HIP(hipStreamSynchronize(c->stream));
-    std::memcpy(o, c->host_pinned, m * sizeof(int));
-    for (int k = 0; k < m; k++) o[k] = std::abs(o[k] - corner);
+    int v;
+    std::memcpy(&v, reinterpret_cast<const int *>(c->host_pinned + PROBE_HOST) + 4, sizeof(int));
+    return v;
+}
+
+bool grid_layout(hala_ctx c, tri_plan &p) {
+    tri_gridplan &q = p.grid;
+    const int n = p.n;
+    if (n < 4) return false;
+    int h[PROBE_WORDS];
+    std::memcpy(h, c->host_pinned + PROBE_HOST, sizeof(h));
+    const int m = h[0];
+    if (m != 2 && m != 3) return false;
+    int *o = h + 1;  // m of them
     std::sort(o, o + m);
     grid_geom g;
-    if (o[0] != 1 || o[1] < 2) return;
+    if (o[0] != 1 || o[1] < 2) return false;
     g.nx = o[1];
     const int P = m == 3 ? o[2] : n;
-    if (P % g.nx != 0 || n % P != 0) return;
+    if (P % g.nx != 0 || n % P != 0) return false;
     g.ny = P / g.nx;
     g.nz = n / P;
-    if (g.ny < 2 || (m == 3 && g.nz < 2)) return;
+    if (g.ny < 2 || (m == 3 && g.nz < 2)) return false;
     const int dim = m, TJ = dim == 3 ? 8 : 64, TK = dim == 3 ? 8 : 1;
     g.ntj = (g.ny + TJ - 1) / TJ;
     g.ntk = (g.nz + TK - 1) / TK;
@@ -716,8 +731,8 @@ void build_grid_plan(hala_ctx c, tri_plan &p) {
     // tiles of short lines or few lanes are mostly padding: streaming it would
     // cost more than the general sweeps' level steps (small systems keep it:
     // they live in the caches)
-    if (g.N > 3 * (int64_t)n && g.N > (1 << 20)) return;
-    if (g.N > (1 << 28)) return;  // 32-bit byte offsets into a vector's frames
+    if (g.N > 3 * (int64_t)n && g.N > (1 << 20)) return false;
+    if (g.N > (1 << 28)) return false;  // 32-bit byte offsets into a vector's frames
     q.g = g;
     // A hop from tile to tile takes as long as about ten levels of a few rows of the column sweep (1.8 us
     // against 0.19): 3-D grids of short lines, a hop every eight levels, run one vector there.  Applies, column
@@ -726,28 +741,26 @@ void build_grid_plan(hala_ctx c, tri_plan &p) {
     // (Several vectors hide each other's hops.)
     q.thin = dim == 3 && p.col.ok && (int64_t)(g.ntj + g.ntk - 2) * 10 > p.nlev && n < 128 * (int64_t)p.nlev;
     const gdims d = dims_of(p);
-    int *flag = reinterpret_cast<int *>(c->scal.as<double>() + S_DOT + 9);
-    HALA_HIP(hipMemsetAsync(flag, 0, sizeof(int), c->stream));
-    grid_check<<<(n + 255) / 256, 256, 0, c->stream>>>(d, n, p.dptr.as<int>(), p.ddep.as<int>(), flag);
-    HALA_CHECK_LAUNCH();
-    const int bad = fetch_i32(c, flag);
-    // forward plans list a row's terms by ascending column (k-1, j-1, i-1); backward ones either way
-    if (bad == 3 || (!p.backward && (bad & 1))) return;
-    q.zyx = (bad & 1) == 0;
-    // tickets by first step
+    int *flag = probe_dev(c) + PROBE_WORDS;
     const int nt = g.ntj * g.ntk;
-    std::vector<int> order(nt);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        return x % g.ntj + x / g.ntj < y % g.ntj + y / g.ntj;
-    });
-    q.order.reserve((size_t)nt * sizeof(int));
-    HALA_HIP(hipMemcpyAsync(q.order.p, order.data(), (size_t)nt * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    q.slot.reserve((size_t)n * sizeof(int));
-    grid_slots<<<(n + 255) / 256, 256, 0, c->stream>>>(d, n, q.slot.as<int>());
+    q.slot.reserve(((size_t)n + nt) * sizeof(int));
+    grid_check<<<(std::max(n, nt) + 255) / 256, 256, 0, c->stream>>>(d, n, p.dptr.as<int>(), p.ddep.as<int>(), flag,
+                                                                     q.slot.as<int>());
     HALA_CHECK_LAUNCH();
-    HALA_HIP(hipStreamSynchronize(c->stream));
-    q.ok = true;
+    HALA_HIP(hipMemcpyAsync(c->host_pinned + PROBE_HOST, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    return true;
+}
+
+void grid_finish(hala_ctx c, tri_plan &p) {
+    int bad;
+    std::memcpy(&bad, c->host_pinned + PROBE_HOST, sizeof(int));
+    // forward plans list a row's terms by ascending column (k-1, j-1, i-1); backward ones either way
+    if (bad == 3 || (!p.backward && (bad & 1))) {
+        p.grid.slot.release();
+        return;
+    }
+    p.grid.zyx = (bad & 1) == 0;
+    p.grid.ok = true;
 }
 
 void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32) {

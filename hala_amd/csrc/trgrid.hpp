@@ -33,11 +33,10 @@ struct grid_geom {
 // The grid side of a plan (member of tri_plan).
 struct tri_gridplan {
     bool ok = false;
-    bool thin = false;  // one vector runs faster on the column sweep (see build_grid_plan)
+    bool thin = false;  // one vector runs faster on the column sweep (see grid_layout)
     bool zyx = true;  // a row's terms in the order k-1, j-1, i-1 (else i-1, j-1, k-1)
     grid_geom g;
-    dbuf order;         // tile per ticket, in dependency order
-    dbuf slot;          // packed element (forward order) of every natural row
+    dbuf slot;          // packed element (forward order) of every natural row, then the tile of every ticket
     dbuf rec64, rec32;  // per (tile, step) the step's coefficients and diagonal (see grid_pack)
     // packed input, output and frames (boundary results the tiles poll; sentinels
     // before a sweep) of `rhs64` / `rhs32` vectors, made on first use
@@ -45,9 +44,13 @@ struct tri_gridplan {
     int rhs64 = 0, rhs32 = 0;
 };
 
-// Recognises p's pattern from its dependency lists and lays the grid plan out
-// (p.grid.ok tells).  Reads a few integers back (synchronises).
-void build_grid_plan(hala_ctx c, tri_plan &p);
+// Recognises p's pattern from its dependency lists and lays the grid plan out (p.grid.ok tells), in three
+// steps that ride on the analysis's own synchronisations (four of their own cost 55 us per triangle):
+// grid_probe, which also returns the device word the analysis waits for there; grid_layout (false: no grid),
+// launches only; after the next synchronisation grid_finish.
+int grid_probe(hala_ctx c, tri_plan &p, const int *word);
+bool grid_layout(hala_ctx c, tri_plan &p);
+void grid_finish(hala_ctx c, tri_plan &p);
 // The factor's values into the step records of one precision.
 void grid_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);
 void grid_reserve_values(tri_plan &p, bool f32);

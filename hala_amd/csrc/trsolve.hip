@@ -379,17 +379,18 @@ void build_schedule(hala_ctx c, tri_plan &p, bool want32, bool have_levels) {
     level_chunks<<<(p.nlev + 255) / 256, 256, 0, c->stream>>>(p.nlev, p.level_ptr.as<int>(), nch.as<int>());
     HALA_CHECK_LAUNCH();
     exclusive_scan_i32(c, nch.as<int>(), chunk_ptr.as<int>(), p.nlev);
-    p.nchunk = fetch_i32(c, chunk_ptr.as<int>() + p.nlev);
+    p.nchunk = grid_probe(c, p, chunk_ptr.as<int>() + p.nlev);
     const int nslots = p.nchunk * WAVE;
     // the column layout lays the slots out in its own order; else (or when it
     // gave up before) the level order does
     if (c->opt.tri_col) build_col_plan(c, p, c->opt.tri_col_cols);
-    build_grid_plan(c, p);
+    const bool grid = grid_layout(c, p);
     if (!p.laid_out) lay_out_slots(c, p, p.perm.as<int>());
     p.out64.reserve((size_t)nslots * sizeof(double));
     if (want32) p.out32.reserve((size_t)nslots * sizeof(float));
     tri_rearm(c, p);
     HALA_HIP(hipStreamSynchronize(c->stream));
+    if (grid) grid_finish(c, p);
 }
 
 void sort_perm(hala_ctx c, tri_plan &p) {

@@ -30,6 +30,17 @@ def test_gather_limits(tmp_path):
     assert r.returncode == 0 and not bad, (bad, r.stderr)
 
 
+def test_tile_tickets(tmp_path):
+    # the grid sweeps' tiles, in an order in which a tile only waits for earlier tickets
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    exe = tmp_path / "tile_order"
+    src = os.path.join(ROOT, "tests", "cpp", "tile_order.cpp")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", src, "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
 def test_offset_products_choose_the_width():
     # whoever instantiates the offset gathers with 32 bits also asks gather_wide
     users = [f for f in os.listdir(CSRC) if f.endswith(".hip") and "csr_block_rowsums<" in open(os.path.join(CSRC, f)).read()]
