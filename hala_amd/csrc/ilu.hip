@@ -275,8 +275,7 @@ bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
     if (transposed ? grid_pair_usable(c, first, second) : use_grid(M)) {
         need(M, first, true, LAYOUT_GRID);
         need(M, second, true, LAYOUT_GRID);
-        grid_reserve(c, first, true, 1);
-        grid_reserve(c, second, true, 1);
+        grid_reserve_pair(c, first, second, true, 1);
         e = ilu_ends{first.grid.slot.as<int>(), first.grid.in64.as<double>(), first.grid.slot.as<int>(),
                      second.grid.out64.as<double>(), false};
         return true;
@@ -352,8 +351,7 @@ bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
     need_pair(M, true, LAYOUT_GRID);
     N = M->L.grid.g.N;
     if (cols_at_once(N, nrhs) < nrhs) return false;
-    grid_reserve(M->ctx, M->L, true, nrhs);
-    grid_reserve(M->ctx, M->U, true, nrhs);
+    grid_reserve_pair(M->ctx, M->L, M->U, true, nrhs);
     e = ilu_ends{M->L.grid.slot.as<int>(), M->L.grid.in64.as<double>(), M->L.grid.slot.as<int>(),
                  M->U.grid.out64.as<double>(), false};
     return true;
@@ -661,10 +659,9 @@ int hala_ilu_factor_f64(hala_ilu M, const double *vals, int want_f32) {
         (void)hipEventDestroy(ev[1]);
         if (columns) col_set_handoff(c, M->L, M->U);
         // the grid sweeps' vectors come from the context's cache, as the rest of the factor
-        for (tri_plan *p : {&M->L, &M->U}) {
-            if (p->grid.thin) continue;
-            if (p->grid.ok) grid_reserve(c, *p, true, 1);
-            if (p->grid.ok && want_f32) grid_reserve(c, *p, false, 1);
+        if (M->L.grid.ok && M->U.grid.ok && !M->L.grid.thin) {
+            grid_reserve_pair(c, M->L, M->U, true, 1);
+            if (want_f32) grid_reserve_pair(c, M->L, M->U, false, 1);
         }
         if (M->sp) stencil_load(M, want_f32);
         check_wait_error(c);  // synchronises; a dependency wait that gave up throws here

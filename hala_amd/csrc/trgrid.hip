@@ -801,27 +801,25 @@ bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second,
            first.backward != second.backward;
 }
 
-void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs) {
+void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs, grid_role role) {
     tri_gridplan &q = p.grid;
     int &have = is64 ? q.rhs64 : q.rhs32;
-    if (nrhs <= have) return;
+    dbuf &in = is64 ? q.in64 : q.in32, &out = is64 ? q.out64 : q.out32, &fr = is64 ? q.fr64 : q.fr32;
+    const size_t w = is64 ? sizeof(double) : sizeof(float);
+    // a sweep re-arms its partner's frames, alone a spare set of its own; a pair's second reads the first's output
+    const size_t e = (size_t)q.g.N * w, f = (size_t)frame_values(q.g) * (role == GRID_ALONE ? 2 : 1) * w;
+    const bool with_in = role != GRID_SECOND;
+    if (nrhs <= have && (!with_in || in.bytes >= e * nrhs) && fr.bytes >= f * nrhs) return;
     if (have) HALA_HIP(hipStreamSynchronize(c->stream));  // sweeps in flight still use the smaller buffers
-    const int64_t e = q.g.N * nrhs, f = frame_values(q.g) * nrhs;
-    const int g = grid_for(2 * f, 256 * 4, 8192);
+    nrhs = std::max(nrhs, have);
     have = 0;
-    // two frame buffers: a sweep uses the first and re-arms its partner's (a
-    // single sweep's own spare one)
-    if (is64) {
-        q.in64.reserve((size_t)e * sizeof(double));
-        q.out64.reserve((size_t)e * sizeof(double));
-        q.fr64.reserve((size_t)(2 * f) * sizeof(double));
-        grid_arm<double><<<g, 256, 0, c->stream>>>(q.fr64.as<double>(), 2 * f);
-    } else {
-        q.in32.reserve((size_t)e * sizeof(float));
-        q.out32.reserve((size_t)e * sizeof(float));
-        q.fr32.reserve((size_t)(2 * f) * sizeof(float));
-        grid_arm<float><<<g, 256, 0, c->stream>>>(q.fr32.as<float>(), 2 * f);
-    }
+    if (with_in) in.reserve(e * nrhs);
+    out.reserve(e * nrhs);
+    fr.reserve(f * nrhs);
+    const int64_t nf = (int64_t)(fr.bytes / w);  // all of it: what is there of earlier sweeps counts as unarmed
+    const int g = grid_for(nf, 256 * 4, 8192);
+    if (is64) grid_arm<double><<<g, 256, 0, c->stream>>>(fr.as<double>(), nf);
+    else grid_arm<float><<<g, 256, 0, c->stream>>>(fr.as<float>(), nf);
     HALA_CHECK_LAUNCH();
     have = nrhs;
 }
@@ -830,7 +828,7 @@ template <class T, class TIO>
 void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_t ldin, TIO *out, int64_t ldout,
                int nrhs, const int *gate, int64_t inc) {
     tri_gridplan &q = p.grid;
-    grid_reserve(c, p, sizeof(T) == 8, nrhs);
+    grid_reserve(c, p, sizeof(T) == 8, nrhs, GRID_ALONE);
     T *xp = buf<T>(q.in64, q.in32), *op = buf<T>(q.out64, q.out32), *fr = buf<T>(q.fr64, q.fr32);
     const int64_t nf = frame_values(q.g);
     const dim3 g((unsigned)xcd_grid((p.n + 255) / 256), (unsigned)nrhs);
@@ -859,8 +857,7 @@ void grid_pair_mid64(hala_ctx c, tri_plan &first, tri_plan &second, int nrhs, co
 template <class T, class TIO>
 void grid_exec_pair(hala_ctx c, tri_plan &first, tri_plan &second, const TIO *in, int64_t ldin, TIO *out,
                     int64_t ldout, int nrhs, const int *gate) {
-    grid_reserve(c, first, sizeof(T) == 8, nrhs);
-    grid_reserve(c, second, sizeof(T) == 8, nrhs);
+    grid_reserve_pair(c, first, second, sizeof(T) == 8, nrhs);
     const tri_gridplan &q = first.grid;
     const dim3 g((unsigned)xcd_grid((first.n + 255) / 256), (unsigned)nrhs);
     grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(), in, ldin, 1,

@@ -58,8 +58,13 @@ void grid_reserve_values(tri_plan &p, bool f32);
 bool grid_usable(hala_ctx c, const tri_plan &p, int nrhs = 1);
 // ... and so does second, in first's packed order (an ILU's two triangles).
 bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second, int nrhs = 1);
-// Packed vectors for nrhs right-hand sides.
-void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs);
+// Packed vectors and frames for nrhs right-hand sides of a plan swept alone or in a pair.
+enum grid_role { GRID_ALONE, GRID_FIRST, GRID_SECOND };
+void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs, grid_role role);
+inline void grid_reserve_pair(hala_ctx c, tri_plan &first, tri_plan &second, bool is64, int nrhs) {
+    grid_reserve(c, first, is64, nrhs, GRID_FIRST);
+    grid_reserve(c, second, is64, nrhs, GRID_SECOND);
+}
 
 // out_k = op^-1 in_k for nrhs vectors in natural order (element r of vector k at in[k ldin + r inc] and
 // out[k ldout + r inc]; out may be in), TRI_SUB / TRI_SUM as tri_exec.

@@ -250,3 +250,24 @@ def test_layout_first_used_under_capture():
             torch.cuda.synchronize()
             assert np.array_equal(bits(host(gr)), ref)
             eng.synchronize()
+
+
+def test_pair_keeps_no_unused_buffers():
+    # a factor's grid sweeps: input and output of L, output of U, one set of boundary values each, and the
+    # records; nothing that no sweep reads (a second input and second sets were 0.6 of an 8-byte vector more)
+    eng = H.gpu_engine(0)
+    p, i, v = st.laplace3d(128, 128, 64)
+    n = len(p) - 1
+    gp, gi, gv = eng.load(p), eng.load(i), eng.load(v)
+    B = torch.zeros(16, n, dtype=torch.float64, device="cuda")
+    X = torch.zeros_like(B)
+    M = H.make_ilu(eng, gp, gi, gv)
+    H.solve_batch_cg_ilu(eng, H.stop_criteria(0.0, 2), gp, gi, gv, M, B[:1].contiguous(), X[:1].contiguous())
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    B[:] = 1.0
+    H.solve_batch_cg_ilu(eng, H.stop_criteria(0.0, 2), gp, gi, gv, M, B, X)
+    torch.cuda.synchronize()
+    grown = free0 - torch.cuda.mem_get_info()[0]
+    packed = 16 * 16 * 8 * 144 * 64 * 8  # 16 vectors of 16 x 8 tiles, 144 steps of 64 lanes
+    assert grown <= 3.75 * packed, grown / packed  # 3 vectors + 2 sets of a quarter, and blocks' rounding
