@@ -279,6 +279,16 @@ class tmp_scope {
 
 namespace hala_amd {
 
+// Whether a capture of the context's stream is under way (launches are recorded, not run).
+inline bool capturing(hala_ctx c) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &s) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
 constexpr int CB = 256;  // canonical block (elements per partial, width of the final pass)
 
 // Layout of hala_ctx_s::scal (doubles / unsigned counters)

@@ -247,11 +247,9 @@ static void need(hala_ilu M, tri_plan &p, bool is64, tri_layout layout) {
     int &loaded = is64 ? p.loaded64 : p.loaded32, &rec = is64 ? p.rec64 : p.rec32;
     if ((loaded & layout) && !(rec & layout)) return;
     hala_ctx c = M->ctx;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    HALA_HIP(hipStreamIsCapturing(c->stream, &capture));
     if (is64) load_values64(c, p, M->factor.as<double>(), layout);
     else load_values32(c, p, M->factor.as<double>(), layout);
-    rec = capture != hipStreamCaptureStatusNone ? rec | layout : rec & ~layout;
+    rec = capturing(c) ? rec | layout : rec & ~layout;
 }
 static void need_pair(hala_ilu M, bool is64, tri_layout layout) {
     need(M, M->L, is64, layout);
@@ -267,6 +265,11 @@ static void need_routes(hala_ilu M, bool is64) {
     need(M, M->U, is64, tri_route(M->ctx, M->U));
 }
 
+static ilu_ends grid_ends(tri_plan &first, tri_plan &second, int nrhs) {
+    const int *slot = first.grid.slot.as<int>();
+    return {slot, first.grid.vecs(true, nrhs).in.as<double>(), slot, second.grid.vecs(true, nrhs).out.as<double>(), false};
+}
+
 bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
     hala_ctx c = M->ctx;
     if (!M->factored) return false;
@@ -276,8 +279,7 @@ bool ilu_fused64(hala_ilu M, bool transposed, ilu_ends &e) {
         need(M, first, true, LAYOUT_GRID);
         need(M, second, true, LAYOUT_GRID);
         grid_reserve_pair(c, first, second, true, 1);
-        e = ilu_ends{first.grid.slot.as<int>(), first.grid.in64.as<double>(), first.grid.slot.as<int>(),
-                     second.grid.out64.as<double>(), false};
+        e = grid_ends(first, second, 1);
         return true;
     }
     if (!transposed && use_columns(M)) {
@@ -352,8 +354,7 @@ bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
     N = M->L.grid.g.N;
     if (cols_at_once(N, nrhs) < nrhs) return false;
     grid_reserve_pair(M->ctx, M->L, M->U, true, nrhs);
-    e = ilu_ends{M->L.grid.slot.as<int>(), M->L.grid.in64.as<double>(), M->L.grid.slot.as<int>(),
-                 M->U.grid.out64.as<double>(), false};
+    e = grid_ends(M->L, M->U, nrhs);
     return true;
 }
 

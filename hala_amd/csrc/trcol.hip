@@ -1051,8 +1051,8 @@ void col_sweep(hala_ctx c, tri_plan &p, int mode, T alpha, const int *gate, tri_
     a.alpha = alpha;
     a.out = is64 ? reinterpret_cast<T *>(p.out64.p) : reinterpret_cast<T *>(p.out32.p);
     if (nrhs > 0) {  // vectors in buffers of their own
-        a.xs = q.mxs.as<T>();
-        a.out = q.mout.as<T>();
+        a.xs = q.many.in.as<T>();
+        a.out = q.many.out.as<T>();
     }
     a.hand = nullptr;
     a.ncol = q.ncol;
@@ -1129,19 +1129,31 @@ __global__ void col_scatter_cols(int n, int64_t stride, const int *__restrict__ 
 
 }  // namespace
 
+void col_reserve_many(hala_ctx c, tri_plan &p, int nrhs) {
+    sweep_vecs &v = p.col.many;
+    if (nrhs > v.rhs) {
+        if (v.rhs) HALA_HIP(hipStreamSynchronize(c->stream));  // sweeps in flight still use the smaller buffers
+        v.drop();
+        const size_t bytes = (size_t)((int64_t)p.nchunk * WAVE + BTMAX) * nrhs * sizeof(double);
+        v.in.reserve(bytes);
+        v.out.reserve(bytes);
+        v.rhs = nrhs;
+    }
+    if (capturing(c)) v.pinned = true;
+}
+
 template <class T>
 void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
     tri_colplan &q = p.col;
     const int nslots = p.nchunk * WAVE;
     const int64_t stride = nslots + BTMAX;
-    q.mxs.reserve((size_t)(stride * nrhs) * sizeof(T));
-    q.mout.reserve((size_t)(stride * nrhs) * sizeof(T));
+    col_reserve_many(c, p, nrhs);
     col_gather_cols<T><<<dim3(xcd_grid((nslots + 255) / 256), nrhs), 256, 0, c->stream>>>(
-        nslots, stride, p.chunk_row.as<int>(), b, ldb, inc, q.mxs.as<T>(), q.mout.as<T>());
+        nslots, stride, p.chunk_row.as<int>(), b, ldb, inc, q.many.in.as<T>(), q.many.out.as<T>());
     HALA_CHECK_LAUNCH();
     col_sweep<T, T>(c, p, mode, alpha, nullptr, nullptr, nullptr, 0, nullptr, nrhs);
     col_scatter_cols<T><<<dim3(xcd_grid((p.n + 255) / 256), nrhs), 256, 0, c->stream>>>(
-        p.n, stride, p.slot_of_row.as<int>(), q.mout.as<T>(), b, ldb, inc);
+        p.n, stride, p.slot_of_row.as<int>(), q.many.out.as<T>(), b, ldb, inc);
     HALA_CHECK_LAUNCH();
 }
 template void tri_col_cols<double>(hala_ctx, tri_plan &, int, double, double *, int64_t, int64_t, int);

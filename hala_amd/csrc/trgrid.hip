@@ -669,11 +669,6 @@ int64_t frame_values(const grid_geom &g) {
     return (int64_t)g.ntj * g.ntk * g.S * (g.nz > 1 ? gtile<3>::FR : gtile<2>::FR);
 }
 
-template <class V>
-V *buf(const dbuf &b64, const dbuf &b32) {
-    return sizeof(V) == 8 ? reinterpret_cast<V *>(b64.p) : reinterpret_cast<V *>(b32.p);
-}
-
 }  // namespace
 
 // What grid_probe reads back: dependency count of the row swept last, their distances, a word of the
@@ -802,26 +797,25 @@ bool grid_pair_usable(hala_ctx c, const tri_plan &first, const tri_plan &second,
 }
 
 void grid_reserve(hala_ctx c, tri_plan &p, bool is64, int nrhs, grid_role role) {
-    tri_gridplan &q = p.grid;
-    int &have = is64 ? q.rhs64 : q.rhs32;
-    dbuf &in = is64 ? q.in64 : q.in32, &out = is64 ? q.out64 : q.out32, &fr = is64 ? q.fr64 : q.fr32;
+    sweep_vecs &v = p.grid.vecs(is64, nrhs);
     const size_t w = is64 ? sizeof(double) : sizeof(float);
     // a sweep re-arms its partner's frames, alone a spare set of its own; a pair's second reads the first's output
-    const size_t e = (size_t)q.g.N * w, f = (size_t)frame_values(q.g) * (role == GRID_ALONE ? 2 : 1) * w;
+    const size_t e = (size_t)p.grid.g.N * w, f = (size_t)frame_values(p.grid.g) * (role == GRID_ALONE ? 2 : 1) * w;
     const bool with_in = role != GRID_SECOND;
-    if (nrhs <= have && (!with_in || in.bytes >= e * nrhs) && fr.bytes >= f * nrhs) return;
-    if (have) HALA_HIP(hipStreamSynchronize(c->stream));  // sweeps in flight still use the smaller buffers
-    nrhs = std::max(nrhs, have);
-    have = 0;
-    if (with_in) in.reserve(e * nrhs);
-    out.reserve(e * nrhs);
-    fr.reserve(f * nrhs);
-    const int64_t nf = (int64_t)(fr.bytes / w);  // all of it: what is there of earlier sweeps counts as unarmed
-    const int g = grid_for(nf, 256 * 4, 8192);
-    if (is64) grid_arm<double><<<g, 256, 0, c->stream>>>(fr.as<double>(), nf);
-    else grid_arm<float><<<g, 256, 0, c->stream>>>(fr.as<float>(), nf);
-    HALA_CHECK_LAUNCH();
-    have = nrhs;
+    if (nrhs > v.rhs || (with_in && v.in.bytes < e * nrhs) || v.fr.bytes < f * nrhs) {
+        if (v.rhs) HALA_HIP(hipStreamSynchronize(c->stream));  // sweeps in flight still use the smaller buffers
+        v.drop();
+        if (with_in) v.in.reserve(e * nrhs);
+        v.out.reserve(e * nrhs);
+        v.fr.reserve(f * nrhs);
+        const int64_t nf = (int64_t)(f * nrhs / w);
+        const int g = grid_for(nf, 256 * 4, 8192);
+        if (is64) grid_arm<double><<<g, 256, 0, c->stream>>>(v.fr.as<double>(), nf);
+        else grid_arm<float><<<g, 256, 0, c->stream>>>(v.fr.as<float>(), nf);
+        HALA_CHECK_LAUNCH();
+        v.rhs = nrhs;
+    }
+    if (capturing(c)) v.pinned = true;
 }
 
 template <class T, class TIO>
@@ -829,7 +823,8 @@ void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_
                int nrhs, const int *gate, int64_t inc) {
     tri_gridplan &q = p.grid;
     grid_reserve(c, p, sizeof(T) == 8, nrhs, GRID_ALONE);
-    T *xp = buf<T>(q.in64, q.in32), *op = buf<T>(q.out64, q.out32), *fr = buf<T>(q.fr64, q.fr32);
+    sweep_vecs &v = q.vecs(sizeof(T) == 8, nrhs);
+    T *xp = v.in.as<T>(), *op = v.out.as<T>(), *fr = v.fr.as<T>();
     const int64_t nf = frame_values(q.g);
     const dim3 g((unsigned)xcd_grid((p.n + 255) / 256), (unsigned)nrhs);
     grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(p.n, q.g.N, q.slot.as<int>(), in, ldin, inc, xp, fr, nf, gate);
@@ -843,9 +838,8 @@ void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_
 // values: first's sweep re-arms second's frames and second's first's.
 template <class T>
 static void pair_mid(hala_ctx c, tri_plan &first, tri_plan &second, int nrhs, const int *gate) {
-    T *xp = buf<T>(first.grid.in64, first.grid.in32), *yp = buf<T>(first.grid.out64, first.grid.out32);
-    T *zp = buf<T>(second.grid.out64, second.grid.out32);
-    T *f1 = buf<T>(first.grid.fr64, first.grid.fr32), *f2 = buf<T>(second.grid.fr64, second.grid.fr32);
+    sweep_vecs &u = first.grid.vecs(sizeof(T) == 8, nrhs), &v = second.grid.vecs(sizeof(T) == 8, nrhs);
+    T *xp = u.in.as<T>(), *yp = u.out.as<T>(), *zp = v.out.as<T>(), *f1 = u.fr.as<T>(), *f2 = v.fr.as<T>();
     sweep<T>(c, first, TRI_SUB, T(1), xp, yp, f1, f2, nrhs, gate);
     sweep<T>(c, second, TRI_SUB, T(1), yp, zp, f2, f1, nrhs, gate);
 }
@@ -861,12 +855,13 @@ void grid_exec_pair(hala_ctx c, tri_plan &first, tri_plan &second, const TIO *in
     const tri_gridplan &q = first.grid;
     const dim3 g((unsigned)xcd_grid((first.n + 255) / 256), (unsigned)nrhs);
     grid_gather<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(), in, ldin, 1,
-                                                  buf<T>(q.in64, q.in32), nullptr, 0, gate);
+                                                  first.grid.vecs(sizeof(T) == 8, nrhs).in.template as<T>(), nullptr, 0,
+                                                  gate);
     HALA_CHECK_LAUNCH();
     pair_mid<T>(c, first, second, nrhs, gate);
     grid_scatter<T, TIO><<<g, 256, 0, c->stream>>>(first.n, q.g.N, q.slot.as<int>(),
-                                                   buf<T>(second.grid.out64, second.grid.out32), out, ldout, 1,
-                                                   gate);
+                                                   second.grid.vecs(sizeof(T) == 8, nrhs).out.template as<T>(), out,
+                                                   ldout, 1, gate);
     HALA_CHECK_LAUNCH();
 }
 

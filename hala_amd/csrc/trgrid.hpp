@@ -17,6 +17,8 @@
 // mirrored grid, whose packed order is the forward one reversed, so an ILU's
 // two sweeps share one order and need no permutation between them.
 #pragma once
+#include <vector>
+
 #include "common.hpp"
 
 namespace hala_amd {
@@ -30,6 +32,26 @@ struct grid_geom {
     bool same(const grid_geom &o) const { return nx == o.nx && ny == o.ny && nz == o.nz; }
 };
 
+// Buffers of `rhs` vectors in a sweep's order, made on first use: input, output and (grid sweeps) frames, the
+// boundary results that the tiles poll, sentinels before a sweep.
+struct sweep_vecs {
+    dbuf in, out, fr;
+    int rhs = 0;
+    bool pinned = false;     // a stream capture recorded work on them,
+    std::vector<dbuf> kept;  // ... so what larger ones replace stays until the plan goes
+    // for larger ones to take their place
+    void drop() {
+        if (pinned)
+            for (dbuf *b : {&in, &out, &fr})
+                if (b->p) kept.emplace_back(std::move(*b));
+        in.release();
+        out.release();
+        fr.release();
+        rhs = 0;
+        pinned = false;
+    }
+};
+
 // The grid side of a plan (member of tri_plan).
 struct tri_gridplan {
     bool ok = false;
@@ -38,10 +60,10 @@ struct tri_gridplan {
     grid_geom g;
     dbuf slot;          // packed element (forward order) of every natural row, then the tile of every ticket
     dbuf rec64, rec32;  // per (tile, step) the step's coefficients and diagonal (see grid_pack)
-    // packed input, output and frames (boundary results the tiles poll; sentinels
-    // before a sweep) of `rhs64` / `rhs32` vectors, made on first use
-    dbuf in64, in32, out64, out32, fr64, fr32;
-    int rhs64 = 0, rhs32 = 0;
+    sweep_vecs one64, one32, many64, many32;
+    // Several vectors have buffers of their own: those of one vector never move, whatever else the plan
+    // solves (a captured apply holds their addresses).
+    sweep_vecs &vecs(bool is64, int nrhs) { return nrhs > 1 ? (is64 ? many64 : many32) : (is64 ? one64 : one32); }
 };
 
 // Recognises p's pattern from its dependency lists and lays the grid plan out (p.grid.ok tells), in three
@@ -76,8 +98,8 @@ void grid_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIO *in, int64_
 template <class T, class TIO>
 void grid_exec_pair(hala_ctx c, tri_plan &first, tri_plan &second, const TIO *in, int64_t ldin, TIO *out,
                     int64_t ldout, int nrhs, const int *gate);
-// The pair without its ends: first's packed input (in64, filled by the caller)
-// to second's packed output (out64), both by first's slot map.
+// The pair without its ends: first's packed input (filled by the caller) to
+// second's packed output, both by first's slot map.
 void grid_pair_mid64(hala_ctx c, tri_plan &first, tri_plan &second, int nrhs, const int *gate);
 
 }  // namespace hala_amd

@@ -50,7 +50,7 @@ struct tri_colplan {
     dbuf spar;                   // per slot: parity of its level within its column (which external buffer it reads)
     dbuf val64, val32;           // packed row records (see col_pack)
     dbuf xs64, xs32;             // input, gathered into slot order per sweep
-    dbuf mxs, mout;              // the same and the polled output for several right-hand sides at once
+    sweep_vecs many;             // the same and the polled output for several right-hand sides at once (bytes: rhs 8-byte vectors)
     bool upward = false;         // some column waits on a higher-numbered one (every column then needs a CU)
     bool hand64 = false;         // val64 carries hand-off slots (col_set_handoff)
 };
@@ -154,6 +154,7 @@ void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb
 // ncol_req = 0 picks the column count.  tri_exec uses it when present and
 // enabled (option tri_col).
 bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req);
+void col_reserve_many(hala_ctx c, tri_plan &p, int nrhs);
 template <class T>
 void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs);
 void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);

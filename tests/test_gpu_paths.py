@@ -271,3 +271,54 @@ def test_pair_keeps_no_unused_buffers():
     grown = free0 - torch.cuda.mem_get_info()[0]
     packed = 16 * 16 * 8 * 144 * 64 * 8  # 16 vectors of 16 x 8 tiles, 144 steps of 64 lanes
     assert grown <= 3.75 * packed, grown / packed  # 3 vectors + 2 sets of a quarter, and blocks' rounding
+
+
+@pytest.mark.parametrize("name", ["grid", "columns"])
+def test_captured_sweeps_survive_larger_solves(name):
+    # a captured apply and a captured trsm hold their buffers' addresses: solves of more vectors on the same
+    # objects leave them alone, and replays give the eager bits
+    p, i, v = st.laplace3d(13, 12, 11)
+    n = len(p) - 1
+    row = np.repeat(np.arange(n), np.diff(p))
+    keep = i <= row
+    q = np.zeros(n + 1, np.int32)
+    q[1:] = np.cumsum(np.bincount(row[keep], minlength=n))
+    li, lv = i[keep].copy(), v[keep].copy()
+    dg, _ = oracle.diag(p, i)
+    f = oracle.ilu0(p, i, v, dg)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        eng = H.gpu_engine(0, stream=s)
+        eng.set_option("sync_checks", 0)
+        eng.set_option("tri_grid", 1 if name == "grid" else 0)
+        gp, gi, gv = eng.load(p), eng.load(i), eng.load(v)
+        M = H.make_ilu(eng, gp, gi, gv)
+        T = H.make_triangular_matrix(eng, "L", "N", eng.load(q), eng.load(li), eng.load(lv))
+        gx, gr = eng.load(st.uniform(1, n)), eng.vector(n)
+        b = np.stack([st.uniform(20 + k, n) for k in range(3)])
+        gb = eng.load(b)
+        M.apply(gx, gr)
+        T.trsm("N", "N", 3, 1.5, gb.clone())
+        eng.synchronize()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            M.apply(gx, gr)
+            T.trsm("N", "N", 3, 1.5, gb)
+        for seed in (4, 5, 6):
+            # more vectors than the captured calls had, on the same objects
+            k = 4 * seed
+            B = torch.rand(k, n, dtype=torch.float64, device="cuda")
+            T.trsm("N", "N", k, 1.0, B)
+            X = torch.zeros(k, n, dtype=torch.float64, device="cuda")
+            H.solve_batch_cg_ilu(eng, H.stop_criteria(0.0, 3), gp, gi, gv, M, torch.ones_like(X), X)
+            x = st.uniform(seed, n)
+            gx.copy_(eng.load(x))
+            gb.copy_(eng.load(b * seed))
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(bits(host(gr)), bits(oracle.ilu_apply(p, i, dg, f, x)))
+            for c in range(3):
+                ref = oracle.trsv("L", "N", "N", 1.5, q, li, lv, b[c] * seed)
+                assert np.array_equal(bits(host(gb[c])), bits(ref))
+            eng.synchronize()
