@@ -8,6 +8,7 @@ computation is a call into libhala_amd.so through its C ABI.  The C++ drop-in
 for user code calling hala:: is include/hala.hpp and include/hala_solvers.hpp.
 """
 import ctypes as C
+import threading
 
 import numpy as np
 
@@ -30,6 +31,47 @@ def _ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
 
+class _context:
+    """An engine's context, destroyed with the last of the engine and the objects made on it.
+
+    Python may finalise an engine before its objects (everything in one garbage cycle, a failed call's
+    traceback say); an object destroyed on a freed context would wait on a freed stream.
+    """
+
+    _lock = threading.RLock()  # reentrant: a collection may finalise objects while it is held
+
+    def __init__(self, handle):
+        self.handle, self.users = handle, 1
+
+    def hold(self):
+        with self._lock:
+            self.users += 1
+        return self
+
+    def drop(self):
+        with self._lock:
+            self.users -= 1
+            last = self.users == 0
+        if last and callable(lib):
+            lib().hala_ctx_destroy(self.handle)
+
+
+class _owned:
+    """A native object on an engine's context; _destroy names its destructor."""
+
+    handle = None
+
+    def _own(self, engine, handle):
+        self._ctx = engine._ctx.hold()
+        self.handle = handle
+
+    def __del__(self):
+        if self.handle is not None and callable(lib):
+            getattr(lib(), self._destroy)(self.handle)
+            self.handle = None
+            self._ctx.drop()
+
+
 class stop_criteria:
     """hex/solvers/hala_solvers_core.hpp:52-71: absolute tolerance and/or iteration cap."""
 
@@ -50,11 +92,12 @@ class gpu_engine:
         h = C.c_void_p()
         call("hala_ctx_create", self._device, C.c_void_p(stream.cuda_stream), C.byref(h))
         self.handle = h
+        self._ctx = _context(h)
 
     def __del__(self):
-        if getattr(self, "handle", None) is not None and callable(lib):
-            lib().hala_ctx_destroy(self.handle)
-            self.handle = None
+        if getattr(self, "_ctx", None) is not None:
+            self._ctx.drop()
+            self._ctx = self.handle = None
 
     def device(self):
         return self._device
@@ -98,8 +141,10 @@ def _dt(t):
     return {torch.float64: 64, torch.float32: 32}[t.dtype]
 
 
-class gpu_sparse_matrix:
+class gpu_sparse_matrix(_owned):
     """gpu/hala_rocm_sparse_general.hpp:74-169: non-owning view of a device CSR (kept alive here)."""
+
+    _destroy = "hala_csr_destroy"
 
     def __init__(self, engine, nrows, ncols, pntr, indx, vals):
         self.engine = engine
@@ -108,12 +153,7 @@ class gpu_sparse_matrix:
         h = C.c_void_p()
         call("hala_csr_create", engine.handle, self.nrows, self.ncols, int(indx.numel()), _ptr(pntr), _ptr(indx),
              C.byref(h))
-        self.handle = h
-
-    def __del__(self):
-        if getattr(self, "handle", None) is not None and callable(lib):
-            lib().hala_csr_destroy(self.handle)
-            self.handle = None
+        self._own(engine, h)
 
     def info(self):
         inf = CsrInfo()
@@ -161,8 +201,10 @@ def sparse_gemv(engine, trans, M, N, alpha, pntr, indx, vals, x, beta, y):
     return gpu_sparse_matrix(engine, M, N, pntr, indx, vals).gemv(trans, alpha, x, beta, y)
 
 
-class gpu_ilu:
+class gpu_ilu(_owned):
     """gpu/hala_gpu_ilu.hpp:45-185: ILU(0) factor owned on the device, pattern aliased."""
+
+    _destroy = "hala_ilu_destroy"
 
     def __init__(self, engine, pntr, indx, vals, policy="N", want_f32=False):
         self.engine = engine
@@ -171,15 +213,10 @@ class gpu_ilu:
         self.nnz = int(indx.numel())
         h = C.c_void_p()
         call("hala_ilu_create", engine.handle, self.n, self.nnz, _ptr(pntr), _ptr(indx), C.byref(h))
-        self.handle = h
+        self._own(engine, h)
         self.policy = policy
         if vals is not None:
             self.factor(vals, want_f32)
-
-    def __del__(self):
-        if getattr(self, "handle", None) is not None and callable(lib):
-            lib().hala_ilu_destroy(self.handle)
-            self.handle = None
 
     def factor(self, vals, want_f32=False):
         call("hala_ilu_factor_f64", self.handle, _ptr(vals), int(bool(want_f32)))
@@ -242,8 +279,10 @@ def make_ilu(engine, pntr, indx, vals, policy="N", want_f32=False):
     return gpu_ilu(engine, pntr, indx, vals, policy, want_f32)
 
 
-class gpu_triangular_matrix:
+class gpu_triangular_matrix(_owned):
     """gpu/hala_rocm_sparse_triangular.hpp:29-178 with sparse_trsv_array semantics."""
+
+    _destroy = "hala_tri_destroy"
 
     def __init__(self, engine, uplo, diag, pntr, indx, vals):
         self.engine = engine
@@ -252,12 +291,7 @@ class gpu_triangular_matrix:
         h = C.c_void_p()
         call("hala_tri_create", engine.handle, uplo.encode(), diag.encode(), self.n, int(indx.numel()), _ptr(pntr),
              _ptr(indx), C.byref(h))
-        self.handle = h
-
-    def __del__(self):
-        if getattr(self, "handle", None) is not None and callable(lib):
-            lib().hala_tri_destroy(self.handle)
-            self.handle = None
+        self._own(engine, h)
 
     def _suffix(self):
         import torch
@@ -433,8 +467,10 @@ def solve_gmres_ir(engine, matrix, vals, vals32, ilu, b, x, rtol=1e-10, inner_rt
 
 
 # ---- batched independent systems -------------------------------------------------
-class batch_solver:
+class batch_solver(_owned):
     """Jacobi-PCG over many independent packed CSR systems in one persistent launch."""
+
+    _destroy = "hala_batch_destroy"
 
     def __init__(self, engine, row_off, pntr, indx):
         self.engine = engine
@@ -442,12 +478,7 @@ class batch_solver:
         self.nsys = int(row_off.numel()) - 1
         h = C.c_void_p()
         call("hala_batch_create", engine.handle, self.nsys, _ptr(row_off), _ptr(pntr), _ptr(indx), C.byref(h))
-        self.handle = h
-
-    def __del__(self):
-        if getattr(self, "handle", None) is not None and callable(lib):
-            lib().hala_batch_destroy(self.handle)
-            self.handle = None
+        self._own(engine, h)
 
     def set_shape(self, team, wg_per_cu):
         call("hala_batch_set_shape", self.handle, int(team), int(wg_per_cu))
