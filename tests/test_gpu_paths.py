@@ -254,7 +254,7 @@ def test_layout_first_used_under_capture():
 
 def test_pair_keeps_no_unused_buffers():
     # a factor's grid sweeps: input and output of L, output of U, one set of boundary values each, and the
-    # records; nothing that no sweep reads (a second input and second sets were 0.6 of an 8-byte vector more)
+    # records; nothing that no sweep reads (U's input and second sets made it 5 packed vectors instead of 3.5)
     eng = H.gpu_engine(0)
     p, i, v = st.laplace3d(128, 128, 64)
     n = len(p) - 1
@@ -263,9 +263,11 @@ def test_pair_keeps_no_unused_buffers():
     X = torch.zeros_like(B)
     M = H.make_ilu(eng, gp, gi, gv)
     H.solve_batch_cg_ilu(eng, H.stop_criteria(0.0, 2), gp, gi, gv, M, B[:1].contiguous(), X[:1].contiguous())
+    B[:] = 1.0
+    # the solver's own work vectors come and go with the call, and the runtime may keep them: not counted
+    H.solve_batch_cg(eng, H.stop_criteria(0.0, 2), gp, gi, gv, None, B, X)
     torch.cuda.synchronize()
     free0 = torch.cuda.mem_get_info()[0]
-    B[:] = 1.0
     H.solve_batch_cg_ilu(eng, H.stop_criteria(0.0, 2), gp, gi, gv, M, B, X)
     torch.cuda.synchronize()
     grown = free0 - torch.cuda.mem_get_info()[0]
