@@ -373,6 +373,7 @@ void run_cg_batch(hala_ctx c, hala_csr A, const double *vals, hala_ilu M, int nr
         if (batch < c->opt.cg_batch_max) batch = std::min(2 * batch, std::max(c->opt.cg_batch_max, 1));
     }
     check_wait_error(c);
+    if (!ident) ilu_cols_done(M);
     if (iterations) *iterations = it;
 }
 

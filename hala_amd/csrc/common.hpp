@@ -176,6 +176,7 @@ struct dbuf {
             hipError_t e = hipMalloc(&p, b);
             if (e != hipSuccess) {
                 p = nullptr;
+                (void)hipGetLastError();  // reported here: a caller that makes do with less launches on
                 throw status_error{HALA_ERR_ALLOC, "hipMalloc of " + std::to_string(b) + " bytes failed"};
             }
             got = b;
@@ -206,6 +207,7 @@ struct hala_options {
     int tri_col_cols = 0;      // columns of the blocked sweep (0: smallest that fits)
     int tri_col_split = 0;     // columns per slab of planes (0: automatic, 1: contiguous row blocks)
     int tri_grid = 1;          // register-wavefront sweeps of complete 5-/7-point grid patterns (0: column sweeps)
+    int rhs_mib = 2048;        // MiB of one packed copy of the right-hand sides swept together; more go in strips
     int cg_small = 1;          // identity / Jacobi CG of a small system in one workgroup (0: launched passes)
     int cg_fuse = 1;           // ILU-PCG: the sweeps' gather/scatter fused into the update and r.z kernels
     int cg_xcd = 1;            // fused ILU-PCG: the update (scatter into L's slot order) in XCD-aware block order

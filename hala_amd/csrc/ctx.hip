@@ -213,6 +213,7 @@ static int *option_slot(hala_ctx c, const char *name) {
     if (k == "tri_col_cols") return &c->opt.tri_col_cols;
     if (k == "tri_col_split") return &c->opt.tri_col_split;
     if (k == "tri_grid") return &c->opt.tri_grid;
+    if (k == "rhs_mib") return &c->opt.rhs_mib;
     if (k == "cg_small") return &c->opt.cg_small;
     if (k == "cg_fuse") return &c->opt.cg_fuse;
     if (k == "cg_xcd") return &c->opt.cg_xcd;

@@ -330,9 +330,13 @@ void ilu_apply64(hala_ilu M, const double *x, double *r, const int *gate) {
     tri_exec<double, double, double>(c, M->U, TRI_SUB, 1.0, M->tmp64.as<double>(), r, gate);
 }
 
-// Vectors swept together at most: enough to fill the chip, and a bound on the packed copies
-static constexpr int64_t COLS_ELEMS = 1ll << 28;
-static int cols_at_once(int64_t N, int nrhs) { return (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, COLS_ELEMS / N, 4096})); }
+// vectors that the grid sweeps take together, their buffers reserved
+static int cols_at_once(hala_ilu M, int nrhs) {
+    hala_ctx c = M->ctx;
+    const int have = std::min(M->L.grid.vecs(true, nrhs).rhs, M->U.grid.vecs(true, nrhs).rhs);
+    return vectors_at_once(c, M->L.grid.g.N * sizeof(double), nrhs, have,
+                           [&](int m) { grid_reserve_pair(c, M->L, M->U, true, m); });
+}
 
 void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const int *gate) {
     hala_ctx c = M->ctx;
@@ -340,7 +344,7 @@ void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const in
     const int64_t n = M->n;
     const bool grid = use_grid(M, nrhs);
     if (grid) need_pair(M, true, LAYOUT_GRID);
-    const int step = grid ? cols_at_once(M->L.grid.g.N, nrhs) : 1;
+    const int step = grid ? cols_at_once(M, nrhs) : 1;
     for (int k = 0; k < nrhs; k += step) {
         const int m = std::min(step, nrhs - k);
         if (grid) grid_exec_pair<double, double>(c, M->L, M->U, x + k * n, n, r + k * n, n, m, gate);
@@ -352,10 +356,14 @@ bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N) {
     if (!use_grid(M, nrhs)) return false;
     need_pair(M, true, LAYOUT_GRID);
     N = M->L.grid.g.N;
-    if (cols_at_once(N, nrhs) < nrhs) return false;
-    grid_reserve_pair(M->ctx, M->L, M->U, true, nrhs);
+    if (cols_at_once(M, nrhs) < nrhs) return false;
     e = grid_ends(M->L, M->U, nrhs);
     return true;
+}
+
+void ilu_cols_done(hala_ilu M) {
+    M->L.grid.many64.give_back();
+    M->U.grid.many64.give_back();
 }
 
 void ilu_apply64_cols_mid(hala_ilu M, int nrhs, const int *gate) {

@@ -78,6 +78,7 @@ void ilu_apply64_mid(hala_ilu M, bool transposed, const int *gate, const hala_am
 void ilu_apply64_cols(hala_ilu M, const double *x, double *r, int nrhs, const int *gate);
 bool ilu_fused64_cols(hala_ilu M, int nrhs, ilu_ends &e, int64_t &N);
 void ilu_apply64_cols_mid(hala_ilu M, int nrhs, const int *gate);
+void ilu_cols_done(hala_ilu M);  // after the last of them (the stream synchronised): large buffers are given back
 void ilu_apply32x64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_apply_t64(hala_ilu M, const double *x, double *r, const int *gate = nullptr);
 void ilu_prepare_adjoint(hala_ilu M);

@@ -236,13 +236,17 @@ void tri_exec(hala_ctx c, tri_plan &p, int mode, T alpha, const TIN *in, TOUT *o
 template <class T>
 void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs) {
     constexpr bool is64 = sizeof(T) == 8;
-    constexpr int64_t ELEMS = 1ll << 28;  // elements of one packed copy at most
     const tri_layout route = tri_route(c, p, nrhs);
     HALA_REQUIRE((is64 ? p.loaded64 : p.loaded32) & route, HALA_ERR_ARG,
                  "triangular solve: values not loaded for this precision");
     const bool grid = route == LAYOUT_GRID, col = route == LAYOUT_COLUMNS && !p.col.upward;
-    const int64_t per = grid ? p.grid.g.N : (int64_t)p.nchunk * WAVE + SLOT_PAD;
-    const int at_once = (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, ELEMS / per, 4096}));
+    int at_once = 1;
+    if (grid)
+        at_once = vectors_at_once(c, p.grid.g.N * sizeof(T), nrhs, p.grid.vecs(is64, nrhs).rhs,
+                                  [&](int m) { grid_reserve(c, p, is64, m, GRID_ALONE); });
+    else if (col && nrhs > 1)
+        at_once = vectors_at_once(c, ((int64_t)p.nchunk * WAVE + SLOT_PAD) * sizeof(double), nrhs, p.col.many.rhs,
+                                  [&](int m) { if (m > 1) col_reserve_many(c, p, m); });
     if (grid || (col && at_once > 1)) {
         for (int k = 0; k < nrhs; k += at_once) {
             const int m = std::min(at_once, nrhs - k);
@@ -250,6 +254,7 @@ void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb
             if (grid) grid_exec<T, T>(c, p, mode, alpha, bk, ldb, bk, ldb, m, nullptr, inc);
             else tri_col_cols<T>(c, p, mode, alpha, bk, ldb, inc, m);
         }
+        (grid ? p.grid.vecs(is64, 2) : p.col.many).give_back();
         return;
     }
     tmp_scope ts(c);

@@ -39,6 +39,11 @@ struct sweep_vecs {
     int rhs = 0;
     bool pinned = false;     // a stream capture recorded work on them,
     std::vector<dbuf> kept;  // ... so what larger ones replace stays until the plan goes
+    // What a plan keeps for the next call of several vectors; more is given back at the end of the call.
+    static constexpr size_t KEEP = size_t(1) << 30;
+    void give_back() {
+        if (!pinned && in.bytes + out.bytes + fr.bytes > KEEP) drop();
+    }
     // for larger ones to take their place
     void drop() {
         if (pinned)

@@ -16,6 +16,7 @@
 // agent-scope loads until it differs from a signalling-NaN sentinel: the
 // value is its own ready flag, no fences are needed.  Every wait is bounded.
 #pragma once
+#include <algorithm>
 #include <vector>
 
 #include "trgrid.hpp"
@@ -155,6 +156,22 @@ void tri_exec_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb
 // enabled (option tri_col).
 bool build_col_plan(hala_ctx c, tri_plan &p, int ncol_req);
 void col_reserve_many(hala_ctx c, tri_plan &p, int nrhs);
+// Vectors of `bytes` in a sweep's order that are taken together of nrhs: within option rhs_mib, and as many as
+// reserve(m) finds memory for, halving (a capture cannot allocate: as many as there is room for, `have`).
+template <class F>
+int vectors_at_once(hala_ctx c, int64_t bytes, int nrhs, int have, const F &reserve) {
+    int m = (int)std::max<int64_t>(1, std::min<int64_t>({nrhs, ((int64_t)c->opt.rhs_mib << 20) / bytes, 4096}));
+    if (m > have && capturing(c)) m = std::max(have, 1);
+    for (;;) {
+        try {
+            reserve(m);
+            return m;
+        } catch (status_error &e) {
+            if (e.code != HALA_ERR_ALLOC || m == 1) throw;
+            m = (m + 1) / 2;
+        }
+    }
+}
 template <class T>
 void tri_col_cols(hala_ctx c, tri_plan &p, int mode, T alpha, T *b, int64_t ldb, int64_t inc, int nrhs);
 void col_load_values(hala_ctx c, tri_plan &p, const double *factor, bool f32);

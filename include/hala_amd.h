@@ -63,7 +63,9 @@ int hala_ctx_device(hala_ctx ctx, int *device);
  * a grid-stride loop).  Paths: "tri_col" (1: column-blocked
  * sweeps where the plan fits, 0: level pool), "tri_grid" (1: register-wavefront sweeps on
  * complete 5-/7-point grids while the column options are automatic, 0: column sweeps), "tri_stencil" (1: pencil sweeps
- * for stencil patterns, read when the ILU object is created), "cg_small" (1: identity
+ * for stencil patterns, read when the ILU object is created), "rhs_mib" (MiB of
+ * one packed copy of the right-hand sides that exact sweeps take together,
+ * default 2048: more are swept in strips, 0: one by one), "cg_small" (1: identity
  * and Jacobi CG of up to 4096 rows in one workgroup, 0: launched passes), "cg_fuse" (1:
  * the sweeps' permutations fused into the PCG vector kernels), "cg_xcd" (1:
  * with cg_fuse, the r update and its scatter into the L sweep's input in

@@ -218,6 +218,42 @@ def test_trsm_many_columns(engine, name, uplo):
         engine.set_option("tri_col", saved[1])
 
 
+@pytest.mark.parametrize("name", ["grid", "columns"])
+@pytest.mark.parametrize("mib", [0, 1, 2])
+def test_strips_of_vectors(engine, name, mib):
+    # more vectors than a packed copy may hold go in strips, with a remainder, down to one by one: same bits
+    p, i, v = st.laplace3d(40, 24, 25)
+    n = len(p) - 1
+    row = np.repeat(np.arange(n), np.diff(p))
+    keep = i <= row
+    q = np.zeros(n + 1, np.int32)
+    q[1:] = np.cumsum(np.bincount(row[keep], minlength=n))
+    li, lv = i[keep].copy(), v[keep].copy()
+    gp, gi, gv = engine.load(p), engine.load(i), engine.load(v)
+    saved = engine.get_option("tri_grid"), engine.get_option("rhs_mib")
+    try:
+        engine.set_option("tri_grid", 1 if name == "grid" else 0)
+        engine.set_option("rhs_mib", mib)
+        T = H.make_triangular_matrix(engine, "L", "N", engine.load(q), engine.load(li), engine.load(lv))
+        B = np.stack([st.uniform(70 + k, n) for k in range(11)])
+        g = engine.load(B)
+        T.trsm("N", "N", 11, 1.5, g)
+        for k in range(11):
+            assert np.array_equal(bits(host(g[k])), bits(oracle.trsv("L", "N", "N", 1.5, q, li, lv, B[k])))
+        M = H.make_ilu(engine, gp, gi, gv)
+        X = torch.zeros(11, n, dtype=torch.float64, device="cuda")
+        H.solve_batch_cg_ilu(engine, H.stop_criteria(0.0, 4), gp, gi, gv, M, engine.load(B), X)
+        assert engine.get_option("path_pcg") == 0  # not fused: the solve's vectors exceed a strip
+        dg, _ = oracle.diag(p, i)
+        f = oracle.ilu0(p, i, v, dg)
+        for k in (0, 4, 10):
+            _, x, _ = oracle.cg(p, i, v, B[k], tol=0.0, max_iter=4, prec=oracle.PREC_ILU, mpntr=p, mindx=i, mdiag=dg, mdata=f)
+            assert np.array_equal(bits(host(X[k])), bits(x)), k
+    finally:
+        engine.set_option("tri_grid", saved[0])
+        engine.set_option("rhs_mib", saved[1])
+
+
 @pytest.mark.parametrize("name", ["grid3", "column"])
 @pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 8, 9])
 def test_multirhs_pcg_grid_and_columns(engine, name, nrhs):
@@ -285,3 +321,23 @@ def test_multirhs_cg_products(engine, name):
         for k in sorted({0, nrhs // 2, nrhs - 1}):
             _, x, _ = oracle.cg(p, i, v, B[k], tol=0.0, max_iter=passes)
             assert np.array_equal(bits(host(X[k])), bits(x)), (nrhs, k)
+
+
+def test_large_strips_are_given_back():
+    # the packed copies of many right-hand sides go back at the end of the call once they pass a gibibyte
+    eng = H.gpu_engine(0)
+    p, i, v = st.laplace3d(96, 96, 96)
+    n = len(p) - 1
+    row = np.repeat(np.arange(n), np.diff(p))
+    keep = i <= row
+    q = np.zeros(n + 1, np.int32)
+    q[1:] = np.cumsum(np.bincount(row[keep], minlength=n))
+    T = H.make_triangular_matrix(eng, "L", "N", eng.load(q), eng.load(i[keep].copy()), eng.load(v[keep].copy()))
+    B = torch.rand(100, n, dtype=torch.float64, device="cuda")
+    for k, most in ((4, 200), (100, 64)):  # MiB that stay: a few vectors' buffers, then none of the large ones
+        T.trsm("N", "N", 1, 1.0, B)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        T.trsm("N", "N", k, 1.0, B)
+        torch.cuda.synchronize()
+        assert free - torch.cuda.mem_get_info()[0] <= most << 20, k
