@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <rocprofiler-sdk-roctx/roctx.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -85,6 +86,13 @@ int guard(F &&body) {
 // on that stream may still read it is handed out again only to later work on
 // the same stream, and owners synchronise the stream before their final
 // release (an ILU destroy does).
+// Bytes of device memory that the library's buffers hold in this process (caches included).
+inline std::atomic<int64_t> held_bytes{0};
+inline void free_block(void *p, size_t b) {
+    (void)hipFree(p);
+    held_bytes -= (int64_t)b;
+}
+
 struct buf_cache {
     std::mutex m;
     std::multimap<size_t, void *> blocks;  // size -> block
@@ -110,10 +118,10 @@ struct buf_cache {
                 return;
             }
         }
-        (void)hipFree(p);
+        free_block(p, b);
     }
     ~buf_cache() {
-        for (auto &kv : blocks) (void)hipFree(kv.second);
+        for (auto &kv : blocks) free_block(kv.second, kv.first);
     }
 };
 
@@ -160,7 +168,7 @@ struct dbuf {
     void release() {
         if (p) {
             if (cache) cache->put(p, bytes);
-            else (void)hipFree(p);
+            else free_block(p, bytes);
         }
         p = nullptr;
         bytes = 0;
@@ -180,6 +188,7 @@ struct dbuf {
                 throw status_error{HALA_ERR_ALLOC, "hipMalloc of " + std::to_string(b) + " bytes failed"};
             }
             got = b;
+            held_bytes += (int64_t)b;
         }
         cache = tl_cache;
         bytes = got;

@@ -251,6 +251,8 @@ int hala_ctx_get_option(hala_ctx c, const char *name, int *value) {
         HALA_REQUIRE(c && value, HALA_ERR_ARG, "null argument");
         const int *slot = option_slot(c, name);
         if (!slot) slot = path_slot(c, name);
+        const int held = (int)(held_bytes >> 20);
+        if (!slot && name && std::strcmp(name, "held_mib") == 0) slot = &held;
         HALA_REQUIRE(slot, HALA_ERR_ARG, std::string("unknown option ") + (name ? name : "(null)"));
         *value = *slot;
     });

@@ -76,7 +76,8 @@ int hala_ctx_device(hala_ctx ctx, int *device);
  * dependency wait that gave up; 0: the report is deferred to the next
  * synchronising call).  Unknown names return HALA_ERR_ARG.
  *
- * hala_ctx_get_option also reads which kernels the context's last call of a
+ * hala_ctx_get_option also reads "held_mib", the device memory that the
+ * library's own buffers hold in this process, and which kernels the context's last call of a
  * family ran (-1: none yet): "path_sweep" (0 level pool, 1 columns, 2 grid
  * wavefronts, 3 pencils), "path_pcg" (ILU-PCG; 0 separate applies, 1 fused
  * column sweeps, 2 fused grid sweeps), "path_cg" (identity and Jacobi CG; 0
