@@ -112,6 +112,9 @@ int hala_tri_create(hala_ctx c, char uplo, char diag, int n, int64_t nnz, const 
         int bad = validate_pattern(c, n, n, nnz, pntr, indx, 1);
         HALA_REQUIRE(bad < 0, HALA_ERR_PATTERN, "hala_tri_create: invalid pattern at row " + std::to_string(bad));
         auto *T = new hala_tri_s();
+        // the plans' buffers come from the context's cache (hala_tri_destroy synchronises before it returns
+        // them): the grid layout's were four allocations and frees more, 30 us each
+        alloc_scope as(c->cache.get());
         try {
             T->ctx = c;
             T->n = n;
