@@ -9,10 +9,11 @@
 //         x_k += a_k p_k; r_k += (-a_k) Ap_k;
 //         stop if it == max_iter or max_k ||r_k|| < tol (batch_max_norm2);
 //         z = M r; nzr_k = <r_k, z_k>; b_k = nzr_k / zr_k; p_k = b_k p_k; p += 1*z; zr = nzr
-// The sweeps of all columns run in one launch (64^3, 8 columns: 17.8 ms per solve
-// of 124 passes; one apply after the other 78 ms).  All columns iterate until the stop.  The dots are this build's canonical
-// order per column; the product reads each matrix tile once for up to
-// CGB_GROUP columns.
+// On complete grids the sweeps of all columns run in one launch (64^3, 8 columns:
+// 17.8 ms per solve of 124 passes; one apply after the other 78 ms); other
+// factors apply to column after column.  All columns iterate until the stop.  The
+// dots are this build's canonical order per column; the product reads each
+// matrix entry once for up to CGB_GROUP columns.
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -34,7 +34,7 @@ struct gtile {
     static constexpr int FR = DIM == 3 ? 16 : 1;
     // lanes that poll one step (3-D: 4 for the k-1 tile's row, 4 for the j-1 tile's, two values each)
     static constexpr int LPS = DIM == 3 ? 8 : 1, FV = DIM == 3 ? 2 : 1;
-    // ring of steps in LDS: per step the 64 results (read two steps later as the
+    // ring of steps in LDS: per step the 64 results (read by the next step as the
     // k-1 values) and the frame values (2-D: the frame value alone)
     static constexpr int SLOT = DIM == 3 ? 64 + 16 : 1;
     static constexpr int R = DIM == 3 ? 32 : 256;
@@ -723,10 +723,12 @@ bool grid_layout(hala_ctx c, tri_plan &p) {
     g.ntk = (g.nz + TK - 1) / TK;
     g.S = (g.nx + lag_of(dim) + 7) / 8 * 8;
     g.N = (int64_t)g.ntj * g.ntk * g.S * WAVE;
-    // tiles of short lines or few lanes are mostly padding: streaming it would
-    // cost more than the general sweeps' level steps (small systems keep it:
-    // they live in the caches)
-    if (g.N > 3 * (int64_t)n && g.N > (1 << 20)) return false;
+    // Tiles of short lines or few lanes are mostly padding.  That costs memory, 32 bytes of record per packed
+    // element, so past 2^23 elements (256 MiB of records) a grid has to fill a third of them; it does not cost
+    // time, a step takes what it takes.  Applies, columns -> grid: 2 x 20000 (36 elements per row) 7407 -> 4314
+    // us, 20000 x 8 (8) 8131 -> 3698, 20 x 60000 (4.4) 31164 -> 13781, 2 x 300 x 300 (8) 345 -> 311, 3 x 500 x
+    // 500 (8) 578 -> 562.
+    if (g.N > 3 * (int64_t)n && g.N > (1 << 23)) return false;
     if (g.N > (1 << 28)) return false;  // 32-bit byte offsets into a vector's frames
     q.g = g;
     // A hop from tile to tile takes as long as about ten levels of a few rows of the column sweep (1.8 us

@@ -6,11 +6,17 @@
 // neighbours at i-1, j-1 and k-1 (backward plans: the mirrored grid) is swept
 // line by line.  A wavefront owns a tile of 8 x 8 lines (64 x 1 in 2-D), one
 // lane per line, and a lane computes one row of its line per step, row (i, j, k)
-// at step i + a + 2 b (a, b: its line's place in the tile).  The i-1 value is
+// at step i + a + b (a, b: its line's place in the tile).  The i-1 value is
 // then the lane's own previous result, the j-1 value its left neighbour's
-// previous result (a DPP move), the k-1 value comes through LDS and was formed
-// two steps earlier, so that nothing but a few FP operations lies between one
-// step and the next, and no barrier is needed.
+// previous result (a DPP move), the k-1 value another lane's previous result,
+// through LDS; nothing but that and a few FP operations lies between one step
+// and the next, and no barrier is needed.
+//
+// From i + a + b follow: a tile takes S >= nx + LAG steps, LAG = (TJ - 1) + (TK
+// - 1) its last line's start; a value that crosses a tile boundary is formed TJ
+// - 1 = TK - 1 steps of its tile after the step that reads it (2-D: TJ - 1), and
+// is staged beside the results of the step before the one that reads it (k - 1)
+// or of that step (j - 1).
 //
 // Vectors live in the packed order of the tiles' steps: element
 // ((tile * S) + step) * 64 + lane.  A backward plan runs the same kernel on the
