@@ -168,7 +168,8 @@ void jac_pattern(hala_ilu M) {
     // columns of 256 rows where padding every row to the longest adds at most a quarter (what the
     // sweep gains, more padding would take back) and rows have at least five entries.  Applies with 3
     // sweeps, packed -> columns: 27-point 96^3 132 -> 107 us FP32, 172 -> 160 FP64; 40^3 41 -> 34, 46 -> 36;
-    // rows of two (5-point 500^2) 38 -> 37, 40 -> 44; of three (7-point 96^3) 71 -> 59, 84 -> 84
+    // rows of two (5-point 500^2) 38 -> 37, 40 -> 44; of three (7-point 96^3) 71 -> 59, 84 -> 84.
+    // The pattern is laid out once for both precisions; rows of three gain in FP32 only and stay packed.
     auto columns = [&](const dbuf &len, int nnz, const dbuf &ptr, dbuf &off) {
         if (!off.p || nnz == 0) return 0;
         const int w = reduce_max_i32(c, len.as<int>(), n);
